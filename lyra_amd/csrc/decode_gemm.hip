@@ -485,6 +485,227 @@ void decode_gemm_kernel(GemmParams p) {
     }
 }
 
+// The epilogue of finish_row for 4 consecutive columns of one row (one group, K not split, no SwiGLU); t is left finished.
+__device__ __forceinline__ void finish_quad(const GemmParams& p, float (&t)[4], const float (&bias4)[4], int row, int col, bool store) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) t[c] = p.bias_post ? round_bf16(round_bf16(t[c]) + bias4[c]) : t[c] + bias4[c];
+    if (!store) return;
+    const size_t at = (size_t)row * p.N + col;
+    if (p.post_scale) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) t[c] = residual_epilogue(p, t[c], at + c);
+    }
+    if (p.out_f32) out_store(p.out, at * 4, f32x4{t[0], t[1], t[2], t[3]});
+    else out_store(p.out, at * 2, u32x2{pack_bf16(t[0], t[1]), pack_bf16(t[2], t[3])});
+}
+
+// ---- one group with thousands of column spans (the LM head), bf16 weights, more rows than the kernel above holds at once ----
+// One workgroup per compute unit, 8 wavefronts, each 16 * MT rows (up to 128) x 64 columns of float32 accumulators, so that
+// the weights are streamed once for 128 rows where the kernel above streams them again for every 64.  The workgroup's spans
+// (6 or 7 of 1600) go round over its 4 pairs of wavefronts; 2 steps of raw weights per wavefront are in flight, across
+// the end of a span into the next one.  The activations pass through LDS in chunks of 64 K rows, double-buffered and already
+// in the order the matrix instruction takes them (tiles of 16 rows x 32 K of 1 KB), so that the wavefronts fetch them once
+// and read them without bank conflicts: slot (kb, x ^ (2 kb + step)) holds row x, K group kb - the exclusive-or keeps the 8
+// lanes that write one row's pieces on different banks.
+// Bound by the stream of weights: 2048 x 204800 at 65 / 96 / 128 rows 161 / 167 / 176 us (5.2-4.8 TB/s of weights; 296 / 303 /
+// 308 us before), 4096 x 204800 at 128 rows 323 us (589 before).  A wavefront of 128 columns and a whole SIMD's registers was
+// built first: 256 accumulators per lane left the compiler copying and spilling them in the K loop.
+constexpr int kWideWaves = 8;
+
+template <int MT, bool TMAX>
+__global__ __launch_bounds__(kWideWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void decode_gemm_wide_kernel(GemmParams p) {
+    constexpr int kWideDepth = 2;              // steps of weights in flight per wavefront: 64 KB per compute unit
+    constexpr int BUF = MT * 2048;             // bytes of one staged chunk
+    constexpr int PIECES = (MT + 3) / 4;       // 16-byte pieces of a chunk per thread
+    extern __shared__ __align__(16) uint8_t sm_wide[];  // [2][BUF] activations, then (TMAX) [8][16 * MT] floats
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int x = lane & 15, kb = lane >> 4;
+    [[maybe_unused]] float* const sm_t = (float*)(sm_wide + 2 * BUF);
+    GemmParams pe = p;  // what the epilogue of this kernel never does
+    pe.ksplit = 1;
+    pe.swiglu = 0;
+    const int total_spans = (p.N + 127) / 128;
+    const int first_span = (int)((long)blockIdx.x * total_spans / gridDim.x), end_span = (int)((long)(blockIdx.x + 1) * total_spans / gridDim.x);
+    const int rounds = (end_span - first_span + kWideWaves / 2 - 1) / (kWideWaves / 2);
+    const int cnt = min(p.group_sizes[0], p.M);
+    const int row_blocks = (cnt + 16 * MT - 1) / (16 * MT);
+    const int chunks = ((p.K + 63) / 64 + 1) & ~1;  // an even number: past the end of K zeros, without memory traffic
+
+    const int row_bytes = p.packed ? 256 : p.N * 2;
+    const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(p.rhs), 0, (uint32_t)p.K * (uint32_t)((p.packed ? p.pspans * 128 : p.N) * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.lhs), 0, 0x7FFFFFFFu, 0x00020000);
+    // this wavefront's half of its pair's span in a round; columns of this lane
+    auto span_of = [&](int round) { return first_span + round * (kWideWaves / 2) + (wave >> 1); };
+    const int half_col = 64 * (wave & 1) + 4 * x;
+    auto weights_at = [&](int round) {  // lane offset of the weights of a round (no span left: nothing is loaded)
+        const int span = span_of(round);
+        const bool ok = round < rounds && span < end_span && span * 128 + half_col < p.N;
+        return !ok ? kNoLoad : (p.packed ? (span * p.K + 8 * kb) * row_bytes + half_col * 2 : 8 * kb * row_bytes + (span * 128 + half_col) * 2);
+    };
+    u32x2 w[kWideDepth][8];
+    auto load_pair = [&](int d, int pr, int voff, int kk) {
+        const bool live = kk < p.K;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            w[d][2 * pr + h] = __builtin_amdgcn_raw_buffer_load_b64(wrsrc, live ? voff : kNoLoad,
+                                                                    __builtin_amdgcn_readfirstlane(live ? (kk + 2 * pr + h) * row_bytes : 0), kStream);
+    };
+    // staging: thread t moves 16-byte piece t & 7 (step, K group) of rows t / 8, t / 8 + 64 of a row block
+    const int piece = threadIdx.x & 7, s_step = piece >> 2, s_kb = piece & 3;
+    int st_off[PIECES], st_next[PIECES];  // of this row block and of the next
+    u32x4 st[PIECES];
+    auto rows_at = [&](int (&off)[PIECES], int block) {
+#pragma unroll
+        for (int j = 0; j < PIECES; ++j) {
+            const int lr = (int)(threadIdx.x >> 3) + 64 * j, row = block * 16 * MT + lr;
+            const bool ok = block < row_blocks && row < cnt && lr < 16 * MT;
+            const int src = ok ? (p.row_map ? p.row_map[row] : row) : 0;
+            off[j] = ok ? (src * p.K + piece * 8) * 2 : kNoLoad;
+        }
+    };
+    auto stage_load = [&](const int (&off)[PIECES], int chunk) {
+        const bool live = chunk * 64 + piece * 8 < p.K;
+#pragma unroll
+        for (int j = 0; j < PIECES; ++j)
+            st[j] = __builtin_amdgcn_raw_buffer_load_b128(arsrc, live ? off[j] : kNoLoad, __builtin_amdgcn_readfirstlane(chunk * 128), 0);
+    };
+    auto stage_store = [&](int buf) {
+#pragma unroll
+        for (int j = 0; j < PIECES; ++j) {
+            const int lr = (int)(threadIdx.x >> 3) + 64 * j;
+            if (MT % 4 == 0 || lr < 16 * MT)
+                *(u32x4*)(sm_wide + buf * BUF + ((lr >> 4) * 2 + s_step) * 1024 + s_kb * 256 + (((lr & 15) ^ (2 * s_kb + s_step)) * 16)) = st[j];
+        }
+    };
+    const int a_at[2] = {kb * 256 + (x ^ (2 * kb)) * 16, 1024 + kb * 256 + (x ^ (2 * kb + 1)) * 16};
+
+    int voff = weights_at(0);
+    rows_at(st_off, 0);
+    stage_load(st_off, 0);
+#pragma unroll
+    for (int d = 0; d < kWideDepth; ++d)
+#pragma unroll
+        for (int pr = 0; pr < 4; ++pr) load_pair(d, pr, voff, 32 * d);
+    __builtin_amdgcn_sched_barrier(0);
+    stage_store(0);
+    lds_barrier();
+
+    for (int rb = 0; rb < row_blocks; ++rb) {
+        const int rowbase = rb * 16 * MT, rows_here = min(16 * MT, cnt - rowbase);
+        rows_at(st_next, rb + 1);
+        for (int round = 0; round < rounds; ++round) {
+            const int span = span_of(round);
+            const bool last_round = round + 1 == rounds;
+            const int voff_next = weights_at(last_round ? (rb + 1 < row_blocks ? 0 : rounds) : round + 1);
+            f32x4 acc[MT][4];
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) acc[mt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int c0 = 0; c0 < chunks; c0 += 2) {
+#pragma unroll
+                for (int cc = 0; cc < 2; ++cc) {  // (chunk parity = LDS buffer)
+                    const int chunk = c0 + cc;
+                    // the chunk behind this one: of this span, or the first of the next (the rows change with the row block)
+                    const bool wrap = cc == 1 && chunk + 1 == chunks;
+                    int off[PIECES];
+#pragma unroll
+                    for (int j = 0; j < PIECES; ++j) off[j] = wrap && last_round ? st_next[j] : st_off[j];
+                    stage_load(off, wrap ? 0 : chunk + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int s = 0; s < 2; ++s) {
+                        constexpr int kAhead = kWideDepth * 32;
+                        const int d = (2 * cc + s) % kWideDepth;
+                        const int k_over = (2 * chunk + s) * 32 + kAhead - chunks * 64;  // >= 0: runs into the next span
+                        const int k_next = k_over >= 0 ? k_over : k_over + chunks * 64;
+                        const int v_next = k_over >= 0 ? voff_next : voff;
+                        Pack8 bop[4];
+#pragma unroll
+                        for (int pr = 0; pr < 4; ++pr) {
+#pragma unroll
+                            for (int c = 0; c < 4; c += 2) {
+                                const uint32_t lo = w[d][2 * pr][c >> 1], hi = w[d][2 * pr + 1][c >> 1];
+                                bop[c].u[pr] = __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+                                bop[c + 1].u[pr] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);
+                            }
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int pr = 0; pr < 4; ++pr) load_pair(d, pr, v_next, k_next);
+                        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) {
+                            const bf16x8 a = *(const bf16x8*)(sm_wide + cc * BUF + mt * 2048 + a_at[s]);
+#pragma unroll
+                            for (int c = 0; c < 4; ++c) acc[mt][c] = mfma_16x16x32(a, bop[c].v, acc[mt][c]);
+                            if (mt & 1) __builtin_amdgcn_sched_barrier(0);  // (at most a few row tiles read ahead: registers)
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    stage_store(1 - cc);
+                    lds_barrier();  // (the weights stay in flight)
+                }
+            }
+            voff = voff_next;
+
+            // (what follows is computed here and not ahead of the K loop, which has no registers to keep it in)
+            int kb4 = 4 * kb;
+            asm volatile("" : "+v"(kb4));
+            const int ncol = span * 128 + half_col;
+            const bool span_ok = span < end_span && ncol < p.N;
+            float bias4[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) bias4[c] = p.bias && span_ok ? p.bias[ncol + c] : 0.f;
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int lr = mt * 16 + kb4 + r;
+                    float t[4];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) t[c] = acc[mt][c][r];
+                    finish_quad(pe, t, bias4, rowbase + lr, ncol, span_ok && lr < rows_here);
+                    if (TMAX) {
+                        const float m = row16_max(span_ok ? fmaxf(fmaxf(t[0], t[1]), fmaxf(t[2], t[3])) : -INFINITY);
+                        if (x == 0) sm_t[wave * (16 * MT) + lr] = m;
+                    }
+                }
+            }
+            if (TMAX) {  // the two halves of a span meet
+                lds_barrier();
+                for (int i = threadIdx.x; i < kWideWaves / 2 * 16 * MT; i += kWideWaves * 64) {
+                    const int pair = i / (16 * MT), lr = i - pair * (16 * MT), sp = first_span + round * (kWideWaves / 2) + pair;
+                    const float m = fmaxf(sm_t[2 * pair * (16 * MT) + lr], sm_t[(2 * pair + 1) * (16 * MT) + lr]);
+                    if (lr < rows_here && sp < end_span) p.tile_max[(size_t)(rowbase + lr) * p.tile_ld + sp] = m;
+                }
+                // (the next writes to sm_t come behind the barriers of another K loop)
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < PIECES; ++j) st_off[j] = st_next[j];
+    }
+    wait_all_memory();  // (what was requested past the end returns nothing, but must not outlive the wavefront's registers)
+
+    // rows at or beyond group_sizes[0]: zero product, with the bias (lax.ragged_dot semantics)
+    for (int span = first_span + wave; span < end_span && cnt < p.M; span += kWideWaves) {
+        const int ncol = span * 128 + 8 * x;
+        const bool ok = ncol < p.N;
+        float bias8[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) bias8[c] = p.bias && ok ? p.bias[ncol + c] : 0.f;
+        for (int row0 = cnt; row0 < p.M; row0 += 4) {
+            float t[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) t[c] = 0.f;
+            finish_row(pe, t, bias8, row0 + kb, ncol, ncol, 0, ok && row0 + kb < p.M, false);
+            if (TMAX) store_tile_max(p, t, row0 + kb, span, ok, row0 + kb < p.M && x == 0);
+        }
+    }
+}
+
 #if LYRA_GEMM_HAS_ENTRY
 // Second pass when K was split across workgroups: sum the partials, then bias / SwiGLU / cast.
 // One thread per 4 output columns.
@@ -1983,7 +2204,28 @@ int launch_planned(GemmParams p, const GemmPlan& pl, int layout, int fused_swigl
     // a very wide single projection (the LM head): one workgroup per compute unit with as many wavefronts as its share of spans
     static const bool no_even = getenv("LYRA_GEMM_NO_EVEN_SPANS") != nullptr;  // tuning override
     const int per_cu = (pl.spans + kGroupMaxWgs - 1) / kGroupMaxWgs;
-    if (!no_even && G == 1 && pl.ksplit == 1 && pl.row_par == 1 && pl.spans >= 4 * kGroupMaxWgs && per_cu <= (pl.mt == 1 ? 12 : 8)) {
+    const bool very_wide = !no_even && G == 1 && pl.ksplit == 1 && pl.row_par == 1 && pl.spans >= 4 * kGroupMaxWgs;
+    if constexpr (WT == 0) {
+        // More than 64 rows of bf16 weights: the kernel that streams them once per 128 rows (2048 x 204800: 161-176 us at 65
+        // to 128 rows, where the kernel below streams them twice in 296-308 us; up to 64 rows the one below is the faster,
+        // 151 against 157 us at 64 and 134 against 142 at 1: it stages the activations once per 512 K rows, not per 64).
+        if (very_wide && !fused_swiglu && M > 64) {
+            const int mt = M > 96 ? 8 : 6;
+            const size_t wide_lds = (size_t)2 * mt * 2048 + (tile_max ? (size_t)kWideWaves * 16 * mt * sizeof(float) : 0);
+#define LYRA_LAUNCH_WIDE(T, X) \
+    hipLaunchKernelGGL((decode_gemm_wide_kernel<T, X>), dim3(kGroupMaxWgs), dim3(kWideWaves * 64), wide_lds, st, p)
+            if (mt == 6) {
+                if (tile_max) LYRA_LAUNCH_WIDE(6, true);
+                else LYRA_LAUNCH_WIDE(6, false);
+            } else {
+                if (tile_max) LYRA_LAUNCH_WIDE(8, true);
+                else LYRA_LAUNCH_WIDE(8, false);
+            }
+#undef LYRA_LAUNCH_WIDE
+            return hipGetLastError() == hipSuccess ? LYRA_OK : LYRA_E_LAUNCH;
+        }
+    }
+    if (very_wide && per_cu <= (pl.mt == 1 ? 12 : 8)) {
         p.even_spans = 1;
         grid = dim3(kGroupMaxWgs, 1, 1);
         block = dim3(per_cu * 64);

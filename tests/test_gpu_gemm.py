@@ -646,3 +646,32 @@ def test_span_major_weights_in_the_general_kernel(M, K, N, kind, block):
     else:
         assert torch.equal(plain[0], packed[0]) and torch.equal(plain[1], packed[1])
         np.testing.assert_array_equal(U.to_np(packed[0]), got)
+
+
+@pytest.mark.parametrize("M,K,N,rows,packed", [
+    (65, 1248, 131968, 65, False),   # one row past a 64-row block; K ends in half a chunk of 64, 1031 spans
+    (96, 1280, 131080, 93, True),    # a last span of 8 columns, padding rows
+    (97, 1248, 132096, 97, True),
+    (128, 2048, 131200, 128, False),
+    (129, 1312, 131208, 129, True),  # a second row block of one row (1026 spans: with 1024 or fewer the plan cuts K in two)
+    (250, 1248, 131968, 201, False),
+])
+def test_lm_head_of_more_than_64_rows(M, K, N, rows, packed):
+    """The very wide bf16 projection of more rows than one 64-row block is bit for bit what the same rows give in calls of
+    at most 64 (one running sum over K per element in either kernel), logits and tile maxima alike."""
+    from lyra_amd.kernels import decode_fused as F
+
+    _note(f"gemm very wide M={M} K={K} N={N} rows={rows} packed={packed}")
+    g = torch.Generator(device=U.dev())
+    g.manual_seed(M + K)
+    x = torch.randn(M, K, generator=g, device=U.dev()).to(torch.bfloat16)
+    w = (torch.randn(1, K, N, generator=g, device=U.dev()) * 0.05).to(torch.bfloat16)
+    bias = torch.randn(N, generator=g, device=U.dev())
+    size = lambda n: torch.full((1,), n, dtype=torch.int32, device=U.dev())
+    rhs = F.pack_weights(w) if packed else w
+    logits, tiles = F.gemm_tile_max(x, rhs, size(rows), bias=bias)
+    want = [F.gemm_tile_max(x[i : i + 64].contiguous(), w, size(max(0, min(64, rows - i))), bias=bias) for i in range(0, M, 64)]
+    assert torch.equal(logits, torch.cat([a for a, _ in want])) and torch.equal(tiles, torch.cat([b for _, b in want]))
+    assert torch.equal(F.gemm(x, rhs, size(rows), bias=bias, out_f32=True), logits)
+    exact = x[:rows].double() @ w[0, :, -1024:].double() + bias[-1024:].double()
+    assert (logits[:rows, -1024:].double() - exact).abs().max() < 2e-3
