@@ -65,6 +65,7 @@ struct GemmParams {
     int bias_post;      // one group, no SwiGLU: the bias is added to the bf16-rounded product, in bf16 (then scale / residual)
     int max_slices;     // grouped kernel: most K slices a left-over unit is cut into
     int snake;          // grouped kernel: odd rounds of units run over the workgroups in the opposite direction (-1: if >= 4 rounds)
+    int xcd_runs;       // grouped kernel: neighbouring units go to workgroups behind the same L2
     int touch_last;     // grouped kernel: touch the first weights of the last group's units before the unit list is known
     int even_spans;     // plain kernel: spans dealt out evenly over one workgroup per compute unit
     int row_block;      // K-split kernel: rows per workgroup (64 or 32)
@@ -1324,6 +1325,9 @@ __global__ __launch_bounds__(kSplitWaves * 64) void decode_gemm_group_kernel(Gem
     // which streams ~14 % faster); otherwise one set of 128 columns and all 4 wavefronts interleave.
     const int NO = p.swiglu ? p.N >> 1 : p.N;
     const int q = threadIdx.x & 31;
+    // this workgroup's place in the dealing: its index, or (xcd_runs) an order in which the workgroups of one XCD - every
+    // eighth - are neighbours
+    const int wg = p.xcd_runs && gridDim.x % 8 == 0 ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
     const int row_bytes = PACKED ? 128 * ES : p.N * ES;
     const int steps = p.K >> 5;
     const int half_stride = p.swiglu ? (p.N >> 1) : 128;
@@ -1357,7 +1361,7 @@ __global__ __launch_bounds__(kSplitWaves * 64) void decode_gemm_group_kernel(Gem
         // them): the real requests, two round trips later, then meet them in L2.  Where it does not hold, a few
         // workgroups have fetched 64 KB each for nothing.
         if constexpr (!WIDE_DYN && !PACKED) {
-            const int blk0 = (int)blockIdx.x / spans, span0 = (int)blockIdx.x - blk0 * spans;
+            const int blk0 = wg / spans, span0 = wg - blk0 * spans;
             const bool guess = p.touch_last && blk0 * (16 * MTM) < p.M;
             const __amdgpu_buffer_rsrc_t trsrc = __builtin_amdgcn_make_buffer_rsrc(
                 const_cast<uint8_t*>(p.rhs) + (size_t)(p.G - 1) * p.K * row_bytes, 0, (uint32_t)p.K * (uint32_t)row_bytes, 0x00020000);
@@ -1440,7 +1444,7 @@ __global__ __launch_bounds__(kSplitWaves * 64) void decode_gemm_group_kernel(Gem
     const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.lhs), 0, 0x7FFFFFFFu, 0x00020000);
 
     // state of the work item whose operands are in flight / being consumed
-    int v = blockIdx.x, round = 0;  // (v = round * nwg + blockIdx.x)
+    int v = wg, round = 0;  // (v = round * nwg + wg)
     bool seg_valid = false;
     int seg_u = 0, seg_r0 = 0, seg_r1 = 0;  // its unit and trips [r0, r1) of it
     int g = 0, row0 = 0, rows = 0, span = 0, ncol = 0, wvoff = kNoLoad, avoff[MTM];
@@ -1467,7 +1471,7 @@ __global__ __launch_bounds__(kSplitWaves * 64) void decode_gemm_group_kernel(Gem
             valid = rev >= 0 && rev < tail;
             vv = n_whole + rev;
         } else if (snake && vv < n_whole && (round & 1)) {
-            vv = vv - (int)blockIdx.x + ((int)nwg - 1 - (int)blockIdx.x);  // odd rounds run the other way
+            vv = vv - wg + ((int)nwg - 1 - wg);  // odd rounds run the other way
         }
         seg_valid = valid;
         if constexpr (SLICED) {
@@ -1865,7 +1869,7 @@ __global__ __launch_bounds__(kSplitWaves * 64) void decode_gemm_group_kernel(Gem
     const int total = total_rows;
     const int pad_rows = p.M - min(total, p.M);
     const int pad_spans = (NO + 127) / 128;
-    for (int i = blockIdx.x; i < pad_rows * pad_spans; i += gridDim.x) {
+    for (int i = wg; i < pad_rows * pad_spans; i += gridDim.x) {
         const int sp = i % pad_spans;
         if (threadIdx.x < 32 && sp * 128 + 4 * q < NO) {
             const int row = min(total, p.M) + i / pad_spans;
@@ -2441,6 +2445,12 @@ static int run_decode_gemm(const void* lhs, const int32_t* lhs_row_map, const vo
     p.snake = snake_env;
     static const bool no_touch = getenv("LYRA_GEMM_NO_TOUCH") != nullptr;  // tuning override
     p.touch_last = no_touch ? 0 : 1;
+    // Row-major pieces of 128 columns that do not start on a 128-byte line: the line in which two neighbouring units meet is
+    // fetched once if both run behind one L2 and twice if not (gpt-oss-20b in FP8, 33 tokens: up 117 -> 101 us, down
+    // 65 -> 58).  Where no line is shared, neighbouring units on different XCDs are the faster ones: lyra-small in bf16 at 7
+    // tokens 57 us for both launches against 69, lyra-medium at 64 tokens 299 against 308.
+    const int es = fp8 ? 1 : 2;
+    p.xcd_runs = pl.grouped && !layout && (N * es % 128 || (fused_swiglu && N / 2 * es % 128));
     p.even_spans = 0;
     p.residual = (const uint16_t*)residual;
     p.out_scale = out_scale;

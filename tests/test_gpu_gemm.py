@@ -332,6 +332,21 @@ def test_many_experts_unit_list(G, M, K, N, swiglu):
     U.assert_close(_run(c, swiglu), _want(c, swiglu, big=True), what="unit list")
 
 
+@pytest.mark.parametrize("kind", ["fp8", "e5m2", "bf16"])
+@pytest.mark.parametrize("K,N,swiglu,rounds", [(96, 5696, True, 8), (288, 2880, False, 8), (96, 328, False, 1), (96, 72, False, 1), (2048, 80, True, 0)])
+def test_widths_off_the_128_byte_line_deal_neighbouring_units_to_one_xcd(kind, K, N, swiglu, rounds):
+    """Widths whose 128-column pieces do not start on 128-byte lines: the workgroups of one XCD take neighbouring units (any
+    number of workgroups: whole rounds with a rest, fewer units than 256, a grid that is not a multiple of 8, units cut into
+    K slices).  The result must not depend on who takes what."""
+    sizes = np.array([3, 0, 70, 64, 33, 1, 130, 5] * max(1, rounds) if rounds else [2, 0, 1], np.int32)
+    G, M = sizes.size, int(sizes.sum()) + 3
+    c = _case(31 + N, M, G, K, N, sizes, kind=kind, block=(K, 1), bias=True, w_std=0.05)
+    want = _want(c, swiglu, big=True)
+    first = _run(c, swiglu)
+    U.assert_close(first, want, what="units dealt out in runs per XCD")
+    assert np.array_equal(_run(c, swiglu), first)
+
+
 @pytest.mark.parametrize("K,N,swiglu", [(512, 2048, True), (512, 2048, False), (256, 8192, True), (256, 8192, False)])
 def test_units_listed_by_cost_over_several_rounds(K, N, swiglu):
     """More (row block, column span) units than one round of workgroups: the row blocks are listed by cost class (full
