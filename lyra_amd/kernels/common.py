@@ -55,6 +55,11 @@ def log_kernel_resolution(op: str, *, shape: str, impl: str, tiling: str | None 
     print(f"[kernel] {op:<15} {shape:<26} -> {detail}", file=sys.stderr)
 
 
+def kernel_decided(implementation: Implementation, config: object | None) -> bool:
+    """Whether ``dispatch_kernel`` would run the kernel and say nothing: the caller may then skip its strings and closures."""
+    return config is not None and not _KERNEL_LOG_ENABLED and implementation in ("auto", "pallas", "hip")
+
+
 def dispatch_kernel(
     op: str,
     *,

@@ -7,12 +7,14 @@ default to the reference behaviour: ``position`` may be a ``[B]`` vector (ragged
 """
 from __future__ import annotations
 
+import functools
+import math
 from dataclasses import dataclass
 
 import torch
 
 from lyra_amd import _lib
-from lyra_amd.kernels.common import Implementation, dispatch_kernel
+from lyra_amd.kernels.common import Implementation, dispatch_kernel, kernel_decided
 from lyra_amd.nn.quant import QArray, dequantize, is_scaled
 
 _DECODE_BLOCK = 128  # lyra/kernels/decode_attention.py:29 (slab granularity of the plain path)
@@ -61,6 +63,9 @@ def select_decode_attention_config(
     return DecodeAttentionConfig(out_dtype=out_dtype, cache_dtype=cache_dtype)
 
 
+_config_of = functools.lru_cache(maxsize=4096)(select_decode_attention_config)
+
+
 def decode_window(sliding_window: int, block: int = _DECODE_BLOCK) -> int:
     """lyra/kernels/decode_attention.py:63-65."""
     n_blocks = -(-(sliding_window + block - 1) // block)
@@ -74,11 +79,11 @@ def is_sw(sliding_window: int, kv_len: int, block: int = _DECODE_BLOCK) -> bool:
 
 def _position_vector(position, batch: int, device) -> tuple[torch.Tensor, int]:
     """int32 device tensor and its stride (0: one scalar for the batch, 1: one entry per row)."""
-    pos = torch.as_tensor(position, device=device)
+    pos = position if isinstance(position, torch.Tensor) and position.device == device else torch.as_tensor(position, device=device)
     if pos.dtype != torch.int32:
         pos = pos.to(torch.int32)
     if pos.ndim == 0 or pos.numel() == 1:
-        return pos.reshape(1).contiguous(), 0
+        return pos, 0
     if pos.numel() != batch:
         raise ValueError(f"position must be a scalar or have one entry per batch row ({batch}), got {tuple(pos.shape)}")
     return pos.reshape(batch).contiguous(), 1
@@ -90,9 +95,17 @@ def rank_rows(position: torch.Tensor) -> torch.Tensor:
     compute it once per step or per batch and hand it to every layer's ``decode_attention(..., row_order=...)``."""
     pos = position.to(torch.int32).reshape(-1).contiguous()
     order = torch.empty_like(pos)
-    rc = _lib.lib.lyra_attention_rank(pos.data_ptr(), pos.numel(), order.data_ptr(), torch.cuda.current_stream(pos.device).cuda_stream)
+    rc = _lib.lib.lyra_attention_rank(pos.data_ptr(), pos.numel(), order.data_ptr(), _lib.raw_stream(pos.device))
     _lib.check(rc, "lyra_attention_rank")
     return order
+
+
+def _laid_out(t: torch.Tensor, dtype: torch.dtype, shape: tuple, device=None) -> torch.Tensor:
+    """A tensor whose memory holds ``t`` as a contiguous array of ``dtype`` and ``shape`` (``t`` itself where it does already,
+    whatever dimensions of size 1 it carries: only its address is used)."""
+    if t.dtype == dtype and t.is_contiguous() and t.numel() == math.prod(shape) and (device is None or t.device == device):
+        return t
+    return t.to(device=device or t.device, dtype=dtype).reshape(shape).contiguous()
 
 
 def _decode_attention(q, k, v, sinks, sm_scale, sliding_window, position, config: DecodeAttentionConfig, dtype, gate=None,
@@ -109,36 +122,35 @@ def _decode_attention(q, k, v, sinks, sm_scale, sliding_window, position, config
         if k.block != (1, H) or v.block != (1, H):
             raise ValueError(f"FP8 KV cache block must be (1, {H}), got {k.block}/{v.block}")
         k_val, v_val = k.qval, v.qval
-        k_scale = k.scale.to(torch.float32).reshape(B, K, S).contiguous()
-        v_scale = v.scale.to(torch.float32).reshape(B, K, S).contiguous()
+        k_scale, v_scale = _laid_out(k.scale, torch.float32, (B, K, S)), _laid_out(v.scale, torch.float32, (B, K, S))
         kv_dtype = _lib.fp8_code(k_val.dtype)
     else:
         if isinstance(k, QArray) or isinstance(v, QArray):
             raise ValueError("dense decode attention config received QArray k/v")
-        k_val, v_val = k.to(torch.bfloat16), v.to(torch.bfloat16)
+        k_val, v_val = (t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16) for t in (k, v))
         k_scale = v_scale = None
         kv_dtype = _lib.DTYPE_BF16
     if not q.is_cuda:
         raise ValueError("the HIP decode attention kernel needs device tensors")
     dev = q.device
-    q_c = q.to(torch.bfloat16).reshape(B, N, H).contiguous()
+    q_c = _laid_out(q, torch.bfloat16, (B, N, H))
     k_c, v_c = k_val.contiguous(), v_val.contiguous()
-    sinks_c = sinks.to(device=dev, dtype=torch.float32).reshape(N).contiguous()
+    sinks_c = _laid_out(sinks, torch.float32, (N,), dev)
     pos, stride = _position_vector(position, B, dev)
     gate_c = None
     if gate is not None:
-        gate_c = gate.to(device=dev, dtype=torch.bfloat16).reshape(B, N).contiguous()
+        gate_c = _laid_out(gate, torch.bfloat16, (B, N), dev)
     out_dtype = torch.float32 if dtype == torch.float32 else torch.bfloat16
     out = torch.empty((B, N, 1, H), dtype=out_dtype, device=dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
-    need = _lib.lib.lyra_decode_attention_workspace(B, N, K, S, H, int(sliding_window))
+    stream = _lib.raw_stream(dev)
+    need = _lib.attention_workspace(B, N, K, S, H, int(sliding_window))
     ws = _lib.workspace("attention", dev, stream, need)
     head = (q_c.data_ptr(), k_c.data_ptr(), v_c.data_ptr(),
             k_scale.data_ptr() if quantized else None, v_scale.data_ptr() if quantized else None,
             sinks_c.data_ptr(), pos.data_ptr(), stride, gate_c.data_ptr() if gate_c is not None else None)
     tail = (out.data_ptr(), ws.data_ptr(), ws.numel(), B, N, K, S, H, float(sm_scale), int(sliding_window), kv_dtype,
             _lib.DTYPE_F32 if out_dtype == torch.float32 else _lib.DTYPE_BF16, stream)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         if xsa_v is not None:
             vn = xsa_v.to(device=dev, dtype=torch.bfloat16).reshape(B, K, H).contiguous()
             alpha = xsa_alpha.to(device=dev, dtype=torch.float32).reshape(N).contiguous()
@@ -255,16 +267,16 @@ def decode_attention(
     cache_dtype = k.dtype if isinstance(k, QArray) else None
     supported_layout = N % K == 0 and q.is_cuda
     config = (
-        select_decode_attention_config(
-            head_dim=H, head_groups=HEAD_GROUPS, kv_len=S, sliding_window=sliding_window, out_dtype=dtype, cache_dtype=cache_dtype,
-            batch=B, kv_heads=K,
-        )
+        _config_of(H, HEAD_GROUPS, S, int(sliding_window), dtype, cache_dtype, B, K)
         if supported_layout
         else None
     )
 
     if (xsa_v is None) != (xsa_alpha is None):
         raise ValueError("xsa_v and xsa_alpha go together")
+    if kernel_decided(implementation, config):
+        return _decode_attention(q, k, v, sinks, sm_scale, sliding_window, position, config, dtype, gate=gate,
+                                 xsa_v=xsa_v, xsa_alpha=xsa_alpha, row_order=row_order)
 
     def reference():
         t = decode_attention_reference(q, k, v, sinks, sm_scale, sliding_window, position, dtype, gate=gate)

@@ -16,7 +16,7 @@ _L = _lib.lib
 
 
 def _stream(dev) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    return _lib.raw_stream(dev)
 
 
 def _ptr(t):
@@ -180,7 +180,7 @@ def gemm_unsummed(lhs: torch.Tensor, rhs, group_sizes: torch.Tensor) -> Unsummed
     rv, rs, bk, bn, rd, (G, _, N) = _rhs_args(rhs)
     if G != 1 or K % 32 or N % 8 or (isinstance(rhs, SpanMajor) and rhs.layout != 1):
         return None
-    splits = _L.lyra_decode_gemm_splits(M, K, N, bk)
+    splits = _lib.gemm_splits(M, K, N, bk)
     if splits <= 0:
         return None
     assert lhs_t.dtype == torch.bfloat16 and lhs_t.is_contiguous()
@@ -358,7 +358,7 @@ def attention_qkv(qkv, qnorm, knorm, cos_t: torch.Tensor, sin_t: torch.Tensor, p
         assert gate.dtype == torch.bfloat16 and gate.is_contiguous() and gate.numel() == B * N
     out = torch.empty((B, N * H), dtype=out_dtype, device=dev)
     stream = _stream(dev)
-    need = _L.lyra_decode_attention_workspace(B, N, K, S, H, int(sliding_window))
+    need = _lib.attention_workspace(B, N, K, S, H, int(sliding_window))
     ws = _lib.workspace("attention", dev, stream, need)
     qkv_bias = qkv.bias if unsummed else None
     if qkv_bias is not None:
@@ -412,7 +412,7 @@ def gemm(lhs: torch.Tensor, rhs, group_sizes: torch.Tensor, *, rows: int | None 
     if bias is not None:
         assert bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == G * N
     stream = _stream(dev)
-    need = _L.lyra_decode_gemm_workspace(M, G, K, N, int(fused_swiglu))
+    need = _lib.gemm_workspace(M, G, K, N, int(fused_swiglu))
     ws = _lib.workspace("gemm", dev, stream, need)
     rc = _L.lyra_decode_gemm_ex(lhs_t.data_ptr(), _ptr(row_map), rv.data_ptr(), _ptr(rs), bk, bn, group_sizes.data_ptr(), _ptr(bias),
                                 _ptr(residual), 1.0 if out_scale is None else float(out_scale),
@@ -452,7 +452,7 @@ def gemm_tile_max(lhs: torch.Tensor, rhs, group_sizes: torch.Tensor, bias: torch
     out = torch.empty((M, N), dtype=torch.float32, device=dev)
     tmax = torch.empty((M, (N + 127) // 128), dtype=torch.float32, device=dev)
     stream = _stream(dev)
-    ws = _lib.workspace("gemm", dev, stream, _L.lyra_decode_gemm_workspace(M, 1, K, N, 0))
+    ws = _lib.workspace("gemm", dev, stream, _lib.gemm_workspace(M, 1, K, N, 0))
     rc = _L.lyra_decode_gemm_tile_max(lhs.data_ptr(), None, rv.data_ptr(), _ptr(rs), bk, bn, group_sizes.data_ptr(), _ptr(bias),
                                       out.data_ptr(), tmax.data_ptr(), ws.data_ptr(), ws.numel(), M, 1, K, N, rd, _lib.DTYPE_F32,
                                       stream)

@@ -6,13 +6,14 @@ implementation)`` runs the gfx950 HIP kernel through ``lyra_decode_gemm`` (inclu
 """
 from __future__ import annotations
 
+import functools
 import math
 from dataclasses import dataclass
 
 import torch
 
 from lyra_amd import _lib
-from lyra_amd.kernels.common import Implementation, dispatch_kernel, swiglu
+from lyra_amd.kernels.common import Implementation, dispatch_kernel, kernel_decided, log_kernel_resolution, swiglu
 from lyra_amd.nn.quant import QArray, dequantize, is_scaled, quantize
 
 
@@ -50,6 +51,24 @@ def select_decode_gemm_config(m: int, groups: int, k: int, n: int, quant_dtype=N
         if block is not None and not _scale_layout_supported(k, n, tuple(block)):
             return None
     return DecodeGEMMConfig(fwd_dtype=quant_dtype)
+
+
+_config_of = functools.lru_cache(maxsize=4096)(select_decode_gemm_config)
+
+
+def one_group(lhs, rhs, quant_dtype, out_dtype):
+    """lhs [M, K] bf16 times rhs [1, K, N] (bf16 or QArray, contiguous scales and codes not required) to ``out_dtype`` (bf16 or
+    float32) on the kernel, or None where it has no configuration for the shape.  What ``decode_gemm`` does with one group of
+    all rows, without the casts to and from float32 that its output type costs there."""
+    M = lhs.shape[0]
+    _, K, N = rhs.shape
+    block = tuple(rhs.block) if isinstance(rhs, QArray) else None
+    config = _config_of(M, 1, K, N, quant_dtype, block, False)
+    if config is None:
+        return None
+    log_kernel_resolution("decode_gemm", shape=f"m{M} g1 k{K} n{N}", impl="hip", tiling=f"n8/k32 dtype={'fp8' if quant_dtype else 'bf16'}")
+    return _decode_gemm(lhs, rhs, _lib.row_count(M, lhs.device), config, bias=None, fused_swiglu=False, swiglu_beta=1.702,
+                        swiglu_limit=7.0, out_dtype=out_dtype)
 
 
 def _expert_ids(group_sizes: torch.Tensor, total: int) -> torch.Tensor:
@@ -97,18 +116,19 @@ def _decode_gemm(lhs, rhs, group_sizes, config: DecodeGEMMConfig, *, bias, fused
         rhs_val = rhs.to(torch.bfloat16).contiguous()
         rhs_scale, bk, bn = None, 0, 0
         rhs_dtype = _lib.DTYPE_BF16
-    lhs_c = lhs.to(torch.bfloat16).contiguous()
-    gs = group_sizes.to(device=dev, dtype=torch.int32).contiguous()
+    lhs_c = (lhs if lhs.dtype == torch.bfloat16 else lhs.to(torch.bfloat16)).contiguous()
+    gs = group_sizes if group_sizes.dtype == torch.int32 and group_sizes.device == dev else group_sizes.to(device=dev, dtype=torch.int32)
+    gs = gs.contiguous()
     bias_c = None
     if bias is not None:
         bias_c = normalize_bias(bias, G, N, torch.float32).to(dev).reshape(G, N).contiguous()
     NO = N // 2 if fused_swiglu else N
     k_out = torch.float32 if out_dtype == torch.float32 else torch.bfloat16
     out = torch.empty((M, NO), dtype=k_out, device=dev)
-    stream = torch.cuda.current_stream(dev).cuda_stream
-    need = _lib.lib.lyra_decode_gemm_workspace(M, G, K, N, int(fused_swiglu))
+    stream = _lib.raw_stream(dev)
+    need = _lib.gemm_workspace(M, G, K, N, int(fused_swiglu))
     ws = _lib.workspace("gemm", dev, stream, need)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.lib.lyra_decode_gemm(
             lhs_c.data_ptr(), rhs_val.data_ptr(), rhs_scale.data_ptr() if rhs_scale is not None else None, bk, bn,
             gs.data_ptr(), bias_c.data_ptr() if bias_c is not None else None, out.data_ptr(), ws.data_ptr(), ws.numel(),
@@ -190,10 +210,15 @@ def decode_gemm(
     out_dtype = lhs.dtype
 
     config = (
-        select_decode_gemm_config(m=M, groups=G, k=K, n=N, quant_dtype=dtype, block=block, fused_swiglu=fused_swiglu)
+        _config_of(M, G, K, N, dtype, None if block is None else tuple(block), fused_swiglu)
         if lhs.is_cuda
         else None
     )
+    if kernel_decided(implementation, config):
+        return _decode_gemm(
+            lhs, rhs_kernel, group_sizes, config, bias=bias, fused_swiglu=fused_swiglu,
+            swiglu_beta=swiglu_beta, swiglu_limit=swiglu_limit, out_dtype=out_dtype,
+        )
 
     def reference():
         rhs_reference = dequantize(rhs_kernel, lhs.dtype) if isinstance(rhs_kernel, QArray) else rhs_kernel.to(lhs.dtype)

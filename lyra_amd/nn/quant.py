@@ -167,8 +167,12 @@ def dot(lhs: torch.Tensor, rhs, *, dimension_numbers=None, preferred_element_typ
             raise ValueError(f"quant.dot: no HIP kernel for lhs {tuple(lhs.shape)} {lhs.dtype} . rhs {tuple(rhs.shape)} {rhs.dtype} "
                              f"with dimension_numbers {dimension_numbers}")
         return _dot_general_torch(lhs, maybe_dequant(rhs, lhs.dtype), ((lc, rc), (lb, rb)), out_dtype)
-    from lyra_amd.kernels.decode_gemm import decode_gemm  # (the kernels package imports this module)
+    from lyra_amd.kernels.decode_gemm import decode_gemm, one_group  # (the kernels package imports this module)
 
+    if implementation in ("auto", "pallas", "hip"):
+        out = one_group(lhs.reshape(-1, lhs.shape[-1]), flat, rhs.dtype if fp8 else None, out_dtype)
+        if out is not None:
+            return out.reshape(*lhs.shape[:-1], *rhs.shape[1:])
     rows = lhs.reshape(-1, lhs.shape[-1])
     if out_dtype == torch.float32:
         rows = rows.to(torch.float32)  # the operator's output dtype is its lhs dtype; the values stay bf16-representable

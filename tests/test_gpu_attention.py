@@ -547,3 +547,36 @@ def test_xla_path_and_dispatch_contract():
         _decode_attention(q, k.qval.to(torch.bfloat16), v.qval.to(torch.bfloat16), sinks, 0.125, 0, 3, DecodeAttentionConfig(cache_dtype=torch.float8_e4m3fn), torch.bfloat16)
     with pytest.raises(ValueError, match="received QArray"):
         _decode_attention(q, k, v, sinks, 0.125, 0, 3, DecodeAttentionConfig(), torch.bfloat16)
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_inputs_in_other_types_and_layouts_give_the_plain_call(fp8):
+    """Operands that already are what the kernel reads go to it as they are; anything else - types, strides, dimensions of size
+    1, a position on the host or in 64 bits - is brought there first.  Both give the same bits."""
+    from lyra_amd.kernels.decode_attention import decode_attention
+    from lyra_amd.nn.quant import QArray, quantize
+
+    g = torch.Generator(device=U.dev()).manual_seed(3)
+    B, N, K, S, H = 3, 8, 2, 96, 64
+    draw = lambda *shape: torch.randn(*shape, device=U.dev(), generator=g)
+    q, k, v = (draw(*s).to(torch.bfloat16) for s in ((B, N, 1, H), (B, K, S, H), (B, K, S, H)))
+    sinks, gate = draw(N), draw(B, N).to(torch.bfloat16)
+    pos = torch.tensor([5, 95, 40], dtype=torch.int32, device=U.dev())
+    if fp8:
+        k, v = (quantize(t, torch.float8_e4m3fn, (1, H)) for t in (k, v))
+    call = lambda q, k, v, sinks, pos, gate: decode_attention(q, k, v, sinks, H**-0.5, 0, pos, gate=gate, dtype=torch.bfloat16)
+    spread = lambda t: torch.stack([t, t], -1)[..., 0]  # the same values, not contiguous
+    if fp8:
+        spread_kv = lambda t: QArray(spread(t.qval.view(torch.uint8)).view(torch.float8_e4m3fn), spread(t.scale).double(), t.block)
+    else:
+        spread_kv = lambda t: spread(t.float())
+    want = call(q, k, v, sinks, pos, gate)
+    others = call(spread(q.float()), spread_kv(k), spread_kv(v), spread(sinks.double())[None, :], pos.long().cpu(), spread(gate.float())[:, :, None])
+    assert torch.equal(others, want)
+    for shared in (40, torch.tensor(40), torch.tensor([[40]], device=U.dev())):
+        one = call(q, k, v, sinks, shared, gate)
+        assert torch.equal(one, call(q, k, v, sinks, torch.full((B,), 40, dtype=torch.int32, device=U.dev()), gate))
+    for bad in (dict(sinks=draw(N + 1)), dict(gate=draw(B, N + 1)), dict(pos=pos[:2])):
+        args = dict(q=q, k=k, v=v, sinks=sinks, pos=pos, gate=gate) | bad
+        with pytest.raises((RuntimeError, ValueError)):
+            call(**args)

@@ -690,3 +690,32 @@ def test_lm_head_of_more_than_64_rows(M, K, N, rows, packed):
     assert torch.equal(F.gemm(x, rhs, size(rows), bias=bias, out_f32=True), logits)
     exact = x[:rows].double() @ w[0, :, -1024:].double() + bias[-1024:].double()
     assert (logits[:rows, -1024:].double() - exact).abs().max() < 2e-3
+
+
+@pytest.mark.parametrize("rows", [1, 63, 4096, 4097])
+def test_quant_dot_row_counts_on_streams_and_in_a_graph(rows):
+    """``quant.dot`` takes its row count from a table kept per device (beyond 4096 rows from a fill): same bits as the operator
+    with sizes of the caller's own, on another stream and in a graph replayed between eager calls, also to float32."""
+    from lyra_amd.kernels.decode_gemm import decode_gemm
+    from lyra_amd.nn.quant import dot
+
+    g = torch.Generator(device=U.dev()).manual_seed(rows)
+    x = torch.randn(rows, 96, device=U.dev(), generator=g).to(torch.bfloat16)
+    w = torch.randn(96, 72, device=U.dev(), generator=g).to(torch.bfloat16)
+    want = decode_gemm(x, w[None], torch.full((1,), rows, dtype=torch.int32, device=U.dev()))
+    want32 = decode_gemm(x.float(), w[None], torch.full((1,), rows, dtype=torch.int32, device=U.dev()))
+    assert torch.equal(dot(x, w), want)
+    assert torch.equal(dot(x, w, preferred_element_type=torch.float32), want32)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        assert torch.equal(dot(x, w), want)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out = dot(x, w)
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(dot(x, w), want)
