@@ -887,3 +887,26 @@ def test_norm_writes_its_rows_in_tiles(B, C, n):
     h2, _, x2 = F.rmsnorm_proj(F.Unsummed(part, x, 0.25), scale, 1e-5, proj, None)
     h2t, _, x2t = F.rmsnorm_proj(F.Unsummed(part, x, 0.25), scale, 1e-5, proj, None, tiled=True)
     assert torch.equal(h2t.untiled(), h2) and torch.equal(x2t, x2)
+
+
+@pytest.mark.parametrize("rows,cols", [(6, 1), (6, 4095), (7, 4097), (6, 8192), (6, 12289), (64, 50000), (520, 9000)])
+def test_argmax_first_of_ties_masked_rows_and_nans(rows, cols):
+    """Chunks of whole and cut 4096-column blocks: ties go to the first column, rows (or chunks) of -inf give their first
+    column, NaNs never win, columns past ``cols`` are not looked at."""
+    from lyra_amd.kernels.decode_fused import argmax
+
+    g = torch.Generator().manual_seed(rows + cols)
+    x = torch.randn(rows, (cols + 3) // 4 * 4 + 4, generator=g)
+    x[0] = -float("inf")
+    x[1, : cols - 1] = -float("inf")
+    x[2] = float("nan")
+    x[2, cols - 1] = -float("inf")
+    x[3] = torch.randint(0, 2, (x.shape[1],), generator=g).float()
+    x[4, ::2] = float("nan")
+    x[:, cols:] = 99.0
+    seen = torch.nan_to_num(x[:, :cols].clone(), nan=-float("inf"), neginf=-float("inf"))
+    want = seen.numpy().argmax(1)
+    want[2] = cols - 1
+    dev = x.to("cuda:0")
+    for _ in range(2):  # (the arrival counters are left zero)
+        assert np.array_equal(argmax(dev, cols).cpu().numpy(), want)
