@@ -65,7 +65,9 @@ struct GemmParams {
     int bias_post;      // one group, no SwiGLU: the bias is added to the bf16-rounded product, in bf16 (then scale / residual)
     int max_slices;     // grouped kernel: most K slices a left-over unit is cut into
     int snake;          // grouped kernel: odd rounds of units run over the workgroups in the opposite direction (-1: if >= 4 rounds)
-    int xcd_runs;       // grouped kernel: neighbouring units go to workgroups behind the same L2
+    // grouped kernel: workgroup b takes place (b & deal_mask) * deal_step + (b >> deal_shift) in the dealing of units: its own
+    // index (0, 0, 0), or one in which the workgroups of an XCD - every eighth - are neighbours (7, grid / 8, 3)
+    int deal_mask, deal_step, deal_shift;
     int touch_last;     // grouped kernel: touch the first weights of the last group's units before the unit list is known
     int even_spans;     // plain kernel: spans dealt out evenly over one workgroup per compute unit
     int row_block;      // K-split kernel: rows per workgroup (64 or 32)
@@ -1325,9 +1327,7 @@ __global__ __launch_bounds__(kSplitWaves * 64) void decode_gemm_group_kernel(Gem
     // which streams ~14 % faster); otherwise one set of 128 columns and all 4 wavefronts interleave.
     const int NO = p.swiglu ? p.N >> 1 : p.N;
     const int q = threadIdx.x & 31;
-    // this workgroup's place in the dealing: its index, or (xcd_runs) an order in which the workgroups of one XCD - every
-    // eighth - are neighbours
-    const int wg = p.xcd_runs && gridDim.x % 8 == 0 ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
+    const int wg = (int)(blockIdx.x & (unsigned)p.deal_mask) * p.deal_step + (int)(blockIdx.x >> p.deal_shift);
     const int row_bytes = PACKED ? 128 * ES : p.N * ES;
     const int steps = p.K >> 5;
     const int half_stride = p.swiglu ? (p.N >> 1) : 128;
@@ -2116,6 +2116,16 @@ int launch_planned(GemmParams p, const GemmPlan& pl, int layout, int fused_swigl
         const int gkw = layout ? (packed_wide ? 2 : kSplitWaves) : ((fused_swiglu || pl.wide) ? 2 : kSplitWaves);
         const long trips_least = std::max(1, ((K / 32 + gkw - 1) / gkw + 7) / 8);  // trips per unit (at least)
         const dim3 ggrid((unsigned)std::max(1L, std::min((long)kGroupMaxWgs, most_units * trips_least))), gblock(kSplitWaves * 64);
+        // Row-major pieces of 128 columns that do not start on a 128-byte line: the line in which two neighbouring units meet is
+        // fetched once if both run behind one L2 and twice if not (gpt-oss-20b in FP8, 33 tokens: up 117 -> 101 us, down
+        // 65 -> 58).  Where no line is shared, neighbouring units on different XCDs are the faster ones: lyra-small in bf16 at
+        // 7 tokens 57 us for both launches against 69, lyra-medium at 64 tokens 299 against 308.
+        const int es = fp8 ? 1 : 2;
+        if (!layout && (N * es % 128 || (fused_swiglu && N / 2 * es % 128)) && ggrid.x % 8 == 0) {
+            p.deal_mask = 7;
+            p.deal_step = (int)ggrid.x / 8;
+            p.deal_shift = 3;
+        }
         const size_t glds = (size_t)kSplitWaves * 16 * kGroupTiles * kSplitPitch * sizeof(float);
         const bool step_scales = fp8 && p.scale_mode == 1 && p.bk < p.K;
 #define LYRA_GROUP_RS(F, S, R, C)                                                                                     \
@@ -2445,12 +2455,7 @@ static int run_decode_gemm(const void* lhs, const int32_t* lhs_row_map, const vo
     p.snake = snake_env;
     static const bool no_touch = getenv("LYRA_GEMM_NO_TOUCH") != nullptr;  // tuning override
     p.touch_last = no_touch ? 0 : 1;
-    // Row-major pieces of 128 columns that do not start on a 128-byte line: the line in which two neighbouring units meet is
-    // fetched once if both run behind one L2 and twice if not (gpt-oss-20b in FP8, 33 tokens: up 117 -> 101 us, down
-    // 65 -> 58).  Where no line is shared, neighbouring units on different XCDs are the faster ones: lyra-small in bf16 at 7
-    // tokens 57 us for both launches against 69, lyra-medium at 64 tokens 299 against 308.
-    const int es = fp8 ? 1 : 2;
-    p.xcd_runs = pl.grouped && !layout && (N * es % 128 || (fused_swiglu && N / 2 * es % 128));
+    p.deal_mask = p.deal_step = p.deal_shift = 0;
     p.even_spans = 0;
     p.residual = (const uint16_t*)residual;
     p.out_scale = out_scale;
