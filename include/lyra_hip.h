@@ -181,6 +181,14 @@ int lyra_decode_attention_static(const void* q, const void* k, const void* v, co
 int lyra_workspace_init(void* workspace, size_t workspace_bytes, lyra_stream_t stream);
 
 /*
+ * Address on the current device of a read-only table of int32 0, 1, ..., LYRA_MAX_ROW_COUNT: entry n serves as the
+ * `group_sizes` of a one-group product of n rows.  Part of the loaded code - no launch, no copy, no wait.  NULL if the
+ * runtime cannot tell.  No counterpart in the reference.
+ */
+#define LYRA_MAX_ROW_COUNT 4096
+const int32_t* lyra_row_counts(void);
+
+/*
  * Decode grouped matmul: out[r,:] = epilogue(lhs[r,:] @ rhs[e(r)]) with rows sorted by group.
  * Stands behind lyra.kernels.decode_gemm.decode_gemm (lyra/kernels/decode_gemm.py:404-474;
  * maths of grouped_gemm_reference, lyra/kernels/gemm.py:1575-1617) and, with G == 1, behind

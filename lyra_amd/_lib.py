@@ -58,6 +58,7 @@ SIGNATURES = {
         _c.c_int,
         [_c.c_void_p] * 7 + [_c.c_int] + [_c.c_void_p] * 2 + [_c.c_int] * 5 + [_c.c_float] + [_c.c_int] * 3 + [_c.c_void_p],
     ),
+    "lyra_row_counts": (_c.c_void_p, []),
     "lyra_workspace_init": (_c.c_int, [_c.c_void_p, _c.c_size_t, _c.c_void_p]),
     "lyra_decode_gemm": (
         _c.c_int,
@@ -199,20 +200,26 @@ def on_device(device):
     return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
-_ROW_COUNTS: dict[int, "object"] = {}
-_MAX_ROW_COUNT = 4096
+_ROW_COUNTS: dict = {}
+_MAX_ROW_COUNT = 4096  # LYRA_MAX_ROW_COUNT
 
 
 def row_count(rows: int, device):
-    """int32 [1] on ``device`` holding ``rows``: the group sizes of a one-group product, from one table of 16 KB per device
-    instead of a fill launch per call.  (The table is copied from the host before anyone sees it, so it can be read on any
-    stream; while a graph is being captured no table is made.)"""
+    """int32 [1] on ``device`` holding ``rows``: the group sizes of a one-group product, a view of the library's own table
+    (lyra_row_counts) instead of a fill launch per call.  The table is part of the loaded code, so there is nothing to wait
+    for: it can be read on any stream and while any thread captures a graph."""
     import torch
 
-    table = _ROW_COUNTS.get(device.index)
-    if table is None and rows <= _MAX_ROW_COUNT and not torch.cuda.is_current_stream_capturing():
-        table = torch.arange(_MAX_ROW_COUNT + 1, dtype=torch.int32).to(device)  # (from pageable memory: done when it returns)
-        table = _ROW_COUNTS.setdefault(device.index, table)
+    table = _ROW_COUNTS.get(device)
+    if table is None and device.type == "cuda" and rows <= _MAX_ROW_COUNT:
+        with on_device(device):
+            address = lib.lyra_row_counts()
+        if address:
+            count = _MAX_ROW_COUNT + 1
+            memory = torch._C._construct_storage_from_data_pointer(address, device, 4 * count)
+            table = torch.empty(0, dtype=torch.int32, device=device).set_(memory, 0, (count,))
+            if type(table) is torch.Tensor:  # (not a stand-in for one)
+                _ROW_COUNTS[device] = table
     if table is None or rows > _MAX_ROW_COUNT:
         return torch.full((1,), rows, dtype=torch.int32, device=device)
     return table[rows : rows + 1]

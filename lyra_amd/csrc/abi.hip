@@ -123,7 +123,26 @@ __global__ __launch_bounds__(64) void selftest_kernel(int32_t* report) {
     if (lane == 0) report[7] = LYRA_ABI_VERSION;
 }
 
+struct RowCounts {
+    int32_t n[LYRA_MAX_ROW_COUNT + 1];
+};
+constexpr RowCounts make_row_counts() {
+    RowCounts t = {};
+    for (int i = 0; i <= LYRA_MAX_ROW_COUNT; ++i) t.n[i] = i;
+    return t;
+}
+__device__ RowCounts row_counts = make_row_counts();
+
 }  // namespace lyra
+
+extern "C" const int32_t* lyra_row_counts(void) {
+    void* at = nullptr;
+    if (hipGetSymbolAddress(&at, HIP_SYMBOL(lyra::row_counts)) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return (const int32_t*)at;
+}
 
 extern "C" int lyra_abi_version(void) { return LYRA_ABI_VERSION; }
 

@@ -719,3 +719,71 @@ def test_quant_dot_row_counts_on_streams_and_in_a_graph(rows):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want) and torch.equal(dot(x, w), want)
+
+
+def test_quant_dot_first_call_on_a_device(monkeypatch):
+    """The table of row counts is looked up by whichever call comes first: behind queued work with the default device set to the
+    GPU and read at once on another stream, on a stream that is being captured, and by one thread while another captures."""
+    import threading
+
+    from lyra_amd import _lib
+    from lyra_amd.kernels.decode_gemm import decode_gemm
+    from lyra_amd.nn.quant import dot
+
+    _note("quant.dot first call")
+    g = torch.Generator(device=U.dev()).manual_seed(11)
+    x = torch.randn(33, 96, device=U.dev(), generator=g).to(torch.bfloat16)
+    w = torch.randn(96, 72, device=U.dev(), generator=g).to(torch.bfloat16)
+    want = decode_gemm(x, w[None], torch.full((1,), 33, dtype=torch.int32, device=U.dev()))
+    busy = torch.randn(4096, 4096, device=U.dev(), generator=g)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for s in (a, b):  # (the streams' workspaces exist)
+        with torch.cuda.stream(s):
+            dot(x, w)
+    torch.cuda.synchronize()
+
+    monkeypatch.setattr(_lib, "_ROW_COUNTS", {})
+    with torch.device("cuda"):
+        with torch.cuda.stream(a):
+            for _ in range(10):
+                busy = busy @ busy * 1e-3
+            first = dot(x, w)
+        with torch.cuda.stream(b):
+            second = dot(x, w)
+    torch.cuda.synchronize()
+    assert torch.equal(first, want) and torch.equal(second, want)
+
+    monkeypatch.setattr(_lib, "_ROW_COUNTS", {})
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=a):
+        out = dot(x, w)
+    for _ in range(3):
+        out.zero_()
+        assert torch.equal(dot(x, w), want)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+    monkeypatch.setattr(_lib, "_ROW_COUNTS", {})
+    got = []
+
+    def other():
+        with torch.cuda.stream(b):
+            got.append(dot(x, w))
+
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=a):
+        out = dot(x, w)
+        thread = threading.Thread(target=other)
+        thread.start()
+        thread.join()
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want) and len(_lib._ROW_COUNTS) == 1
+    counts = [_lib.row_count(n, U.dev()) for n in range(_lib._MAX_ROW_COUNT + 2)]
+    assert torch.equal(torch.cat(counts), torch.arange(len(counts), dtype=torch.int32, device=U.dev()))
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)

@@ -376,3 +376,22 @@ def test_quant_dot_and_einsum_on_the_plain_path():
     # the kernel cannot be asked for on CPU tensors
     with pytest.raises(ValueError, match="no HIP kernel"):
         dot(x, w, implementation="pallas")
+
+
+def test_row_counts_survive_default_devices_and_fake_tensors(monkeypatch):
+    """The kept table of row counts is made on the device it is for, whatever the default device is, and a table made while
+    fake tensors stand in for real ones is not kept."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from lyra_amd import _lib
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    cpu = torch.device("cpu")
+    for context in (torch.device("meta"), FakeTensorMode()):
+        monkeypatch.setattr(_lib, "_ROW_COUNTS", {})
+        with context:
+            during = _lib.row_count(7, cpu)
+        assert during.device == cpu and during.shape == (1,) and during.dtype == torch.int32
+        after = _lib.row_count(9, cpu)
+        assert type(after) is torch.Tensor and after.tolist() == [9]
+    assert _lib.row_count(4096, cpu).tolist() == [4096] and _lib.row_count(4097, cpu).tolist() == [4097]
