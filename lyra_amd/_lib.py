@@ -210,16 +210,16 @@ def row_count(rows: int, device):
     for: it can be read on any stream and while any thread captures a graph."""
     import torch
 
-    table = _ROW_COUNTS.get(device)
-    if table is None and device.type == "cuda" and rows <= _MAX_ROW_COUNT:
+    count = _ROW_COUNTS.get((rows, device))
+    if count is not None:
+        return count
+    if device.type == "cuda" and 0 <= rows <= _MAX_ROW_COUNT:
         with on_device(device):
-            address = lib.lyra_row_counts()
-        if address:
-            count = _MAX_ROW_COUNT + 1
-            memory = torch._C._construct_storage_from_data_pointer(address, device, 4 * count)
-            table = torch.empty(0, dtype=torch.int32, device=device).set_(memory, 0, (count,))
-            if type(table) is torch.Tensor:  # (not a stand-in for one)
-                _ROW_COUNTS[device] = table
-    if table is None or rows > _MAX_ROW_COUNT:
-        return torch.full((1,), rows, dtype=torch.int32, device=device)
-    return table[rows : rows + 1]
+            table = lib.lyra_row_counts()
+        if table:
+            memory = torch._C._construct_storage_from_data_pointer(table + 4 * rows, device, 4)
+            count = torch.empty(0, dtype=torch.int32, device=device).set_(memory, 0, (1,))
+            if type(count) is torch.Tensor:  # (not a stand-in for one)
+                _ROW_COUNTS[rows, device] = count
+            return count
+    return torch.full((1,), rows, dtype=torch.int32, device=device)

@@ -18,6 +18,7 @@ from functools import lru_cache
 import numpy as np
 import torch
 
+from lyra_amd import _lib
 from lyra_amd.kernels.common import Implementation
 from lyra_amd.kernels.op import Mode, attn_op, gmm_op
 from lyra_amd.nn.quant import QArray, dot, quantize
@@ -446,14 +447,7 @@ def dense_mlp_apply(x, w: DenseMLPWeights, cfg: ModelConfig):
 
 
 # ---- the same layers with every step between the two hot kernels as one fused HIP launch --------------------
-def _one_group(rows: int, device) -> torch.Tensor:
-    key = (rows, str(device))
-    if key not in _ONE_GROUP:
-        _ONE_GROUP[key] = torch.full((1,), rows, dtype=torch.int32, device=device)
-    return _ONE_GROUP[key]
-
-
-_ONE_GROUP: dict = {}
+_one_group = _lib.row_count  # group sizes of a product of one group, int32 [1]
 _SEPARATE_COMBINE = os.environ.get("LYRA_MOE_COMBINE_KERNEL") is not None  # tuning override: combine in a launch of its own
 _SEPARATE_QKV_POST = os.environ.get("LYRA_QKV_POST_KERNEL") is not None  # tuning override: QK norm + RoPE + cache append in a launch of its own
 _TILED_ACTIVATIONS = os.environ.get("LYRA_ROW_MAJOR_ACTIVATIONS") is None  # tuning override: expert matmuls read row-major activations

@@ -535,3 +535,21 @@ def test_config5_lyra_max_full_depth_b128_ctx4096():
               f"CPU side {time.perf_counter() - t2:.0f} s", file=sys.stderr, flush=True)
         assert rel[ok].max() <= 0.01, f"layer {idx}: {rel[ok].max()}"
         del wn, cn
+
+
+def test_one_group_first_asked_for_while_a_graph_is_captured():
+    """The group sizes of a step's one-group products hold their value although the call that first asked for them was only
+    recorded, and never replayed, and on whatever stream they are read."""
+    from lyra_amd import model as M
+
+    dev = torch.device("cuda:0")
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        kept = [M._one_group(rows, dev) for rows in (3, 1237, 4096)]
+        out = [k * 2 for k in kept]
+    assert [M._one_group(rows, dev).item() for rows in (3, 1237, 4096)] == [3, 1237, 4096]
+    for _ in range(3):
+        for o in out:
+            o.zero_()
+        graph.replay()
+        assert [o.item() for o in out] == [6, 2474, 8192]

@@ -395,3 +395,15 @@ def test_row_counts_survive_default_devices_and_fake_tensors(monkeypatch):
         after = _lib.row_count(9, cpu)
         assert type(after) is torch.Tensor and after.tolist() == [9]
     assert _lib.row_count(4096, cpu).tolist() == [4096] and _lib.row_count(4097, cpu).tolist() == [4097]
+
+
+def test_one_group_of_a_step_is_not_kept_from_a_stand_in():
+    """The group sizes of a step's one-group products are never a tensor that was made in place of a real one."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from lyra_amd import model
+
+    with FakeTensorMode():
+        model._one_group(1237, torch.device("cpu"))
+    after = model._one_group(1237, torch.device("cpu"))
+    assert type(after) is torch.Tensor and after.dtype == torch.int32 and after.tolist() == [1237]
