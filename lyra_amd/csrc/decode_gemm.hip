@@ -2223,7 +2223,10 @@ int launch_planned(GemmParams p, const GemmPlan& pl, int layout, int fused_swigl
         // More than 64 rows of bf16 weights: the kernel that streams them once per 128 rows (2048 x 204800: 161-176 us at 65
         // to 128 rows, where the kernel below streams them twice in 296-308 us; up to 64 rows the one below is the faster,
         // 151 against 157 us at 64 and 134 against 142 at 1: it stages the activations once per 512 K rows, not per 64).
-        if (very_wide && !fused_swiglu && M > 64) {
+        // It addresses the activations with 31-bit offsets: they have to end below 2 GiB, which is not known of rows picked by
+        // a map.
+        const bool near_rows = !p.row_map && (size_t)M * K * 2 < (1ull << 31);
+        if (very_wide && !fused_swiglu && M > 64 && near_rows) {
             const int mt = M > 96 ? 8 : 6;
             const size_t wide_lds = (size_t)2 * mt * 2048 + (tile_max ? (size_t)kWideWaves * 16 * mt * sizeof(float) : 0);
 #define LYRA_LAUNCH_WIDE(T, X) \

@@ -787,3 +787,20 @@ def test_quant_dot_first_call_on_a_device(monkeypatch):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+def test_lm_head_rows_picked_out_of_more_than_2_gib_of_activations():
+    """More than 64 rows of a very wide projection picked by ``row_map`` out of an array whose last rows lie beyond 2 GiB."""
+    from lyra_amd.kernels import decode_fused as F
+
+    _note("gemm very wide, row_map beyond 2 GiB")
+    K, N, M = 4096, 131200, 70
+    g = torch.Generator(device=U.dev()).manual_seed(70)
+    x = torch.empty(262144 + 64, K, device=U.dev(), dtype=torch.bfloat16).normal_(generator=g)
+    w = torch.empty(1, K, N, device=U.dev(), dtype=torch.bfloat16).normal_(0.0, 0.02, generator=g)
+    rows = torch.randint(0, 262144, (M,), device=U.dev(), generator=g)
+    rows[::3] = 262144 + torch.arange((M + 2) // 3, device=U.dev())
+    rows[5] = rows[6]
+    sizes = torch.full((1,), M, dtype=torch.int32, device=U.dev())
+    got = F.gemm(x, w, sizes, rows=M, row_map=rows.to(torch.int32), out_f32=True)
+    assert torch.equal(got, F.gemm(x[rows], w, sizes, out_f32=True))
