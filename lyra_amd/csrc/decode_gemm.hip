@@ -2226,7 +2226,10 @@ int launch_planned(GemmParams p, const GemmPlan& pl, int layout, int fused_swigl
         // It addresses the activations with 31-bit offsets: they have to end below 2 GiB, which is not known of rows picked by
         // a map.
         const bool near_rows = !p.row_map && (size_t)M * K * 2 < (1ull << 31);
-        if (very_wide && !fused_swiglu && M > 64 && near_rows) {
+        // Its K loop runs on to a multiple of 128, where it multiplies what the offset "no load" gives by zeros: zeros, unless
+        // there are weights at that offset (2 GiB), which may be infinite.
+        const bool k_ends_in_zeros = K % 128 == 0 || (size_t)K * N * 2 <= (1ull << 31);
+        if (very_wide && !fused_swiglu && M > 64 && near_rows && k_ends_in_zeros) {
             const int mt = M > 96 ? 8 : 6;
             const size_t wide_lds = (size_t)2 * mt * 2048 + (tile_max ? (size_t)kWideWaves * 16 * mt * sizeof(float) : 0);
 #define LYRA_LAUNCH_WIDE(T, X) \

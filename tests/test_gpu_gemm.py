@@ -804,3 +804,20 @@ def test_lm_head_rows_picked_out_of_more_than_2_gib_of_activations():
     sizes = torch.full((1,), M, dtype=torch.int32, device=U.dev())
     got = F.gemm(x, w, sizes, rows=M, row_map=rows.to(torch.int32), out_f32=True)
     assert torch.equal(got, F.gemm(x[rows], w, sizes, out_f32=True))
+
+
+def test_lm_head_past_the_end_of_k_with_more_than_2_gib_of_weights():
+    """K rows that no weight row stands behind (K rounded up to 128) add nothing, infinite weights elsewhere or not."""
+    from lyra_amd.kernels import decode_fused as F
+
+    _note("gemm very wide, weights beyond 2 GiB")
+    K, N, M = 8224, 131200, 65
+    g = torch.Generator(device=U.dev()).manual_seed(65)
+    x = torch.randn(M, K, device=U.dev(), generator=g).to(torch.bfloat16)
+    w = torch.empty(1, K, N, device=U.dev(), dtype=torch.bfloat16).normal_(0.0, 0.02, generator=g)
+    w.view(-1)[1 << 30 : (1 << 30) + 4] = float("inf")  # (the first weights beyond 2 GiB: row 8184, columns 1024 to 1027)
+    size = lambda n: torch.full((1,), n, dtype=torch.int32, device=U.dev())
+    got = F.gemm(x, w, size(M), out_f32=True)
+    want = torch.cat([F.gemm(x[i : i + 64], w, size(min(64, M - i)), out_f32=True) for i in (0, 64)])
+    finite = torch.arange(N, device=U.dev()).sub(1024).div(4, rounding_mode="floor") != 0
+    assert torch.isfinite(got[:, finite]).all() and torch.equal(got[:, finite], want[:, finite])
