@@ -288,25 +288,29 @@ __device__ __forceinline__ void store_tile_max(const GemmParams& p, const float 
 
 constexpr int kTileMaxPitch = 20;  // floats per row of a wavefront's tile-maximum staging area (conflict-free for 4 rows x 16 lanes)
 
-template <int FP8, int MT, bool TMAX = false>
-__global__ __launch_bounds__(MT == 1 ? 768 : 512) __attribute__((amdgpu_waves_per_eu(MT == 1 ? 3 : 2)))
-void decode_gemm_kernel(GemmParams p) {
+// Element i of an array in global memory.  (Behind a loop's stores the compiler no longer sees that a pointer of the kernel's
+// arguments points there, and a load that might be from LDS makes it wait for everything in flight.)
+template <class T>
+__device__ __forceinline__ T global_at(const T* p, size_t i) {
+    return ((const T __attribute__((address_space(1)))*)p)[i];
+}
+
+// One wavefront's span of 128 columns (64 + 64 with SwiGLU) of group g: the row blocks rpar, rpar + row_par, ... over the K
+// slice ks.  Called by all nwaves wavefronts of a workgroup, which share the activations in LDS: sm_x [16 * MT rows][kGemmPitch],
+// then (TMAX) 16 * MT rows of kTileMaxPitch floats per wavefront.
+constexpr int kGemmChunk = 512;             // rows of K whose activations are staged in LDS at a time
+constexpr int kGemmPitch = kGemmChunk + 8;  // LDS pitch of a staged row in bf16 elements (keeps 16-lane reads conflict free)
+
+constexpr size_t gemm_lds_bytes(int mt, int waves, bool tile_max) {
+    return (size_t)16 * mt * kGemmPitch * sizeof(uint16_t) + (tile_max ? (size_t)waves * 16 * mt * kTileMaxPitch * sizeof(float) : 0);
+}
+
+template <int FP8, int MT, bool TMAX>
+__device__ __forceinline__ void gemm_span(const GemmParams& p, uint16_t* sm_x, int g, int rpar, int ks, int span, int end_span, int nwaves) {
     constexpr int ES = FP8 ? 1 : 2;
-    constexpr int KC = 512;          // rows of K whose activations are staged in LDS at a time
-    constexpr int XPITCH = KC + 8;   // LDS pitch of a staged row in bf16 elements (keeps 16-lane reads conflict free)
-    extern __shared__ uint16_t sm_x[];  // [16*MT rows][XPITCH] activations of the current K chunk, zero padded
+    constexpr int KC = kGemmChunk, XPITCH = kGemmPitch;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int x = lane & 15, kb = lane >> 4;
-    const int g = blockIdx.z / p.row_par, rpar = blockIdx.z - g * p.row_par, ks = blockIdx.y;
-    const int nwaves = blockDim.x >> 6;
-    // which 128-column span this wavefront owns: 4 per workgroup, or (p.even_spans, one workgroup per compute unit)
-    // workgroup i of n takes spans [i * total / n, (i + 1) * total / n), so that every compute unit has the same number
-    // of spans to within one - 1600 spans as 400 workgroups of 4 leave 144 compute units with 8 spans and 112 with 4
-    const int total_spans = p.swiglu ? ((p.N >> 1) + 63) / 64 : (p.N + 127) / 128;  // (the last span may be partly filled)
-    const int first_span = p.even_spans ? (int)((long)blockIdx.x * total_spans / gridDim.x) : (int)blockIdx.x * kGemmWaves;
-    const int end_span = p.even_spans ? (int)((long)(blockIdx.x + 1) * total_spans / gridDim.x) : total_spans;
-    const int span = first_span + wave;
-    // (TMAX: behind the activations, 16 * MT rows of kTileMaxPitch floats per wavefront)
     float* const sm_t = (float*)(sm_x + 16 * MT * XPITCH) + wave * (16 * MT * kTileMaxPitch);
 
     // rows of this group: [off, off + cnt)
@@ -433,7 +437,7 @@ void decode_gemm_kernel(GemmParams p) {
 
         float colscale[8], bias8[8];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) bias8[c] = (p.bias && p.ksplit == 1) ? p.bias[(size_t)g * p.N + ncol + c] : 0.f;
+        for (int c = 0; c < 8; ++c) bias8[c] = (p.bias && p.ksplit == 1) ? global_at(p.bias, (size_t)g * p.N + ncol + c) : 0.f;
 #pragma unroll
         for (int c = 0; c < 8; ++c) colscale[c] = s_cur;
         if (FP8 && p.scale_mode == 2) {
@@ -478,7 +482,7 @@ void decode_gemm_kernel(GemmParams p) {
     // rows at or beyond sum(group_sizes): zero product, bias of the last group (lax.ragged_dot semantics)
     float pad_bias8[8];
 #pragma unroll
-    for (int c = 0; c < 8; ++c) pad_bias8[c] = (p.bias && p.ksplit == 1 && pad_from < p.M) ? p.bias[(size_t)g * p.N + ncol + c] : 0.f;
+    for (int c = 0; c < 8; ++c) pad_bias8[c] = (p.bias && p.ksplit == 1 && pad_from < p.M) ? global_at(p.bias, (size_t)g * p.N + ncol + c) : 0.f;
     for (int row0 = pad_from; row0 < p.M; row0 += 4) {
         float t[8];
 #pragma unroll
@@ -486,6 +490,20 @@ void decode_gemm_kernel(GemmParams p) {
         finish_row(p, t, pad_bias8, row0 + kb, ncol, out_col, ks, span_ok && row0 + kb < p.M, is_lin_lane);
         if (TMAX) store_tile_max(p, t, row0 + kb, span, span_ok, span < end_span && row0 + kb < p.M && x == 0);
     }
+}
+
+template <int FP8, int MT, bool TMAX = false>
+__global__ __launch_bounds__(MT == 1 ? 768 : 512) __attribute__((amdgpu_waves_per_eu(MT == 1 ? 3 : 2)))
+void decode_gemm_kernel(GemmParams p) {
+    extern __shared__ uint16_t sm_x[];
+    const int g = blockIdx.z / p.row_par, rpar = blockIdx.z - g * p.row_par;
+    // which 128-column span a wavefront owns: 4 per workgroup, or (p.even_spans, one workgroup per compute unit)
+    // workgroup i of n takes spans [i * total / n, (i + 1) * total / n), so that every compute unit has the same number
+    // of spans to within one - 1600 spans as 400 workgroups of 4 leave 144 compute units with 8 spans and 112 with 4
+    const int total_spans = p.swiglu ? ((p.N >> 1) + 63) / 64 : (p.N + 127) / 128;  // (the last span may be partly filled)
+    const int first_span = p.even_spans ? (int)((long)blockIdx.x * total_spans / gridDim.x) : (int)blockIdx.x * kGemmWaves;
+    const int end_span = p.even_spans ? (int)((long)(blockIdx.x + 1) * total_spans / gridDim.x) : total_spans;
+    gemm_span<FP8, MT, TMAX>(p, sm_x, g, rpar, blockIdx.y, first_span + (threadIdx.x >> 6), end_span, blockDim.x >> 6);
 }
 
 // The epilogue of finish_row for 4 consecutive columns of one row (one group, K not split, no SwiGLU); t is left finished.
@@ -513,6 +531,9 @@ __device__ __forceinline__ void finish_quad(const GemmParams& p, float (&t)[4], 
 // Bound by the stream of weights: 2048 x 204800 at 65 / 96 / 128 rows 161 / 167 / 176 us (5.2-4.8 TB/s of weights; 296 / 303 /
 // 308 us before), 4096 x 204800 at 128 rows 323 us (589 before).  A wavefront of 128 columns and a whole SIMD's registers was
 // built first: 256 accumulators per lane left the compiler copying and spilling them in the K loop.
+// Up to 64 rows of a longer array (the device's row count decides) go the way of the kernel above, whose wavefronts are not in
+// step, so that their stores do not all come at once: 64 of 128 rows, 2048 x 204800 178 -> 164 us, 2880 x 201088 241 -> 204,
+// 4096 x 204800 314 -> 295.
 constexpr int kWideWaves = 8;
 
 template <int MT, bool TMAX>
@@ -532,6 +553,11 @@ void decode_gemm_wide_kernel(GemmParams p) {
     const int first_span = (int)((long)blockIdx.x * total_spans / gridDim.x), end_span = (int)((long)(blockIdx.x + 1) * total_spans / gridDim.x);
     const int rounds = (end_span - first_span + kWideWaves / 2 - 1) / (kWideWaves / 2);
     const int cnt = min(p.group_sizes[0], p.M);
+    if (cnt <= 64) {
+        for (int span = first_span; span < end_span; span += kWideWaves)
+            gemm_span<0, 4, TMAX>(p, (uint16_t*)sm_wide, 0, 0, 0, span + wave, end_span, kWideWaves);
+        return;
+    }
     const int row_blocks = (cnt + 16 * MT - 1) / (16 * MT);
     const int chunks = ((p.K + 63) / 64 + 1) & ~1;  // an even number: past the end of K zeros, without memory traffic
 
@@ -564,8 +590,7 @@ void decode_gemm_wide_kernel(GemmParams p) {
         for (int j = 0; j < PIECES; ++j) {
             const int lr = (int)(threadIdx.x >> 3) + 64 * j, row = block * 16 * MT + lr;
             const bool ok = block < row_blocks && row < cnt && lr < 16 * MT;
-            const int src = ok ? (p.row_map ? p.row_map[row] : row) : 0;
-            off[j] = ok ? (src * p.K + piece * 8) * 2 : kNoLoad;
+            off[j] = ok ? (row * p.K + piece * 8) * 2 : kNoLoad;
         }
     };
     auto stage_load = [&](const int (&off)[PIECES], int chunk) {
@@ -661,7 +686,7 @@ void decode_gemm_wide_kernel(GemmParams p) {
             const bool span_ok = span < end_span && ncol < p.N;
             float bias4[4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) bias4[c] = p.bias && span_ok ? p.bias[ncol + c] : 0.f;
+            for (int c = 0; c < 4; ++c) bias4[c] = p.bias && span_ok ? global_at(p.bias, ncol + c) : 0.f;
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
@@ -698,7 +723,7 @@ void decode_gemm_wide_kernel(GemmParams p) {
         const bool ok = ncol < p.N;
         float bias8[8];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) bias8[c] = p.bias && ok ? p.bias[ncol + c] : 0.f;
+        for (int c = 0; c < 8; ++c) bias8[c] = p.bias && ok ? global_at(p.bias, ncol + c) : 0.f;
         for (int row0 = cnt; row0 < p.M; row0 += 4) {
             float t[8];
 #pragma unroll
@@ -2231,9 +2256,15 @@ int launch_planned(GemmParams p, const GemmPlan& pl, int layout, int fused_swigl
         const bool k_ends_in_zeros = K % 128 == 0 || (size_t)K * N * 2 <= (1ull << 31);
         if (very_wide && !fused_swiglu && M > 64 && near_rows && k_ends_in_zeros) {
             const int mt = M > 96 ? 8 : 6;
-            const size_t wide_lds = (size_t)2 * mt * 2048 + (tile_max ? (size_t)kWideWaves * 16 * mt * sizeof(float) : 0);
-#define LYRA_LAUNCH_WIDE(T, X) \
-    hipLaunchKernelGGL((decode_gemm_wide_kernel<T, X>), dim3(kGroupMaxWgs), dim3(kWideWaves * 64), wide_lds, st, p)
+            const size_t wide_lds = std::max((size_t)2 * mt * 2048 + (tile_max ? (size_t)kWideWaves * 16 * mt * sizeof(float) : 0),
+                                             gemm_lds_bytes(4, kWideWaves, tile_max != nullptr));
+#define LYRA_LAUNCH_WIDE(T, X)                                                                                                    \
+    do {                                                                                                                          \
+        static const hipError_t attr = hipFuncSetAttribute((const void*)decode_gemm_wide_kernel<T, X>,                            \
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);               \
+        if (attr != hipSuccess) return LYRA_E_LAUNCH;                                                                             \
+        hipLaunchKernelGGL((decode_gemm_wide_kernel<T, X>), dim3(kGroupMaxWgs), dim3(kWideWaves * 64), wide_lds, st, p);          \
+    } while (0)
             if (mt == 6) {
                 if (tile_max) LYRA_LAUNCH_WIDE(6, true);
                 else LYRA_LAUNCH_WIDE(6, false);
@@ -2250,8 +2281,7 @@ int launch_planned(GemmParams p, const GemmPlan& pl, int layout, int fused_swigl
         grid = dim3(kGroupMaxWgs, 1, 1);
         block = dim3(per_cu * 64);
     }
-    const size_t lds = (size_t)16 * pl.mt * (512 + 8) * sizeof(uint16_t) +
-                       (tile_max ? (size_t)(block.x / 64) * 16 * pl.mt * kTileMaxPitch * sizeof(float) : 0);
+    const size_t lds = gemm_lds_bytes(pl.mt, (int)block.x / 64, tile_max != nullptr);
 #define LYRA_LAUNCH_GEMM(F, T)                                                                                         \
     do {                                                                                                               \
         if (tile_max) {                                                                                                \

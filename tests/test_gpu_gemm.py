@@ -821,3 +821,24 @@ def test_lm_head_past_the_end_of_k_with_more_than_2_gib_of_weights():
     want = torch.cat([F.gemm(x[i : i + 64], w, size(min(64, M - i)), out_f32=True) for i in (0, 64)])
     finite = torch.arange(N, device=U.dev()).sub(1024).div(4, rounding_mode="floor") != 0
     assert torch.isfinite(got[:, finite]).all() and torch.equal(got[:, finite], want[:, finite])
+
+
+@pytest.mark.parametrize("K,N,packed", [(1248, 131976, False), (640, 270088, True)])  # 1032 spans; 2111 (9 to a workgroup)
+@pytest.mark.parametrize("M,rows", [(65, 0), (65, 1), (97, 64), (130, 16), (300, 63)])
+def test_lm_head_of_more_than_64_rows_of_which_at_most_64_count(M, rows, K, N, packed):
+    """The device's row count may be far below the array's: bit for bit the call of 64 rows, then rows of the bias alone."""
+    from lyra_amd.kernels import decode_fused as F
+
+    _note(f"gemm very wide, padded, M={M} rows={rows} K={K} N={N}")
+    g = torch.Generator(device=U.dev()).manual_seed(M + rows)
+    x = torch.randn(M, K, generator=g, device=U.dev()).to(torch.bfloat16)
+    w = (torch.randn(1, K, N, generator=g, device=U.dev()) * 0.05).to(torch.bfloat16)
+    bias = torch.randn(N, generator=g, device=U.dev())
+    size = torch.full((1,), rows, dtype=torch.int32, device=U.dev())
+    rhs = F.pack_weights(w) if packed else w
+    logits, tiles = F.gemm_tile_max(x, rhs, size, bias=bias)
+    want, want_tiles = F.gemm_tile_max(x[:64].contiguous(), w, size, bias=bias)
+    pad = torch.nn.functional.pad(bias, (0, -N % 128), value=-float("inf")).view(-1, 128).amax(1)
+    assert torch.equal(logits[:64], want) and torch.equal(tiles[:64], want_tiles)
+    assert torch.equal(logits[rows:], bias.expand(M - rows, N)) and torch.equal(tiles[rows:], pad.expand(M - rows, -1))
+    assert torch.equal(F.gemm(x, rhs, size), F.gemm(x, rhs, size, out_f32=True).to(torch.bfloat16))
