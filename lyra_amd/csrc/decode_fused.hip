@@ -537,8 +537,9 @@ __global__ __launch_bounds__(256) void argmax_kernel(ArgmaxParams p) {
     int bi = 0x7FFFFFFF;
     // chunk_len % 4 == 0, ld % 4 == 0: aligned 16-byte loads through a descriptor of the row's `cols` columns (loads past it
     // return zeros); columns at or past `hi` are not compared.  Two blocks of four loads are in flight per thread: the launch
-    // is bound by the latency of its loads (two workgroups per compute unit).  64 / 96 / 128 rows x 201088 columns: 15.0 / 19.1 /
-    // 23.2 us with one block in flight and indices compared, 13.5 / 15.2 / 19.7 us (5.1 TB/s) now.
+    // is bound by the latency of its loads (two workgroups per compute unit).  64 / 96 / 128 rows x 201088 columns, launches one
+    // behind the other on rotating inputs: 15.0 / 22.4 / 27.5 us with one block in flight and indices compared, 13.8 / 16.5 /
+    // 22.7 us now (3.7 / 4.7 / 4.5 TB/s); masked rows (99.9 % -inf) 13.8 / 16.8 / 22.6.
     const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xr), 0, (uint32_t)p.cols * 4u, 0x00020000);
     const int blocks = (hi - lo + 4095) / 4096;
     u32x4 v[2][4];
@@ -564,13 +565,16 @@ __global__ __launch_bounds__(256) void argmax_kernel(ArgmaxParams p) {
             }
     };
     load(0, 0);
+    const int mine = lo + (int)threadIdx.x * 4;  // this thread's first column
+    const float first = __uint_as_float(v[0][0][0]);
     for (int b = 0; b < blocks; b += 2) {
         load(1, b + 1);
         compare(0, b);
         load(0, b + 2);
         compare(1, b + 1);
     }
-    if (bi == 0x7FFFFFFF) {  // nothing above -inf (a masked chunk): the first -inf counts, NaNs do not
+    if (bi == 0x7FFFFFFF && first == -INFINITY && mine < hi) bi = mine;  // nothing above -inf (masked columns): the first -inf counts
+    if (bi == 0x7FFFFFFF) {  // ... and NaNs do not
         for (int b = 0; b < blocks && bi == 0x7FFFFFFF; ++b) {
             load(0, b);
             const int i0 = lo + b * 4096 + (int)threadIdx.x * 4;

@@ -910,3 +910,20 @@ def test_argmax_first_of_ties_masked_rows_and_nans(rows, cols):
     dev = x.to("cuda:0")
     for _ in range(2):  # (the arrival counters are left zero)
         assert np.array_equal(argmax(dev, cols).cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("cols", [3, 4100, 12289, 201088])
+def test_argmax_masked_rows_whose_first_columns_are_nan(cols):
+    """A thread without any value above -inf: its first column counts if that is -inf, else its first -inf, else none."""
+    from lyra_amd.kernels.decode_fused import argmax
+
+    x = torch.full((4, (cols + 3) // 4 * 4 + 4), -float("inf"))
+    x[0, ::4] = float("nan")            # every thread's first column
+    x[1, : min(cols - 1, 4096)] = float("nan")  # a whole first block
+    x[2] = float("nan")                 # no column at all
+    x[3, cols - 1] = -3e38
+    x[:, cols:] = 99.0
+    want = [1, min(cols - 1, 4096), 0, cols - 1]
+    dev = x.to("cuda:0")
+    for _ in range(2):
+        assert argmax(dev, cols).tolist() == want
