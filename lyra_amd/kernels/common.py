@@ -39,7 +39,7 @@ def swiglu(x: torch.Tensor, beta: float = 1.702, limit: float = 7.0, shift: floa
     return ((lin + shift) * gate).to(dtype)
 
 
-_KERNEL_LOG_SEEN: set[str] = set()
+_KERNEL_LOG_SEEN: set = set()  # lines that are out, and the keys of the calls that go straight to their kernel since
 _KERNEL_LOG_ENABLED = os.environ.get("LYRA_LOG_KERNELS", "1") != "0"
 
 
@@ -55,9 +55,15 @@ def log_kernel_resolution(op: str, *, shape: str, impl: str, tiling: str | None 
     print(f"[kernel] {op:<15} {shape:<26} -> {detail}", file=sys.stderr)
 
 
-def kernel_decided(implementation: Implementation, config: object | None) -> bool:
-    """Whether ``dispatch_kernel`` would run the kernel and say nothing: the caller may then skip its strings and closures."""
-    return config is not None and not _KERNEL_LOG_ENABLED and implementation in ("auto", "pallas", "hip")
+def kernel_log_done(key: tuple) -> bool:
+    """Whether the line of the calls that ``key`` stands for is out, or is not wanted."""
+    return not _KERNEL_LOG_ENABLED or key in _KERNEL_LOG_SEEN
+
+
+def kernel_decided(implementation: Implementation, config: object | None, key: tuple) -> bool:
+    """Whether ``dispatch_kernel`` would run the kernel and say nothing: the caller may then skip its strings and closures.
+    ``key`` (operator, shape and types) is the one given to ``dispatch_kernel`` when it did say something."""
+    return config is not None and kernel_log_done(key) and implementation in ("auto", "pallas", "hip")
 
 
 def dispatch_kernel(
@@ -70,6 +76,7 @@ def dispatch_kernel(
     kernel: Callable[[], torch.Tensor],
     reference: Callable[[], torch.Tensor],
     fallback_reason: str | None = None,
+    key: tuple | None = None,
 ) -> torch.Tensor:
     """lyra/kernels/common.py:132-155 with "hip" for "pallas" in messages."""
     if implementation not in ("auto", "pallas", "xla", "hip"):
@@ -77,6 +84,8 @@ def dispatch_kernel(
     if config is not None and implementation != "xla":
         assert tiling is not None
         log_kernel_resolution(op, shape=shape, impl="hip", tiling=tiling)
+        if key is not None:
+            _KERNEL_LOG_SEEN.add(key)
         return kernel()
     if implementation in ("pallas", "hip"):
         raise ValueError(

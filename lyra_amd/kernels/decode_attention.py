@@ -274,7 +274,8 @@ def decode_attention(
 
     if (xsa_v is None) != (xsa_alpha is None):
         raise ValueError("xsa_v and xsa_alpha go together")
-    if kernel_decided(implementation, config):
+    key = ("decode_attention", B, N, K, S, H, int(sliding_window), cache_dtype)
+    if kernel_decided(implementation, config, key):
         return _decode_attention(q, k, v, sinks, sm_scale, sliding_window, position, config, dtype, gate=gate,
                                  xsa_v=xsa_v, xsa_alpha=xsa_alpha, row_order=row_order)
 
@@ -297,4 +298,5 @@ def decode_attention(
         tiling=tiling,
         kernel=kernel,
         reference=reference,
+        key=key,
     )

@@ -13,7 +13,7 @@ from dataclasses import dataclass
 import torch
 
 from lyra_amd import _lib
-from lyra_amd.kernels.common import Implementation, dispatch_kernel, kernel_decided, log_kernel_resolution, swiglu
+from lyra_amd.kernels.common import Implementation, dispatch_kernel, kernel_decided, kernel_log_done, swiglu
 from lyra_amd.nn.quant import QArray, dequantize, is_scaled, quantize
 
 
@@ -58,15 +58,14 @@ _config_of = functools.lru_cache(maxsize=4096)(select_decode_gemm_config)
 
 def one_group(lhs, rhs, quant_dtype, out_dtype):
     """lhs [M, K] bf16 times rhs [1, K, N] (bf16 or QArray, contiguous scales and codes not required) to ``out_dtype`` (bf16 or
-    float32) on the kernel, or None where it has no configuration for the shape.  What ``decode_gemm`` does with one group of
-    all rows, without the casts to and from float32 that its output type costs there."""
+    float32) on the kernel, or None where it has no configuration for the shape or the shape's log line is still to come.
+    What ``decode_gemm`` does with one group of all rows, without the casts to and from float32 that its output type costs there."""
     M = lhs.shape[0]
     _, K, N = rhs.shape
     block = tuple(rhs.block) if isinstance(rhs, QArray) else None
     config = _config_of(M, 1, K, N, quant_dtype, block, False)
-    if config is None:
+    if config is None or not kernel_log_done(("decode_gemm", M, 1, K, N, config.fwd_dtype)):  # (decode_gemm has the line)
         return None
-    log_kernel_resolution("decode_gemm", shape=f"m{M} g1 k{K} n{N}", impl="hip", tiling=f"n8/k32 dtype={'fp8' if quant_dtype else 'bf16'}")
     return _decode_gemm(lhs, rhs, _lib.row_count(M, lhs.device), config, bias=None, fused_swiglu=False, swiglu_beta=1.702,
                         swiglu_limit=7.0, out_dtype=out_dtype)
 
@@ -214,7 +213,8 @@ def decode_gemm(
         if lhs.is_cuda
         else None
     )
-    if kernel_decided(implementation, config):
+    key = ("decode_gemm", M, G, K, N, dtype)
+    if kernel_decided(implementation, config, key):
         return _decode_gemm(
             lhs, rhs_kernel, group_sizes, config, bias=bias, fused_swiglu=fused_swiglu,
             swiglu_beta=swiglu_beta, swiglu_limit=swiglu_limit, out_dtype=out_dtype,
@@ -236,5 +236,6 @@ def decode_gemm(
     tiling = None if config is None else f"n8/k32 dtype={'fp8' if config.fwd_dtype else 'bf16'}"
     op_shape = f"m{M} g{G} k{K} n{N}"
     return dispatch_kernel(
-        "decode_gemm", implementation=implementation, shape=op_shape, config=config, tiling=tiling, kernel=kernel, reference=reference
+        "decode_gemm", implementation=implementation, shape=op_shape, config=config, tiling=tiling, kernel=kernel, reference=reference,
+        key=key,
     )

@@ -842,3 +842,35 @@ def test_lm_head_of_more_than_64_rows_of_which_at_most_64_count(M, rows, K, N, p
     assert torch.equal(logits[:64], want) and torch.equal(tiles[:64], want_tiles)
     assert torch.equal(logits[rows:], bias.expand(M - rows, N)) and torch.equal(tiles[rows:], pad.expand(M - rows, -1))
     assert torch.equal(F.gemm(x, rhs, size), F.gemm(x, rhs, size, out_f32=True).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("log", [True, False])
+def test_operator_calls_go_straight_to_the_kernel_once_their_line_is_out(log, monkeypatch, capsys):
+    """With the log on, a shape's first call prints its line; from then on, and from the start with the log off, the operators
+    launch without a dispatch - the same bits on either way."""
+    from lyra_amd.kernels import common
+    from lyra_amd.kernels import decode_attention as A
+    from lyra_amd.kernels import decode_gemm as G
+    from lyra_amd.nn.quant import dot
+
+    monkeypatch.setattr(common, "_KERNEL_LOG_ENABLED", log)
+    monkeypatch.setattr(common, "_KERNEL_LOG_SEEN", set())
+    _note(f"direct path log={log}")
+    g = torch.Generator(device=U.dev()).manual_seed(5)
+    draw = lambda *s: torch.randn(*s, device=U.dev(), generator=g).to(torch.bfloat16)
+    x, w, experts, sizes = draw(7, 96), draw(96, 72), draw(3, 96, 72), torch.tensor([3, 0, 4], dtype=torch.int32, device=U.dev())
+    q, k, v, sinks = draw(2, 4, 1, 64), draw(2, 2, 40, 64), draw(2, 2, 40, 64), torch.zeros(4, device=U.dev())
+    calls = [
+        lambda: dot(x, w), lambda: dot(x, w, preferred_element_type=torch.float32), lambda: G.decode_gemm(x, experts, sizes),
+        lambda: A.decode_attention(q, k, v, sinks, 0.125, 0, 39),
+    ]
+    first = [call() for call in calls]
+
+    def refuse(*_, **__):
+        raise AssertionError("a dispatch")
+
+    monkeypatch.setattr(G, "dispatch_kernel", refuse)
+    monkeypatch.setattr(A, "dispatch_kernel", refuse)
+    assert all(torch.equal(call(), want) for call, want in zip(calls, first))
+    lines = [line for line in capsys.readouterr().err.splitlines() if line.startswith("[kernel]")]
+    assert len(lines) == (3 if log else 0)  # (both products of the projection's shape have one)

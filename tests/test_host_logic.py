@@ -407,3 +407,27 @@ def test_one_group_of_a_step_is_not_kept_from_a_stand_in():
         model._one_group(1237, torch.device("cpu"))
     after = model._one_group(1237, torch.device("cpu"))
     assert type(after) is torch.Tensor and after.dtype == torch.int32 and after.tolist() == [1237]
+
+
+@pytest.mark.parametrize("enabled", [True, False])
+def test_direct_path_from_the_second_call_on_with_the_log_on_and_off(enabled, monkeypatch, capsys):
+    """A call whose log line is out (or is not wanted) goes to its kernel without the strings and closures of a dispatch."""
+    from lyra_amd.kernels import common
+
+    monkeypatch.setattr(common, "_KERNEL_LOG_ENABLED", enabled)
+    monkeypatch.setattr(common, "_KERNEL_LOG_SEEN", set())
+    key, other = ("op", 3, 64), ("op", 4, 64)
+    run = lambda key, shape, **kw: common.dispatch_kernel("op", shape=shape, tiling="t", key=key, kernel=lambda: 1, reference=lambda: 2, **kw)
+    config = object()
+    assert common.kernel_decided("auto", config, key) == (not enabled)
+    assert run(key, "m3", implementation="auto", config=config) == 1
+    for implementation in ("auto", "pallas", "hip"):
+        assert common.kernel_decided(implementation, config, key)
+        assert common.kernel_decided(implementation, config, other) == (not enabled)
+    assert not common.kernel_decided("xla", config, key) and not common.kernel_decided("auto", None, key)
+    assert not common.kernel_decided("cuda", config, key)
+    run(key, "m3", implementation="pallas", config=config)
+    assert run(other, "m4", implementation="xla", config=config) == 2
+    assert common.kernel_decided("auto", config, other) == (not enabled)  # (the plain path says nothing about the kernel's)
+    lines = capsys.readouterr().err.splitlines()
+    assert [line.split("->")[1].strip() for line in lines] == (["hip    t", "xla"] if enabled else [])
