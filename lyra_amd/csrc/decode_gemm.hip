@@ -1470,6 +1470,12 @@ __global__ __launch_bounds__(kSplitWaves * 64) void decode_gemm_group_kernel(Gem
 
     // state of the work item whose operands are in flight / being consumed
     int v = wg, round = 0;  // (v = round * nwg + wg)
+    if (p.deal_mask && n_whole == 0) {
+        // fewer items than workgroups: an even run of them for every XCD, and not the first XCDs full and the last ones idle
+        // (2048 x 2832 in bf16, 170 units: 26.5 -> 23.8 us)
+        const int xcd = (int)(blockIdx.x & 7), mine = xcd * n_work / 8 + (int)(blockIdx.x >> 3);
+        v = mine < (xcd + 1) * n_work / 8 ? mine : n_work;
+    }
     bool seg_valid = false;
     int seg_u = 0, seg_r0 = 0, seg_r1 = 0;  // its unit and trips [r0, r1) of it
     int g = 0, row0 = 0, rows = 0, span = 0, ncol = 0, wvoff = kNoLoad, avoff[MTM];
@@ -2142,9 +2148,11 @@ int launch_planned(GemmParams p, const GemmPlan& pl, int layout, int fused_swigl
         const long trips_least = std::max(1, ((K / 32 + gkw - 1) / gkw + 7) / 8);  // trips per unit (at least)
         const dim3 ggrid((unsigned)std::max(1L, std::min((long)kGroupMaxWgs, most_units * trips_least))), gblock(kSplitWaves * 64);
         // Row-major pieces of 128 columns that do not start on a 128-byte line: the line in which two neighbouring units meet is
-        // fetched once if both run behind one L2 and twice if not (gpt-oss-20b in FP8, 33 tokens: up 117 -> 101 us, down
-        // 65 -> 58).  Where no line is shared, neighbouring units on different XCDs are the faster ones: lyra-small in bf16 at
-        // 7 tokens 57 us for both launches against 69, lyra-medium at 64 tokens 299 against 308.
+        // fetched once if both run behind one L2 and twice if not (gpt-oss-20b in FP8, both launches at 1 / 2 / 4 / 8 / 33 / 128
+        // tokens: 46 / 64 / 114 / 137 / 197 / 215 us, in runs per XCD 43 / 57 / 98 / 116 / 168 / 189; 2048 x 2832 and 1416 wide in
+        // bf16, 32 experts, 2 / 32 tokens: 55 / 173 -> 51 / 157).  Where no line is shared, neighbouring units on different XCDs
+        // are the faster ones: lyra-small in bf16 at 7 tokens 57 us for both launches against 69, lyra-medium at 64 tokens 299
+        // against 308.
         const int es = fp8 ? 1 : 2;
         if (!layout && (N * es % 128 || (fused_swiglu && N / 2 * es % 128)) && ggrid.x % 8 == 0) {
             p.deal_mask = 7;

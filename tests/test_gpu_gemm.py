@@ -874,3 +874,20 @@ def test_operator_calls_go_straight_to_the_kernel_once_their_line_is_out(log, mo
     assert all(torch.equal(call(), want) for call, want in zip(calls, first))
     lines = [line for line in capsys.readouterr().err.splitlines() if line.startswith("[kernel]")]
     assert len(lines) == (3 if log else 0)  # (both products of the projection's shape have one)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp8"])
+@pytest.mark.parametrize("K,N,swiglu,blocks", [
+    (512, 2832, False, 1), (512, 2832, False, 5), (96, 2832, False, 11), (96, 2832, False, 12),  # 23 units to a row block: cut into slices, 253, 276
+    (512, 2832, True, 3), (96, 2832, True, 21), (96, 2832, True, 22), (96, 200, False, 3),       # 12 units: 36 in slices, 252, 264; 2 units
+])
+def test_fewer_units_than_workgroups_dealt_out_in_even_runs(kind, K, N, swiglu, blocks):
+    """Widths off the 128-byte line with just under, and just over, one round of units, and with units cut into K slices: every
+    unit is taken once, whatever its place."""
+    sizes = np.zeros(blocks + 2, np.int32)
+    sizes[1 : blocks + 1] = np.arange(blocks) % 5 + 1
+    M = int(sizes.sum()) + 1
+    c = _case(97 + N + blocks, M, sizes.size, K, N, sizes, kind=kind, block=(K, 1), bias=True, w_std=0.05)
+    first = _run(c, swiglu)
+    U.assert_close(first, _want(c, swiglu, big=True), what="units in even runs")
+    assert np.array_equal(_run(c, swiglu), first)
