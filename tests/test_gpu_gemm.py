@@ -891,3 +891,33 @@ def test_fewer_units_than_workgroups_dealt_out_in_even_runs(kind, K, N, swiglu, 
     first = _run(c, swiglu)
     U.assert_close(first, _want(c, swiglu, big=True), what="units in even runs")
     assert np.array_equal(_run(c, swiglu), first)
+
+
+@pytest.mark.parametrize("M,rows,K,N,packed", [(65, 65, 1248, 131976, False), (96, 80, 1280, 131080, True), (130, 129, 1248, 131200, False), (257, 257, 640, 270088, False)])
+def test_lm_head_of_more_than_64_rows_with_every_epilogue(M, rows, K, N, packed):
+    """bf16 and float32 results, no bias, a bias before and after the cast, scale and residual, rows picked by a map (some of
+    them twice), and more than two rounds of spans per workgroup (270088 columns): bit for bit the calls of at most 64 rows."""
+    from lyra_amd.kernels import decode_fused as F
+
+    _note(f"gemm very wide, epilogues, M={M} rows={rows} K={K} N={N} packed={packed}")
+    g = torch.Generator(device=U.dev()).manual_seed(M + N)
+    x = torch.randn(M, K, generator=g, device=U.dev()).to(torch.bfloat16)
+    w = (torch.randn(1, K, N, generator=g, device=U.dev()) * 0.05).to(torch.bfloat16)
+    rhs = F.pack_weights(w) if packed else w
+    bias = torch.randn(N, generator=g, device=U.dev())
+    residual = torch.randn(M, N, generator=g, device=U.dev()).to(torch.bfloat16)
+    row_map = torch.randint(0, M, (M,), generator=g, device=U.dev()).to(torch.int32)
+    row_map[: M // 2] = row_map[M // 2 : M // 2 * 2]
+    size = lambda n: torch.full((1,), n, dtype=torch.int32, device=U.dev())
+    options = [dict(), dict(out_f32=True), dict(bias=bias, out_f32=True), dict(bias=bias.to(torch.bfloat16).float(), bias_after_cast=True),
+               dict(residual=residual, out_scale=0.4375), dict(out_scale=0.25, bias=bias.to(torch.bfloat16).float(), bias_after_cast=True, residual=residual),
+               dict(row_map=row_map, out_f32=True)]
+    for kw in options:
+        got = F.gemm(x, rhs, size(rows), rows=M, **kw)
+        part = []
+        for i in range(0, M, 64):
+            n = min(64, M - i)
+            cut = {k: (v[i : i + n].contiguous() if k in ("residual", "row_map") else v) for k, v in kw.items()}
+            lhs = x if "row_map" in kw else x[i : i + n].contiguous()
+            part.append(F.gemm(lhs, w, size(max(0, min(n, rows - i))), rows=n, **cut))
+        assert torch.equal(got, torch.cat(part)), f"{sorted(kw)}: differs"
