@@ -313,12 +313,13 @@ __device__ __forceinline__ void gemm_span(const GemmParams& p, uint16_t* sm_x, i
     const int x = lane & 15, kb = lane >> 4;
     float* const sm_t = (float*)(sm_x + 16 * MT * XPITCH) + wave * (16 * MT * kTileMaxPitch);
 
-    // rows of this group: [off, off + cnt)
+    // rows of this group: [off, off + cnt) (a count below zero is taken as none: the rows past the last group would
+    // otherwise begin before the first)
     int part_sum = 0;
-    for (int i = lane; i < g; i += 64) part_sum += p.group_sizes[i];
+    for (int i = lane; i < g; i += 64) part_sum += max(0, p.group_sizes[i]);
     part_sum = wave_sum(part_sum);
     const int off = min(part_sum, p.M);
-    const int cnt = min(p.group_sizes[g], p.M - off);
+    const int cnt = max(0, min(p.group_sizes[g], p.M - off));
     const int pad_from = (g == p.G - 1 && rpar == 0 && p.ksplit == 1 && ks == 0) ? off + cnt : p.M;  // rows past the last group
     if (cnt <= rpar * 16 * MT && pad_from >= p.M) return;  // no rows for this workgroup: its weights are never touched
 
@@ -770,7 +771,7 @@ __global__ __launch_bounds__(256) void decode_gemm_finish_kernel(GemmParams p) {
     }
     int total = 0, g = p.G - 1;
     for (int i = 0; i < p.G; ++i) {
-        const int nt = total + p.group_sizes[i];
+        const int nt = total + max(0, p.group_sizes[i]);
         if (row >= total && row < nt) g = i;
         total = nt;
     }
@@ -1378,7 +1379,7 @@ __global__ __launch_bounds__(kSplitWaves * 64) void decode_gemm_group_kernel(Gem
     int my_cnt = 0, my_before = 0;  // rows of "my" group and rows of all groups before it (in lhs order)
     int total_rows;
     {
-        const int v = t < p.G ? p.group_sizes[t] : 0;
+        const int v = t < p.G ? max(0, p.group_sizes[t]) : 0;
         // The list starts with the row blocks of the last group, which is where a model keeps its shared expert: every
         // token has a row there, so the units with the most rows - the ones that decide how long the launch lasts - are
         // known before the group sizes are.  The workgroups that own them if that holds touch the lines of their first

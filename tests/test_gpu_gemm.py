@@ -921,3 +921,17 @@ def test_lm_head_of_more_than_64_rows_with_every_epilogue(M, rows, K, N, packed)
             lhs = x if "row_map" in kw else x[i : i + n].contiguous()
             part.append(F.gemm(lhs, w, size(max(0, min(n, rows - i))), rows=n, **cut))
         assert torch.equal(got, torch.cat(part)), f"{sorted(kw)}: differs"
+
+
+@pytest.mark.parametrize("M,K,N,G", [(3, 64, 131200, 1), (65, 1248, 131976, 1), (9, 64, 8, 300), (9, 512, 136, 300), (9, 96, 328, 8), (5, 2048, 512, 1)])
+def test_row_counts_below_zero_count_as_none(M, K, N, G):
+    """The general kernel, the very wide one, the one for several groups and the K-split one write nothing before the first row."""
+    from lyra_amd.kernels import decode_fused as F
+
+    _note(f"gemm negative count M={M} K={K} N={N} G={G}")
+    g = torch.Generator(device=U.dev()).manual_seed(G)
+    x = torch.randn(M, K, generator=g, device=U.dev()).to(torch.bfloat16)
+    w = torch.randn(G, K, N, generator=g, device=U.dev()).to(torch.bfloat16)
+    sizes = torch.full((G,), -1000, dtype=torch.int32, device=U.dev())
+    sizes[G // 2 + 1 : G // 2 + 2] = 4
+    assert torch.equal(F.gemm(x, w, sizes, out_f32=True), F.gemm(x, w, sizes.clamp(min=0), out_f32=True))
