@@ -84,7 +84,7 @@ struct GemmParams {
     // one matrix instruction with 16 consecutive rows then read one contiguous KB instead of 16 pieces a row apart.
     // lhs_tiled: lhs comes in that layout (grouped kernel); out_tiled: the bf16 output is written in it (for the next matmul).
     int lhs_tiled, out_tiled;
-    // Plain kernel, one group, float32 output, K not split: the maximum of every 128-column tile of every output row,
+    // General and very wide kernel, one group, float32 output, K not split: the maximum of every 128-column tile of every output row,
     // [M, tile_ld] float32 (tile t = columns 128 t ...; NaNs are skipped as fmaxf skips them), for a sampler that then
     // only looks into the few tiles that can hold a row's best values.  Null: not wanted.
     float* tile_max;
@@ -529,8 +529,8 @@ __device__ __forceinline__ void finish_quad(const GemmParams& p, float (&t)[4], 
 // in the order the matrix instruction takes them (tiles of 16 rows x 32 K of 1 KB), so that the wavefronts fetch them once
 // and read them without bank conflicts: slot (kb, x ^ (2 kb + step)) holds row x, K group kb - the exclusive-or keeps the 8
 // lanes that write one row's pieces on different banks.
-// Bound by the stream of weights: 2048 x 204800 at 65 / 96 / 128 rows 161 / 167 / 176 us (5.2-4.8 TB/s of weights; 296 / 303 /
-// 308 us before), 4096 x 204800 at 128 rows 323 us (589 before).  A wavefront of 128 columns and a whole SIMD's registers was
+// Bound by the stream of weights: 2048 x 204800 at 65 / 96 / 128 rows 163 / 169 / 180 us (5.1-4.7 TB/s of weights; 297 / 304 /
+// 308 us before), 4096 x 204800 at 128 rows 328 us (590 before); one box runs up to 4 % above or below another.  A wavefront of 128 columns and a whole SIMD's registers was
 // built first: 256 accumulators per lane left the compiler copying and spilling them in the K loop.
 // Up to 64 rows of a longer array (the device's row count decides) go the way of the kernel above, whose wavefronts are not in
 // step, so that their stores do not all come at once: 64 of 128 rows, 2048 x 204800 178 -> 164 us, 2880 x 201088 241 -> 204,
@@ -2254,9 +2254,10 @@ int launch_planned(GemmParams p, const GemmPlan& pl, int layout, int fused_swigl
     const int per_cu = (pl.spans + kGroupMaxWgs - 1) / kGroupMaxWgs;
     const bool very_wide = !no_even && G == 1 && pl.ksplit == 1 && pl.row_par == 1 && pl.spans >= 4 * kGroupMaxWgs;
     if constexpr (WT == 0) {
-        // More than 64 rows of bf16 weights: the kernel that streams them once per 128 rows (2048 x 204800: 161-176 us at 65
-        // to 128 rows, where the kernel below streams them twice in 296-308 us; up to 64 rows the one below is the faster,
-        // 151 against 157 us at 64 and 134 against 142 at 1: it stages the activations once per 512 K rows, not per 64).
+        // More than 64 rows of bf16 weights: the kernel that streams them once per 128 rows (2048 x 204800: 163-180 us at 65
+        // to 128 rows, where the kernel below streams them twice in 297-308 us; 129 rows 350 against 462, 256 rows 375 against 640.
+        // Up to 64 rows the one below is the faster, 151 against 157 us at 64 and 134 against 142 at 1: it stages the activations
+        // once per 512 K rows, not per 64).
         // It addresses the activations with 31-bit offsets: they have to end below 2 GiB, which is not known of rows picked by
         // a map.
         const bool near_rows = !p.row_map && (size_t)M * K * 2 < (1ull << 31);
@@ -2464,7 +2465,8 @@ static int run_decode_gemm(const void* lhs, const int32_t* lhs_row_map, const vo
     if (out_tiled && (out_dtype != LYRA_DTYPE_BF16 || residual || (fused_swiglu ? N / 2 : N) % 32)) return LYRA_E_UNSUPPORTED;
     p.lhs_tiled = lhs_tiled;
     p.out_tiled = out_tiled;
-    // tile maxima: what the plain kernel's epilogue can give - every (row, span) finished by one wavefront, in float32
+    // tile maxima: what the general kernel's epilogue can give (every (row, span) finished by one wavefront, in float32) and the
+    // very wide kernel's (by two, which meet in LDS)
     if (tile_max && (G != 1 || pl.grouped || pl.split_k || pl.one_pass || pl.ksplit > 1 || fused_swiglu ||
                      out_dtype != LYRA_DTYPE_F32 || post_scale || bias_post))
         return LYRA_E_UNSUPPORTED;
