@@ -37,14 +37,15 @@ struct AttnParams {
     int pos_stride;
     const uint16_t* gate;
     void* out;
-    float* part_o;   // [B,K,n_chunks,G,H]
-    float* part_ml;  // [B,K,n_chunks,G,2]
+    float* part_o;   // [chunked pairs,n_chunks,G,H]
+    float* part_ml;  // [chunked pairs,n_chunks,G,2]
     int* arrivals;   // [B,K] zero on entry, zero again on exit
     int B, N, K, S, G;
     float scale_log2;  // sm_scale * log2(e)
     int sw;
     int chunk;     // tokens per workgroup, multiple of 128
-    int n_chunks;  // grid.x
+    int n_chunks;  // workgroups per chunked (batch row, kv head) pair; grid.x unless whole > 0
+    int whole;     // > 0: one-dimensional grid, the pairs below `whole` are one workgroup each, the others n_chunks each
     int out_f32;
     int scale_vec4;  // S % 4 == 0 -> scales are fetched as float4
     // learned exclusive self attention (lyra/model.py:351-363), both null when the model has none
@@ -519,9 +520,24 @@ void decode_attention_kernel(AttnParams p) {
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int x = lane & 15, kb = lane >> 4;
-    const int c_idx = blockIdx.x;
+    int c_idx = blockIdx.x, n_chunks = p.n_chunks, chunk = p.chunk;
     int kh = blockIdx.y, b = blockIdx.z;
     const int G = p.G;
+    if (EARLY && __builtin_expect(p.whole > 0, 0)) {  // (out of the way: falling through costs the others nothing)
+        int pair = (int)blockIdx.x;
+        if (pair < p.whole) {
+            c_idx = 0;
+            n_chunks = 1;
+            chunk = p.S;
+        } else {
+            const int i = pair - p.whole, q = i / n_chunks;
+            c_idx = i - q * n_chunks;
+            pair = p.whole + q;
+        }
+        b = __builtin_amdgcn_readfirstlane(pair / p.K);
+        kh = __builtin_amdgcn_readfirstlane(pair - b * p.K);
+        c_idx = __builtin_amdgcn_readfirstlane(c_idx);
+    }
     if (p.row_order) {
         // Workgroups are started in the order of their linear index (kv head fastest), 256 at a time, one per compute
         // unit: workgroup L of a round shares its unit with workgroup L of the next.  Pairs are ranked by length (row
@@ -585,7 +601,7 @@ void decode_attention_kernel(AttnParams p) {
     if constexpr (early) {
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
-            const int early_base = c_idx * p.chunk + (tile + d * WAVES) * kTile;
+            const int early_base = c_idx * chunk + (tile + d * WAVES) * kTile;
             load_k<H, FP8>(rk[d], sl, early_base, true);
             if constexpr (FP8) load_s<VEC4>(rs[d], sl, early_base, true);
             load_v<H, FP8>(rv[d], sl, early_base, true);
@@ -608,7 +624,7 @@ void decode_attention_kernel(AttnParams p) {
 
     const int pos = __builtin_amdgcn_readfirstlane((int)pos_raw);  // (waited for here, with everything above in flight)
     const Range rg = visible_range(pos, p.sw, p.S);
-    const int c_lo = rg.start + c_idx * p.chunk;
+    const int c_lo = rg.start + c_idx * chunk;
     if (c_lo > rg.hi) {  // chunk holds no visible key (whole workgroup leaves together)
         // First chunk empty = no chunk of this row holds a key (position < 0): only the sink is attended and its value is
         // 0.  No workgroup of the row then reaches the merge, so the first one writes the zeros, however many chunks the
@@ -619,12 +635,12 @@ void decode_attention_kernel(AttnParams p) {
         wait_all_memory();
         return;
     }
-    const int c_hi = min(c_lo + p.chunk, rg.hi + 1);
+    const int c_hi = min(c_lo + chunk, rg.hi + 1);
     const int n_tiles = (c_hi - c_lo + kTile - 1) / kTile;
     // QKV: this workgroup appends the new token's key and value when its chunk holds them, through the wavefront that
     // reads that key's tile (kv_wave); when the tile is that wavefront's first, it is requested a second time after the
     // rows have been written (`redo`).
-    [[maybe_unused]] const bool owner = QKV && pos >= 0 && pos < p.S && pos >= c_lo && pos < c_lo + p.chunk;
+    [[maybe_unused]] const bool owner = QKV && pos >= 0 && pos < p.S && pos >= c_lo && pos < c_lo + chunk;
     [[maybe_unused]] const int kv_wave = owner ? ((pos - c_lo) / kTile) % WAVES : -1;
     [[maybe_unused]] const bool redo = owner && wave == kv_wave && (pos - c_lo) / kTile < WAVES;
     [[maybe_unused]] float rope_cs = 0.f, rope_sn = 0.f;
@@ -772,7 +788,7 @@ void decode_attention_kernel(AttnParams p) {
     }
     __syncthreads();
 
-    const bool final_out = p.n_chunks == 1;
+    const bool final_out = n_chunks == 1;
     for (int idx = threadIdx.x; idx < G * H; idx += WAVES * 64) {
         const int g = idx / H, col = idx - g * H;
         float mm = sm_m[g];
@@ -791,7 +807,7 @@ void decode_attention_kernel(AttnParams p) {
             if (p.xsa_v) smem[p.xsa_lds + idx] = gated(p, o / den, sm_gate[g]);
             else store_out(p, ((size_t)b * p.N + n) * H + col, o / den, sm_gate[g]);
         } else {
-            const size_t item = ((size_t)b * p.K + kh) * p.n_chunks + c_idx;
+            const size_t item = (size_t)(b * p.K + kh - p.whole) * n_chunks + c_idx;
             store_agent(p.part_o + (item * G + g) * H + col, o);
             if (col == 0) {
                 store_agent(p.part_ml + (item * G + g) * 2, mm);
@@ -805,7 +821,7 @@ void decode_attention_kernel(AttnParams p) {
     }
 
     // ---- merge the chunks: the workgroup that arrives last reads every partial of this kv head ----
-    const int n_valid = min((rg.hi + 1 - rg.start + p.chunk - 1) / p.chunk, p.n_chunks);
+    const int n_valid = min((rg.hi + 1 - rg.start + chunk - 1) / chunk, n_chunks);
     __shared__ int sm_last;
     wait_all_memory();  // this lane's partials have reached device-wide visibility
     __syncthreads();    // ... and so have everybody else's in this workgroup, before the arrival is counted
@@ -818,7 +834,7 @@ void decode_attention_kernel(AttnParams p) {
     if (!sm_last) return;
     // weights of the chunks: every thread fetches one (max, sum) pair, then LDS holds exp2(m_c - m*) and the
     // denominator per head; the output columns are then gathered with all loads of a thread in flight at once
-    const size_t item0 = ((size_t)b * p.K + kh) * p.n_chunks;
+    const size_t item0 = (size_t)(b * p.K + kh - p.whole) * n_chunks;
     float* sm_w = smem;                 // [n_valid][G] weight of chunk c for head g
     float* sm_den = smem + 1024;        // [G]
     float* sm_cm = smem + 1024 + 16;    // [n_valid][G] chunk maxima
@@ -1082,12 +1098,22 @@ void decode_attention_rows_kernel(AttnParams p) {
 // ---- host side ---------------------------------------------------------------------------------
 struct AttnPlan {
     int chunk, n_chunks, waves;
+    int whole = 0;  // AttnParams::whole
 };
 constexpr long kMaxSplitPairs = 16384;  // (batch row, kv head) pairs beyond which a launch is never chunked
 
 static long env_long(const char* name) {
     const char* e = getenv(name);
     return e ? atol(e) : 0L;
+}
+
+// n chunks (or as many as there are passes of the workgroup's wavefronts) over `span` keys
+static void cut_chunks(AttnPlan& pl, int span, long n) {
+    const int unit = pl.waves * kTile;
+    const int n_chunks = (int)std::max(1L, std::min((long)((span + unit - 1) / unit), n));
+    const int chunk = ((span + n_chunks - 1) / n_chunks + unit - 1) / unit * unit;
+    pl.n_chunks = (span + chunk - 1) / chunk;
+    pl.chunk = chunk;
 }
 
 // Split so that the launch fills the 256 compute units even at small batch, never below one pass of the
@@ -1101,17 +1127,34 @@ static AttnPlan plan_attention(int B, int K, int S, int sliding_window) {
     AttnPlan pl;
     pl.waves = 4;
     if (waves_env == 4 || waves_env == 8 || waves_env == 16) pl.waves = (int)waves_env;
-    const int unit = pl.waves * kTile;
-    const int max_chunks = (span + unit - 1) / unit;
     const long target = target_env > 0 ? target_env : 256;  // workgroups: one per compute unit
     long want = (target + pairs - 1) / pairs;
     if (span <= 2 * 128) want = 1;  // a window of a few tiles: one workgroup, no merge
     if (pairs > kMaxSplitPairs) want = 1;
-    int n_chunks = (int)std::max(1L, std::min((long)max_chunks, want));
-    int chunk = (span + n_chunks - 1) / n_chunks;
-    chunk = (chunk + unit - 1) / unit * unit;
-    pl.n_chunks = (span + chunk - 1) / chunk;
-    pl.chunk = chunk;
+    cut_chunks(pl, span, want);
+    return pl;
+}
+
+// The plan above in even shares: as many whole pairs on each compute unit as there are full rounds of them, and the pairs left
+// over (all, when there are fewer than 256) cut into as many chunks each as still make one workgroup per unit.  A unit that
+// gets a second pair, or a chunk more than the others, sets the launch's time: 65 rows x 4 heads x 2000 keys in FP8 took
+// 39.2 us, with the 4 left-over pairs in chunks 27.5; 37 x 8 x 1777 in bf16 62.7 and 48.5; 48 x 8 x 3001 at H = 64 34.2 and
+// 31.3; 23 x 4 x 2000 in 3 chunks 20.6, in 2 16.4; 50 x 4 x 2000 in 2 chunks 27.3, whole 22.9.  A chunk costs its merge
+// (2-3 us), so pairs are only cut where that saves the streaming of 128 KB or more (64 KB where only part of the device is
+// busy, which streams faster per unit): 33 x 8 x 1000 FP8 21.9 -> 18.0 us, 16 x 8 x 1000 in 2 chunks 12.5, whole 13.9; but
+// 45 x 8 x 300 10.6 whole, 13.4 cut.
+// Rows with a position each leave more than 256 pairs whole (the whole-row kernel takes those).  key_bytes: of one key and its
+// value.  Its parts may need more room than those of the plan above; a caller's workspace is held to that plan, and gets it
+// when it is too small for this one.
+static AttnPlan plan_shares(int B, int K, int S, int key_bytes, int sliding_window, bool one_position) {
+    AttnPlan pl = plan_attention(B, K, S, sliding_window);
+    static const bool off = env_long("LYRA_ATTN_TARGET_WGS") > 0;  // (the override states the number of chunks)
+    const long pairs = (long)B * K, left = pairs % 256;
+    if (off || sliding_window > 0 || left == 0 || pairs > kMaxSplitPairs || (pairs > 256 && !one_position)) return pl;
+    long want = std::min(256 / left, ((long)S + pl.waves * kTile - 1) / (pl.waves * kTile));
+    if ((double)S * key_bytes * (want - 1) < (pairs > 256 ? 131072.0 : 65536.0) * want) want = 1;
+    cut_chunks(pl, S, want);
+    pl.whole = pairs > 256 && pl.n_chunks > 1 ? (int)(pairs - left) : 0;
     return pl;
 }
 
@@ -1128,7 +1171,7 @@ static AttnWorkspace attention_workspace(int B, int N, int K, int H, const AttnP
     // fixed size whatever the shape, so calls of different shapes sharing one workspace never leave
     // partial results where another call's counters live (chunking only happens below kMaxSplitPairs pairs)
     w.arrivals_bytes = kMaxSplitPairs * sizeof(int);
-    const size_t items = (size_t)B * K * pl.n_chunks * (N / K);
+    const size_t items = (size_t)(B * K - pl.whole) * pl.n_chunks * (N / K);
     w.o_bytes = up(items * H * sizeof(float));
     w.ml_bytes = up(items * 2 * sizeof(float));
     return w;
@@ -1140,9 +1183,14 @@ __global__ void zero_fill_kernel(uint32_t* p, size_t n) {
 
 extern "C" size_t lyra_decode_attention_workspace(int B, int N, int K, int S, int H, int sliding_window) {
     if (B <= 0 || N <= 0 || K <= 0 || S <= 0 || H <= 0 || N % K) return 0;
-    const lyra::AttnPlan pl = lyra::plan_attention(B, K, S, sliding_window);
-    if (pl.n_chunks == 1) return 256;
-    return lyra::attention_workspace(B, N, K, H, pl).total();
+    size_t need = 256;
+    auto cover = [&](const lyra::AttnPlan& pl) {
+        if (pl.n_chunks > 1) need = std::max(need, lyra::attention_workspace(B, N, K, H, pl).total());
+    };
+    cover(lyra::plan_attention(B, K, S, sliding_window));
+    for (int es = 1; es <= 2; ++es)
+        for (const bool one_position : {false, true}) cover(lyra::plan_shares(B, K, S, 2 * H * es, sliding_window, one_position));
+    return need;
 }
 
 extern "C" int lyra_workspace_init(void* workspace, size_t workspace_bytes, lyra_stream_t stream) {
@@ -1195,7 +1243,18 @@ static int run_attention(const void* q, const void* k, const void* v, const floa
     if ((H != 64 && H != 128) || G > 16) return LYRA_E_UNSUPPORTED;
     if (K > 65535 || B > 65535) return LYRA_E_UNSUPPORTED;
 
+    // (the workspace is held to the first plan, whichever is taken)
     AttnPlan pl = plan_attention(B, K, S, sliding_window);
+    const bool room = workspace && (uintptr_t)workspace % 256 == 0;
+    if (pl.n_chunks > 1) {
+        if (!room) return LYRA_E_WORKSPACE;
+        if (workspace_bytes < attention_workspace(B, N, K, H, pl).total()) return too_small;
+    }
+    const AttnPlan shares = plan_shares(B, K, S, 2 * H * (kv_dtype == LYRA_DTYPE_BF16 ? 2 : 1), sliding_window, position_stride == 0);
+    // (a launch that the static scratch did not serve so far stays out of it: overlapping calls of such shapes are allowed)
+    if (shares.n_chunks == 1 || (room && workspace_bytes >= attention_workspace(B, N, K, H, shares).total() &&
+                                 !(clear_counters && pl.n_chunks == 1)))
+        pl = shares;
     // ranked rows: only the unchunked global-layer launch with one position per row and more pairs than compute units deals
     // pairs out by length; every other launch ignores the order
     const bool ranked = row_order && position_stride == 1 && sliding_window == 0 && pl.n_chunks == 1 && (long)B * K > 256 && !front;
@@ -1222,6 +1281,7 @@ static int run_attention(const void* q, const void* k, const void* v, const floa
     p.sw = sliding_window;
     p.chunk = pl.chunk;
     p.n_chunks = pl.n_chunks;
+    p.whole = pl.whole;
     p.out_f32 = out_dtype == LYRA_DTYPE_F32;
     const bool vec4 = (S % 4 == 0) && (((uintptr_t)k_scale | (uintptr_t)v_scale) % 16 == 0);
     p.scale_vec4 = vec4;
@@ -1250,8 +1310,6 @@ static int run_attention(const void* q, const void* k, const void* v, const floa
     p.arrivals = nullptr;
     if (pl.n_chunks > 1) {
         const AttnWorkspace w = attention_workspace(B, N, K, H, pl);
-        if (!workspace || ((uintptr_t)workspace % 256)) return LYRA_E_WORKSPACE;
-        if (workspace_bytes < w.total()) return too_small;
         p.arrivals = (int*)workspace;
         p.part_o = (float*)((char*)workspace + w.arrivals_bytes);
         p.part_ml = (float*)((char*)workspace + w.arrivals_bytes + w.o_bytes);
@@ -1264,7 +1322,8 @@ static int run_attention(const void* q, const void* k, const void* v, const floa
                            (uint32_t*)p.arrivals, n);
         if (hipGetLastError() != hipSuccess) return LYRA_E_LAUNCH;
     }
-    const dim3 grid(pl.n_chunks, K, B), block(pl.waves * 64);
+    const dim3 grid = pl.whole > 0 ? dim3((unsigned)(pl.whole + (B * K - pl.whole) * pl.n_chunks)) : dim3(pl.n_chunks, K, B);
+    const dim3 block(pl.waves * 64);
     const size_t lds_merge = ((size_t)pl.waves * G * (H + 4) + 2 * pl.waves * 16 + 32) * sizeof(float);
     const size_t lds_q = (size_t)(pl.waves * 64 / (H / 8)) * (H + 8) * sizeof(uint16_t);  // one 16-byte piece of q per thread
     const size_t lds_stage = pl.n_chunks > 1 ? kMergeStageFloats * sizeof(float) : 0;

@@ -1,0 +1,71 @@
+"""The attention launch whose (row, kv head) pairs do not make whole rounds over the compute units: whole pairs and a chunked
+remainder in one launch, against the oracle and against the plan it replaces."""
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import clib
+from oracle import lyra_oracle as O
+from tests import gpu_util as U
+from tests.test_gpu_fused import test_attention_with_the_front_step_equals_the_two_launches as front_step
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(case, B, N, K, S, H, pos, ws):
+    from lyra_amd import _lib
+
+    q, k, v, sinks = U.attention_torch_inputs(case)
+    fp8 = case["fp8"]
+    ptr = lambda t: t.data_ptr()  # noqa: E731
+    kv = (ptr(k.qval), ptr(v.qval), ptr(k.scale), ptr(v.scale)) if fp8 else (ptr(k), ptr(v), None, None)
+    out = torch.full((B, N, 1, H), float("nan"), dtype=torch.float32, device=U.dev())
+    p = torch.tensor(pos, dtype=torch.int32, device=U.dev())
+    rc = _lib.lib.lyra_decode_attention(ptr(q), *kv, ptr(sinks), ptr(p), 0 if p.dim() == 0 else 1, None, ptr(out),
+                                        None if ws is None else ptr(ws), 0 if ws is None else ws.numel(), B, N, K, S, H, H**-0.5, 0,
+                                        _lib.DTYPE_E4M3FN if fp8 else _lib.DTYPE_BF16, _lib.DTYPE_F32,
+                                        torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    return rc, U.to_np(out)
+
+
+# pairs = B * K: remainders of 1 (cut finest), 4, 8, 36 and 128 pairs (2 chunks) behind one and two rounds, one too large to cut,
+# and fewer pairs than units (3 or 2 chunks instead of 4 or 3; whole instead of 2)
+@pytest.mark.parametrize("B,K,N,S,H,fp8", [
+    (257, 1, 4, 1300, 128, True), (65, 4, 16, 700, 128, True), (33, 8, 32, 1025, 64, True), (73, 4, 16, 300, 128, False),
+    (129, 4, 8, 1000, 64, False), (96, 4, 16, 1200, 128, True), (100, 4, 16, 600, 128, True), (23, 4, 16, 1100, 128, True),
+    (17, 4, 64, 900, 64, False), (50, 4, 16, 500, 128, True),
+])
+def test_whole_pairs_and_a_chunked_remainder(B, K, N, S, H, fp8):
+    from lyra_amd import _lib
+
+    print(f"attention shares B={B} N={N} K={K} S={S} H={H} fp8={fp8}", file=sys.stderr, flush=True)
+    case = U.attention_case(B + S, B, N, K, S, H, fp8=fp8)
+    need = _lib.lib.lyra_decode_attention_workspace(B, N, K, S, H, 0)
+    ws = torch.zeros(need, dtype=torch.uint8, device=U.dev())
+    rng = np.random.default_rng(S)
+    for pos in (S - 1, S // 2, 0, -1, rng.integers(-1, S, B)):
+        rc, got = _call(case, B, N, K, S, H, pos, ws)
+        _lib.check(rc, "lyra_decode_attention")
+        rc, again = _call(case, B, N, K, S, H, pos, ws)
+        assert rc == 0 and np.array_equal(got, again)
+        assert int(ws[: 64 * 1024].view(torch.int32).abs().sum()) == 0 or need == 256  # the counters are zero again
+        if fp8:
+            (kq, ks), (vq, vs) = case["k"], case["v"]
+            full = np.broadcast_to(np.asarray(pos, np.int32), (B,)).copy()
+            want = clib.decode_attention(O.bf16_bits(case["q"]), kq, vq, ks[..., 0], vs[..., 0], case["sinks"], full, None, H**-0.5, 0)
+        else:
+            want = O.decode_attention_reference(case["q"], case["k"], case["v"], case["sinks"], H**-0.5, 0, pos)
+        U.assert_close(got, want, what=f"shares pos={pos}")
+        if B * K > 256:  # without a workspace these ran unchunked, and still do: the same sums in another order
+            rc, plain = _call(case, B, N, K, S, H, pos, None)
+            assert rc == 0
+            # (float32 outputs of probabilities rounded to bf16 against another running maximum: 2^-8 of sum p |v|, |v| < 6)
+            np.testing.assert_allclose(got, plain, rtol=0, atol=6 * 2.0**-8)
+
+
+@pytest.mark.parametrize("B,N,K,S", [(65, 16, 4, 600), (33, 32, 8, 1100), (23, 16, 4, 1100)])
+def test_front_step_in_a_launch_of_uneven_pairs(B, N, K, S):
+    front_step(B, N, K, S, 128, True, True, 0, True, "full")
