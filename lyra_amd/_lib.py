@@ -12,7 +12,7 @@ LIB_PATH = os.path.join(PKG_DIR, "liblyra_hip.so")
 DTYPE_BF16, DTYPE_E4M3FN, DTYPE_F32, DTYPE_E5M2 = 0, 1, 2, 3
 RHS_SPAN_MAJOR, RHS_SPAN_MAJOR_GLU = 0x100, 0x200  # LYRA_RHS_SPAN_MAJOR(_GLU): OR-ed into a matmul's rhs_dtype
 LHS_TILED16, OUT_TILED16 = 0x400, 0x800  # LYRA_LHS_TILED16 / LYRA_OUT_TILED16, likewise
-ABI_VERSION = 15
+ABI_VERSION = 16
 E_UNSUPPORTED = -2  # LYRA_E_UNSUPPORTED: a shape or dtype the kernels do not cover
 
 
@@ -84,6 +84,23 @@ SIGNATURES = {
     "lyra_decode_gemm_partials": (
         _c.c_int,
         [_c.c_void_p] * 3 + [_c.c_int] * 2 + [_c.c_void_p] * 2 + [_c.c_size_t] + [_c.c_int] * 4 + [_c.c_void_p],
+    ),
+    "lyra_rows_proj_sums": (_c.c_int, [_c.c_int] * 4),
+    "lyra_rows_proj_norm": (
+        _c.c_int,
+        [_c.c_void_p, _c.c_int] + [_c.c_void_p] * 2 + [_c.c_float] + [_c.c_void_p] * 4 + [_c.c_int] + [_c.c_void_p] * 3 + [_c.c_int] * 2
+        + [_c.c_void_p, _c.c_size_t] + [_c.c_int] * 4 + [_c.c_void_p],
+    ),
+    "lyra_rows_proj_swiglu": (
+        _c.c_int,
+        [_c.c_void_p, _c.c_int] + [_c.c_void_p] * 2 + [_c.c_int] * 2 + [_c.c_float] * 3 + [_c.c_void_p] * 2 + [_c.c_int] * 2
+        + [_c.c_void_p, _c.c_size_t] + [_c.c_int] * 4 + [_c.c_void_p],
+    ),
+    "lyra_decode_attention_rows": (
+        _c.c_int,
+        [_c.c_void_p, _c.c_int] + [_c.c_void_p] * 2 + [_c.c_int] * 2 + [_c.c_float, _c.c_void_p, _c.c_int] + [_c.c_void_p] * 4
+        + [_c.c_int, _c.c_float] + [_c.c_void_p] * 6 + [_c.c_int] + [_c.c_void_p] * 2 + [_c.c_size_t] + [_c.c_int] * 5 + [_c.c_float]
+        + [_c.c_int] * 3 + [_c.c_void_p],
     ),
     "lyra_rmsnorm_proj_sum": (
         _c.c_int,
@@ -179,6 +196,7 @@ def workspace(kind: str, device, stream_ptr: int, nbytes: int):
 attention_workspace = functools.lru_cache(maxsize=4096)(lib.lyra_decode_attention_workspace)
 gemm_workspace = functools.lru_cache(maxsize=4096)(lib.lyra_decode_gemm_workspace)
 gemm_splits = functools.lru_cache(maxsize=4096)(lib.lyra_decode_gemm_splits)
+rows_proj_sums = functools.lru_cache(maxsize=4096)(lib.lyra_rows_proj_sums)
 
 
 def raw_stream(device) -> int:

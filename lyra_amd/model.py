@@ -456,6 +456,7 @@ _LOGIT_TILE_MAX = os.environ.get("LYRA_NO_LOGIT_TILE_MAX") is None  # tuning ove
 # a K-split workgroup then reads one contiguous run per wavefront instead of pieces a weight row apart (0.2-0.3 us of each
 # 5-10 us launch).  Expert weights keep the reference's array unless their rows straddle cache lines (the copy costs the
 # expert kernel more than it gains there).  LYRA_SPAN_MAJOR_DENSE=0: the alignment rule for every array.
+_ROWS_PROJ = os.environ.get("LYRA_NO_ROWS_PROJ") is None  # tuning override: norm and SwiGLU in launches of their own at every batch
 _DENSE_SPAN_MAJOR = os.environ.get("LYRA_SPAN_MAJOR_DENSE", "1") != "0"
 
 
@@ -480,6 +481,17 @@ def _bf16_bias(bias, groups: int = 1):
     return kept[1]
 
 
+def _norm_in_projection(x) -> bool:
+    """Whether the norm of ``x`` runs inside the launch of the projection behind it: slices of a few rows (beyond that the sums,
+    which every column span repeats, cost more than the norm's launch), of 1024 columns or more.  The operand there is bf16(x *
+    scale) with the row's factor applied to the float32 product, so it skips one of the reference's roundings to bf16: closer
+    to the exact product, but where a router's two best experts are within that rounding of each other a token may go to the
+    other one.  Narrower models are held to the reference's own roundings, launch by launch."""
+    from lyra_amd.kernels import decode_fused as F
+
+    return _ROWS_PROJ and isinstance(x, F.Unsummed) and x.partials.shape[1] <= F.ROWS_PROJ_MAX and x.partials.shape[2] >= 1024
+
+
 def attention_apply_fused(x, w: AttentionWeights, idx: int, pos, cos_t, sin_t, cache: LayerCache, cfg: ModelConfig):
     """attention_apply as 4 launches: norm(+gate) | qkv matmul | QK norm + RoPE + cache append + attention | output matmul.
     ``x`` is the residual stream or an ``Unsummed`` projection that still has to be added to it; the return value likewise
@@ -488,6 +500,21 @@ def attention_apply_fused(x, w: AttentionWeights, idx: int, pos, cos_t, sin_t, c
 
     H, N, K = cfg.head_dim, cfg.n_attn_heads, cfg.n_kv_heads
     tiled = _TILED_ACTIVATIONS and cfg.n_embd % 32 == 0  # (the normalised rows only feed the q/k/v projection: 16 x 32 tiles)
+    sliding_window = cfg.sliding_window if idx % 2 == 0 else 0
+    # (learned exclusive self attention needs the value rows that a launch of its own hands over)
+    front_step = w.xsa_alpha is None and not _SEPARATE_QKV_POST
+    w_qkv, w_out = F.span_major(w.qkv, always=_DENSE_SPAN_MAJOR), F.span_major(w.out, always=_DENSE_SPAN_MAJOR)
+    t = None
+    if front_step and pos.numel() == 1 and _norm_in_projection(x):
+        # a few rows: the norm inside the projection's launch
+        rows = F.rows_proj_norm(x, w.norm_scale, cfg.norm_eps, w_qkv, gate=w.sdpa_gate)
+        if rows is not None:
+            qkv, x_done = rows
+            qkv.bias = None if w.qkv_bias is None else _bf16_bias(w.qkv_bias).reshape(-1)
+            t = F.attention_qkv(qkv, w.qnorm_scale, w.knorm_scale, cos_t, sin_t, pos, cache.k, cache.v, w.sinks, H**-0.5,
+                                sliding_window, N, K, H, cfg.norm_eps)
+            if t is not None:
+                return _attention_out(t, w_out, x_done, w, cfg), cache
     if isinstance(x, TokenRows):  # first layer of a step: the embedding rows are gathered by the norm kernel
         h, gate, x = F.embed_rmsnorm_proj(x.table, x.tokens, w.norm_scale, cfg.norm_eps, w.sdpa_gate, None, gate=True, tiled=tiled)
     elif isinstance(x, (F.Unsummed, F.Uncombined)):
@@ -496,18 +523,14 @@ def attention_apply_fused(x, w: AttentionWeights, idx: int, pos, cos_t, sin_t, c
         h, gate = F.rmsnorm_proj(x, w.norm_scale, cfg.norm_eps, w.sdpa_gate, None, gate=True, tiled=tiled)
     B = x.shape[0]
     one = _one_group(B, x.device)
-    w_qkv, w_out = F.span_major(w.qkv, always=_DENSE_SPAN_MAJOR), F.span_major(w.out, always=_DENSE_SPAN_MAJOR)
     # (:310-313: a bias is added to the projection's bf16 result, in bf16: by the attention launch that sums the slices when
     # that launch is certain to take them - one position for the batch, no learned exclusive self attention - else inside
     # the matmul's epilogue, which costs the launch that sums the slices)
-    front_step = w.xsa_alpha is None and not _SEPARATE_QKV_POST
     qkv = F.gemm_unsummed(h, w_qkv, one) if (w.qkv_bias is None or (front_step and pos.numel() == 1)) else None
     if qkv is not None and w.qkv_bias is not None:
         qkv.bias = _bf16_bias(w.qkv_bias).reshape(-1)
     if qkv is None:
         qkv = F.gemm(h, w_qkv, one, bias=_bf16_bias(w.qkv_bias), bias_after_cast=w.qkv_bias is not None)
-    sliding_window = cfg.sliding_window if idx % 2 == 0 else 0
-    t = None
     if front_step:  # QK norm + RoPE + cache append inside the attention launch
         t = F.attention_qkv(qkv, w.qnorm_scale, w.knorm_scale, cos_t, sin_t, pos, cache.k, cache.v, w.sinks, H**-0.5,
                             sliding_window, N, K, H, cfg.norm_eps, gate=gate)
@@ -522,14 +545,22 @@ def attention_apply_fused(x, w: AttentionWeights, idx: int, pos, cos_t, sin_t, c
         attn = attn_op(cfg.mode, cfg.implementation)
         t = attn(q[:, :, None, :], cache.k, cache.v, w.sinks, H**-0.5, sliding_window, pos, gate=gate, xsa_v=xsa_v,
                  xsa_alpha=w.xsa_alpha).reshape(B, N * H)
-    # :366-373: projection, + bias, * residual scale, + residual, each a bf16 result - left to the norm that sums the slices
+    return _attention_out(t, w_out, x, w, cfg), cache
+
+
+def _attention_out(t, w_out, x, w: AttentionWeights, cfg: ModelConfig):
+    """lyra/model.py:366-373: projection, + bias, * residual scale, + residual, each a bf16 result - left to the norm that sums
+    the slices, where there are slices."""
+    from lyra_amd.kernels import decode_fused as F
+
+    one = _one_group(t.shape[0], t.device)
     out = F.gemm_unsummed(t, w_out, one)
     if out is None:
         return F.gemm(t, w_out, one, bias=_bf16_bias(w.out_bias), bias_after_cast=w.out_bias is not None, residual=x,
-                      out_scale=cfg.residual_scale), cache
+                      out_scale=cfg.residual_scale)
     out.residual, out.scale = x, cfg.residual_scale
     out.bias = None if w.out_bias is None else _bf16_bias(w.out_bias).reshape(-1)
-    return out, cache
+    return out
 
 
 def moe_apply_fused(x, w: MoEWeights, cfg: ModelConfig, groups_out: list | None = None):
@@ -558,16 +589,29 @@ def moe_apply_fused(x, w: MoEWeights, cfg: ModelConfig, groups_out: list | None 
     return F.moe_combine(t, scores, dest, x, cfg.residual_scale)
 
 
+def _flat(bias):
+    return None if bias is None else bias.reshape(-1)
+
+
 def dense_mlp_apply_fused(x, w: DenseMLPWeights, cfg: ModelConfig):
     from lyra_amd.kernels import decode_fused as F
 
     tiled = _TILED_ACTIVATIONS and cfg.n_embd % 32 == 0 and cfg.dense_hidden % 32 == 0
+    w_up, w_down = F.span_major(w.mlp_up, always=_DENSE_SPAN_MAJOR), F.span_major(w.mlp_down, always=_DENSE_SPAN_MAJOR)
+    if _norm_in_projection(x) and F.rows_proj_swiglu_exists(x.partials.shape[1], w_down):
+        # a few rows: norm and SwiGLU inside the launches of the projections behind them
+        rows = F.rows_proj_norm(x, w.norm_scale, cfg.norm_eps, w_up)
+        if rows is not None:
+            down = F.rows_proj_swiglu(rows[0], w_down, cfg.swiglu_beta, cfg.swiglu_limit, bias=_flat(_bf16_bias(w.mlp_up_bias)))
+            if down is not None:
+                down.residual, down.scale = rows[1], cfg.dense_residual_scale
+                down.bias = _flat(_bf16_bias(w.mlp_down_bias))
+                return down
     if isinstance(x, (F.Unsummed, F.Uncombined)):
         t, _, x = F.rmsnorm_proj(x, w.norm_scale, cfg.norm_eps, tiled=tiled)
     else:
         t, _ = F.rmsnorm_proj(x, w.norm_scale, cfg.norm_eps, tiled=tiled)
     one = _one_group(x.shape[0], x.device)
-    w_up, w_down = F.span_major(w.mlp_up, always=_DENSE_SPAN_MAJOR), F.span_major(w.mlp_down, always=_DENSE_SPAN_MAJOR)
     t = F.gemm(t, w_up, one, fused_swiglu=True, swiglu_beta=cfg.swiglu_beta, swiglu_limit=cfg.swiglu_limit,
                bias=_bf16_bias(w.mlp_up_bias), out_tiled=tiled)
     # :628-636: projection, + bias, * residual scale, + residual, each a bf16 result - left to the norm that sums the slices
