@@ -51,7 +51,8 @@ struct GemmParams {
     const float* bias;
     void* out;
     float* part;  // [ksplit, M, N] float32 partial products when ksplit > 1; grouped: two tile slots per workgroup
-    int* arrivals;  // grouped: arrival counters of split units (zero between launches)
+    int* arrivals;  // grouped, K-split: arrival counters of split units (zero between launches)
+    int finish_in_launch;  // K-split kernel (at most 16 rows): whoever arrives last at a tile adds its slices and applies the epilogue
     int M, G, K, N;
     int bk, bn, KB, NB;
     int bn_shift;  // log2(bn): scale columns are power-of-two wide
@@ -1021,6 +1022,83 @@ __global__ __launch_bounds__(kSmallWaves * 64) void decode_gemm_small_kernel(Gem
 constexpr int kSplitWaves = 4;
 constexpr int kSplitPitch = 132;  // floats per row of a partial tile in LDS (128 + padding against bank conflicts)
 
+// 4 finished columns of one row, as the finish kernel leaves them: a the sums (with SwiGLU of the gate columns, b of the linear).
+__device__ __forceinline__ void splitk_epilogue(const GemmParams& p, float (&a)[4], float (&b)[4], int row, int col, int NO, int cnt) {
+    if (row >= cnt) {  // rows past the last group: zero product (lax.ragged_dot)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a[c] = b[c] = 0.f;
+    }
+    if (p.bias) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float bv = p.bias[col + c];
+            a[c] = p.bias_post ? round_bf16(round_bf16(a[c]) + bv) : a[c] + bv;
+            if (p.swiglu) b[c] += p.bias[NO + col + c];
+        }
+    }
+    if (p.swiglu) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a[c] = swiglu_one(a[c], b[c], p.beta, p.limit);
+    }
+    if (p.post_scale) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a[c] = residual_epilogue(p, a[c], (size_t)row * NO + col + c);
+    }
+    if (p.out_f32) {
+        out_store(p.out, ((size_t)row * NO + col) * 4, f32x4{a[0], a[1], a[2], a[3]});
+    } else {
+        u32x2 d;
+        d[0] = pack_bf16(a[0], a[1]);
+        d[1] = pack_bf16(a[2], a[3]);
+        out_store(p.out, out_index(p, row, col, NO) * 2, d);
+    }
+}
+
+// The slices of one tile (rows row0 ... row0 + rows - 1, the 128 columns of a span; with SwiGLU the gate span and its linear
+// span) summed by the workgroup that arrives last, with the epilogue of the finish kernel, element for element in its order.
+// The arrival protocol is the grouped kernel's: slices stored at agent scope and acknowledged before the arrival is counted.
+__device__ __forceinline__ void splitk_finish(const GemmParams& p, int span, int row0, int rows, int cnt) {
+    __shared__ int sm_last;
+    const int half = p.swiglu ? (int)gridDim.x >> 1 : 0, NO = p.swiglu ? p.N / 2 : p.N;  // (with SwiGLU N % 256 == 0)
+    if (p.swiglu && span >= half) span -= half;
+    wait_all_memory();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int* counter = p.arrivals + blockIdx.z * gridDim.x + span;
+        const bool last = add_agent(counter, 1) == p.ksplit * (p.swiglu ? 2 : 1) - 1;
+        if (last) store_agent(counter, 0);  // leave the counter ready for the next launch
+        sm_last = last;
+    }
+    __syncthreads();
+    if (!sm_last) return;
+    const __amdgpu_buffer_rsrc_t rsrc = through_rsrc(p.part);
+    const int col = span * 128 + 4 * ((int)threadIdx.x & 31);
+    if (col >= NO) return;
+    const int slab = p.M * p.N * 4;
+    for (int r = threadIdx.x >> 5; r < rows && row0 + r < p.M; r += 8) {
+        const int row = row0 + r, off = (row * p.N + col) * 4;
+        float a[4] = {0.f, 0.f, 0.f, 0.f}, b[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int s0 = 0; s0 < p.ksplit; s0 += 8) {  // (8 slices in flight; 16, or two rows at once, cost more than their round trip)
+            f32x4 va[8], vb[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const bool live = s0 + j < p.ksplit;
+                va[j] = load_agent_b128(rsrc, live ? (s0 + j) * slab + off : kNoLoad);
+                vb[j] = load_agent_b128(rsrc, live && p.swiglu ? (s0 + j) * slab + off + NO * 4 : kNoLoad);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    a[c] += va[j][c];
+                    b[c] += vb[j][c];
+                }
+            }
+        }
+        splitk_epilogue(p, a, b, row, col, NO, cnt);
+    }
+}
+
 // STEP_SCALES: 0 scales constant along K (applied to the finished tile); 1 scale blocks shorter than K, every wavefront's
 // rows within one block (its scale applied to its finished tile); 2 one scale per 32-row step.  With 1 and 2 a wavefront
 // takes DEPTH consecutive steps instead of every 4th.
@@ -1028,7 +1106,9 @@ constexpr int kSplitPitch = 132;  // floats per row of a partial tile in LDS (12
 // the DEPTH register sets are refilled as they are used, wavefronts interleave, STEP_SCALES is 0 or 2.
 // MT: 16-row tiles the instantiation holds (1, 2 or 4 = row blocks of 16, 32, 64 rows): a launch with smaller blocks runs
 // less code - these launches are bound by the instructions one wavefront per SIMD gets through, not by arithmetic.
-template <int FP8, int DEPTH, int STEP_SCALES, bool LOOP, int MT = 4>
+// FINISH: whoever arrives last at a tile adds its slices (an instantiation of its own: the code behind the stores costs the
+// launches that leave their slices to a consumer 1.5 us each, though they skip it).
+template <int FP8, int DEPTH, int STEP_SCALES, bool LOOP, int MT = 4, bool FINISH = false>
 __global__ __launch_bounds__(kSplitWaves * 64) void decode_gemm_splitk_kernel(GemmParams p) {
     constexpr int ES = FP8 ? 1 : 2;
     extern __shared__ float sm_part[];  // [kSplitWaves][64][kSplitPitch]
@@ -1212,6 +1292,7 @@ __global__ __launch_bounds__(kSplitWaves * 64) void decode_gemm_splitk_kernel(Ge
         }
         if (span * 128 + 4 * q < p.N) store_through(p.part, (((size_t)ks * p.M + row) * p.N + span * 128 + 4 * q) * 4, v);
     }
+    if constexpr (FINISH) splitk_finish(p, span, row0, 16 * n_mt, cnt);
 }
 
 __device__ __forceinline__ f32x4 load_f32x4_at(__amdgpu_buffer_rsrc_t rsrc, int voff, int soff) {
@@ -2363,25 +2444,24 @@ int launch_split_k_fmt(const GemmParams& p, const GemmPlan& pl, hipStream_t st) 
     // scales that change along K: free when every wavefront's rows (32 * depth) lie within one scale block
     const int step_scales =
         !(WT != 0 && p.scale_mode == 1 && p.bk < p.K) ? 0 : ((!loop && p.bk % (32 * std::max(1, std::min(depth, 4))) == 0) ? 1 : 2);
-#define LYRA_SPLITK_M(D, S, M_)                                                                                        \
+#define LYRA_SPLITK_L(...)                                                                                             \
     do {                                                                                                              \
-        static const hipError_t attr = hipFuncSetAttribute((const void*)decode_gemm_splitk_kernel<WT, D, S, false, M_>, \
+        static const hipError_t attr = hipFuncSetAttribute((const void*)decode_gemm_splitk_kernel<WT, __VA_ARGS__>,    \
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);     \
         if (attr != hipSuccess) return LYRA_E_LAUNCH;                                                                 \
-        hipLaunchKernelGGL((decode_gemm_splitk_kernel<WT, D, S, false, M_>), grid, block, lds, st, p);                \
+        hipLaunchKernelGGL((decode_gemm_splitk_kernel<WT, __VA_ARGS__>), grid, block, lds, st, p);                     \
     } while (0)
-#define LYRA_SPLITK(D, S)                              \
-    do {                                               \
-        if (pl.row_block <= 16) LYRA_SPLITK_M(D, S, 1); \
-        else if (pl.row_block <= 32) LYRA_SPLITK_M(D, S, 2); \
-        else LYRA_SPLITK_M(D, S, 4);                   \
+#define LYRA_SPLITK(D, S)                                     \
+    do {                                                      \
+        if (p.finish_in_launch) LYRA_SPLITK_L(D, S, false, 1, true); /* (16 rows at most) */ \
+        else if (pl.row_block <= 16) LYRA_SPLITK_L(D, S, false, 1); \
+        else if (pl.row_block <= 32) LYRA_SPLITK_L(D, S, false, 2); \
+        else LYRA_SPLITK_L(D, S, false, 4);                   \
     } while (0)
-#define LYRA_SPLITK_LOOP(S)                                                                                            \
-    do {                                                                                                              \
-        static const hipError_t attr = hipFuncSetAttribute((const void*)decode_gemm_splitk_kernel<WT, (WT ? 4 : 2), S, true>, \
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);     \
-        if (attr != hipSuccess) return LYRA_E_LAUNCH;                                                                 \
-        hipLaunchKernelGGL((decode_gemm_splitk_kernel<WT, (WT ? 4 : 2), S, true>), grid, block, lds, st, p);           \
+#define LYRA_SPLITK_LOOP(S)                                                       \
+    do {                                                                          \
+        if (p.finish_in_launch) LYRA_SPLITK_L((WT ? 4 : 2), S, true, 4, true);    \
+        else LYRA_SPLITK_L((WT ? 4 : 2), S, true);                                \
     } while (0)
 #define LYRA_SPLITK_D(S)                   \
     do {                                   \
@@ -2404,7 +2484,7 @@ int launch_split_k_fmt(const GemmParams& p, const GemmPlan& pl, hipStream_t st) 
 #undef LYRA_SPLITK_D
 #undef LYRA_SPLITK_LOOP
 #undef LYRA_SPLITK
-#undef LYRA_SPLITK_M
+#undef LYRA_SPLITK_L
     return hipGetLastError() == hipSuccess ? LYRA_OK : LYRA_E_LAUNCH;
 }
 
@@ -2555,8 +2635,15 @@ int launch_planned(GemmParams p, const GemmPlan& pl, int layout, int fused_swigl
         return hipGetLastError() == hipSuccess ? LYRA_OK : LYRA_E_LAUNCH;
     }
     if (pl.split_k) {
+        // The sum of the slices inside the launch, by the last workgroup of a tile to arrive, for a few rows: one launch less on
+        // the host (3 us a call, which is what bounds a call from Python: lyra-small q/k/v at 5 rows 18.3 -> 15.1 us) and no slower
+        // on the device (8.6 -> 8.1 us, MLP up 9.5 -> 9.1, gpt-oss-20b out 9.6 -> 8.7, all in a graph).  With more rows the few
+        // workgroups that finish take longer than a launch of the whole device (16 rows: 12 slices 9.0 -> 11.0 us, SwiGLU 10.2 ->
+        // 10.7, 8 slices 9.3 -> 9.5; 64 rows 12.4 -> 14.0).
+        p.finish_in_launch = (M <= 8 || (M <= 16 && !fused_swiglu && pl.ksplit <= 8)) && (!fused_swiglu || N % 256 == 0) &&
+                             (size_t)pl.spans * pl.row_par * sizeof(int) <= kGemmCounterBytes;
         const int rc = launch_split_k_fmt<WT>(p, pl, st);
-        if (rc != LYRA_OK) return rc;
+        if (rc != LYRA_OK || p.finish_in_launch) return rc;
         return launch_finish(p, st);
     }
     if (pl.one_pass) {
@@ -2845,6 +2932,7 @@ static int run_decode_gemm(const void* lhs, const int32_t* lhs_row_map, const vo
     p.post_scale = post_scale != 0;
     p.bias_post = bias_post ? 1 : 0;
     p.arrivals = nullptr;
+    p.finish_in_launch = 0;
     if (pl.ksplit > 1 || pl.split_k || pl.grouped) {
         // the first kGemmCounterBytes belong to the grouped kernel's arrival counters, whichever kernel runs
         // (checked against the plan that is launched: never more than lyra_decode_gemm_workspace answers for the shape)
