@@ -459,6 +459,56 @@ int lyra_sample_topk_tiles(const float* x, const float* tile_max, const float* u
                            void* workspace, size_t workspace_bytes, int rows, int cols, int ld, int tile_ld, int k,
                            float temperature, int32_t* advance, lyra_stream_t stream);
 
+/*
+ * A whole decode step up to the final norm (lyra/model.py:752-783 with one new token per sequence): every layer's launches of
+ * the entry points above, on `stream`, in one call, for a caller whose own time between launches would otherwise bound the
+ * step.  Models without learned exclusive self attention, one position for the batch, layers that are either dense
+ * (router_t null) or experts.  The caches' rows at the position are written; logits and sampling stay with the caller
+ * (lyra_decode_gemm_tile_max, lyra_argmax_tiles, ...).  Results are those of the single calls bit for bit.
+ *   lyra_matrix_t  one weight array [K,N] or [E,K,N]; scale, bk, bn, dtype as in lyra_decode_gemm_ex (dtype with its layout flag)
+ *   lyra_layer_t   norm scales [C]; sinks [N]; qnorm, knorm [H] or null; gate_t [N,C] or null; biases as lyra_rmsnorm_proj_sum_bias
+ *                  and lyra_decode_gemm_ex take them, or null; k, v, ks, vs the layer's caches; S their length; router_t [n_routed,C]
+ *   lyra_step_t    table [table_rows,C] bf16, tokens [B] int32; out [B,C] bf16: the normalised rows behind the last layer;
+ *                  gemm_ws / attn_ws: workspaces large enough for every launch; scratch: lyra_decode_step_scratch bytes, 256-byte
+ *                  aligned, for the results between the launches (contents irrelevant)
+ * lyra_decode_step_scratch answers 0 for a step that lyra_decode_step refuses by its sizes.  A launch that refuses its shape ends
+ * the call with that launch's code; nothing but the caches' rows at the position, out and the workspaces has been written then.
+ */
+typedef struct {
+    const void* data;
+    const float* scale;
+    int32_t bk, bn, dtype, reserved;
+} lyra_matrix_t;
+typedef struct {
+    const float* attn_norm;
+    lyra_matrix_t qkv, out;
+    const float *sinks, *qnorm, *knorm, *gate_t, *qkv_bias, *out_bias;
+    void *k, *v;
+    float *ks, *vs;
+    int32_t S, sliding_window;
+    const float* mlp_norm;
+    lyra_matrix_t up, down;
+    const float *up_bias, *down_bias, *router_t, *router_bias;
+} lyra_layer_t;
+typedef struct {
+    const lyra_layer_t* layers;
+    const void* table;
+    const int32_t* tokens;
+    const float *cos_t, *sin_t;
+    const int32_t* position;
+    const float* final_norm;
+    void* out;
+    void* gemm_ws;
+    size_t gemm_ws_bytes;
+    void* attn_ws;
+    size_t attn_ws_bytes;
+    void* scratch;
+    size_t scratch_bytes;
+    int32_t n_layers, B, C, N, K, H, kv_dtype, table_rows, rope_rows, dense_hidden, expert_hidden, n_routed, n_shared, k_routed;
+    float eps, residual_scale, dense_residual_scale, sm_scale, beta, limit;
+} lyra_step_t;
+size_t lyra_decode_step_scratch(const lyra_step_t* step);
+int lyra_decode_step(const lyra_step_t* step, lyra_stream_t stream);
 
 /*
  * Self-check of the matrix-core register layouts and FP8 conversions the kernels rely on.

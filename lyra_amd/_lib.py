@@ -136,6 +136,8 @@ SIGNATURES = {
         _c.c_int,
         [_c.c_void_p] * 6 + [_c.c_size_t] + [_c.c_int] * 5 + [_c.c_float, _c.c_void_p, _c.c_void_p],
     ),
+    "lyra_decode_step_scratch": (_c.c_size_t, [_c.c_void_p]),
+    "lyra_decode_step": (_c.c_int, [_c.c_void_p] * 2),
     "lyra_selftest": (_c.c_int, [_c.c_void_p, _c.c_void_p]),
 }
 

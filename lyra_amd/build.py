@@ -22,6 +22,7 @@ UNITS = (
     ("decode_gemm_e5m2", "decode_gemm.hip", ("-DLYRA_GEMM_PART=3",)),
     ("decode_gemm_splitk_e5m2", "decode_gemm.hip", ("-DLYRA_GEMM_PART=4", *_VGPR_FORM)),
     ("decode_fused", "decode_fused.hip", ()),
+    ("decode_step", "decode_step.hip", ()),
 )
 HIPCC_FLAGS = (
     "--offload-arch=gfx950",

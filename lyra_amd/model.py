@@ -9,9 +9,10 @@ one thing a decode loop cannot afford), everything else is a pure function of it
 """
 from __future__ import annotations
 
-import os
-
+import ctypes
 import math
+import os
+import struct
 from dataclasses import dataclass, field, replace
 from functools import lru_cache
 
@@ -637,21 +638,135 @@ def _fused_supported(model: ModelWeights, cfg: ModelConfig) -> bool:
             and cfg.n_active_routed_experts <= 8 and cfg.padded_vocab_size % 8 == 0)
 
 
+# lyra_matrix_t, lyra_layer_t and lyra_step_t of the C ABI
+_MATRIX = "QQiiii"
+_LAYER = struct.Struct("=Q" + 2 * _MATRIX + 10 * "Q" + "iiQ" + 2 * _MATRIX + 4 * "Q")
+_STEP = struct.Struct("=14Q14i6f")
+_NATIVE_STEP = os.environ.get("LYRA_NO_NATIVE_STEP") is None  # tuning override: every launch of a step from Python
+_NATIVE_REFUSED: set = set()  # shapes that a launch refused (a plan without a kernel for them): their steps run from Python
+
+
+class _NotNative(Exception):
+    """What lyra_decode_step does not take as it is: the Python loop does, or says what is wrong with it."""
+
+
+def _need(ok: bool) -> None:
+    if not ok:
+        raise _NotNative
+
+
+def _layers_native(tokens: torch.Tensor, model: ModelWeights, cache: ModelCache, cfg: ModelConfig, cos_t, sin_t) -> torch.Tensor | None:
+    """All layers and the final norm in one call of the library (lyra_decode_step): the launches of ``attention_apply_fused``,
+    ``moe_apply_fused`` and ``dense_mlp_apply_fused`` issued from native code, where one costs the host 2.5 us instead of 8-12.
+    Pointers are read from the tensors on every call.  Returns the normalised rows [B, C], or None for what the call does not
+    cover; the caches then hold at most the rows that the Python loop writes again."""
+    from lyra_amd.kernels import decode_fused as F
+
+    B, C, N, K, H = tokens.shape[0], cfg.n_embd, cfg.n_attn_heads, cfg.n_kv_heads, cfg.head_dim
+    shape = (B, C, N, K, H, cfg.dense_hidden, cfg.expert_hidden, cfg.n_routed_experts, cfg.n_shared_experts, cfg.mlp_map)
+    pos = cache.pos
+    if (cfg.use_learned_xsa or pos.numel() != 1 or pos.dtype != torch.int32 or tokens.dtype != torch.int32 or not tokens.is_contiguous()
+            or not 0 < B <= 256 or shape in _NATIVE_REFUSED):
+        return None
+    dev = model.emb.device
+    if pos.device != dev or tokens.device != dev or model.emb.dtype != torch.bfloat16 or not model.emb.is_contiguous():
+        return None
+
+    def f32(t, n=None):
+        if t is None:
+            return 0
+        _need(t.dtype == torch.float32 and t.is_contiguous() and t.device == dev and (n is None or t.numel() == n))
+        return t.data_ptr()
+
+    def matrix(rhs, groups, k, n):
+        data, scale, bk, bn, dtype, dims = F._rhs_args(rhs)
+        _need(dims == (groups, k, n) and data.device == dev)
+        return data.data_ptr(), 0 if scale is None else scale.data_ptr(), bk, bn, dtype, 0
+
+    width, heads, E, k_routed = (N + 2 * K) * H, N * H, cfg.n_experts, cfg.n_active_routed_experts
+    rows, topk = [], cfg.n_active_experts
+    gemm_need, attn_need, kv_dtype = 0, 0, None
+    for idx, (layer, c) in enumerate(zip(model.layers, cache.layers)):
+        a, w = layer.attn, layer.mlp
+        if a.xsa_alpha is not None:
+            return None
+        fp8 = isinstance(c.k, QArray)
+        kq, vq, ks, vs = (c.k.qval, c.v.qval, c.k.scale, c.v.scale) if fp8 else (c.k, c.v, None, None)
+        dtype = _lib.fp8_code(kq.dtype) if fp8 else _lib.DTYPE_BF16
+        if idx == 0:
+            kv_dtype = dtype
+        _need(dtype == kv_dtype and isinstance(c.v, QArray) == fp8 and vq.dtype == kq.dtype and kq.device == vq.device == dev)
+        _need(tuple(c.k.block) == tuple(c.v.block) == (1, H) if fp8 else kq.dtype == torch.bfloat16)
+        _need(kq.is_contiguous() and vq.is_contiguous() and tuple(kq.shape) == tuple(vq.shape) == (B, K, kq.shape[2], H))
+        window = cfg.sliding_window if idx % 2 == 0 else 0
+        attn_need = max(attn_need, _lib.attention_workspace(B, N, K, kq.shape[2], H, window))
+        moe = isinstance(w, MoEWeights)
+        groups, hidden = (E, cfg.expert_hidden) if moe else (1, cfg.dense_hidden)
+        up = F.span_major(w.mlp_up, glu=True) if moe else F.span_major(w.mlp_up, always=_DENSE_SPAN_MAJOR)
+        down = F.span_major(w.mlp_down) if moe else F.span_major(w.mlp_down, always=_DENSE_SPAN_MAJOR)
+        m_rows = B * topk if moe else B
+        gemm_need = max(gemm_need, _lib.gemm_workspace(m_rows, groups, C, 2 * hidden, 1), _lib.gemm_workspace(m_rows, groups, hidden, C, 0))
+        rows.append(_LAYER.pack(
+            f32(a.norm_scale, C), *matrix(F.span_major(a.qkv, always=_DENSE_SPAN_MAJOR), 1, C, width),
+            *matrix(F.span_major(a.out, always=_DENSE_SPAN_MAJOR), 1, heads, C), f32(a.sinks, N), f32(a.qnorm_scale, H), f32(a.knorm_scale, H),
+            0 if a.sdpa_gate is None else f32(F._transposed(a.sdpa_gate), N * C), f32(_bf16_bias(a.qkv_bias), width),
+            f32(_bf16_bias(a.out_bias), C), kq.data_ptr(), vq.data_ptr(), f32(ks, B * K * kq.shape[2]), f32(vs, B * K * kq.shape[2]),
+            kq.shape[2], window, f32(w.norm_scale, C), *matrix(up, groups, C, 2 * hidden), *matrix(down, groups, hidden, C),
+            f32(_bf16_bias(w.mlp_up_bias, groups), groups * 2 * hidden), f32(_bf16_bias(w.mlp_down_bias, groups), groups * C),
+            f32(F._transposed(w.router), cfg.n_routed_experts * C) if moe else 0, f32(w.router_bias, cfg.n_routed_experts) if moe else 0))
+    gemm_need = max(gemm_need, _lib.gemm_workspace(B, 1, C, width, 0), _lib.gemm_workspace(B, 1, heads, C, 0))
+    stream = _lib.raw_stream(dev)
+    gemm_ws, attn_ws = _lib.workspace("gemm", dev, stream, gemm_need), _lib.workspace("attention", dev, stream, attn_need)
+    layers = ctypes.create_string_buffer(b"".join(rows), len(rows) * _LAYER.size)
+    out = torch.empty((B, C), dtype=torch.bfloat16, device=dev)
+
+    def step(scratch, nbytes):
+        return _STEP.pack(
+            ctypes.addressof(layers), model.emb.data_ptr(), tokens.data_ptr(), f32(cos_t), f32(sin_t), pos.data_ptr(),
+            f32(model.norm_scale, C), out.data_ptr(), gemm_ws.data_ptr(), gemm_ws.numel(), attn_ws.data_ptr(), attn_ws.numel(), scratch,
+            nbytes, len(rows), B, C, N, K, H, kv_dtype, model.emb.shape[0], cos_t.shape[0], cfg.dense_hidden, cfg.expert_hidden,
+            cfg.n_routed_experts, cfg.n_shared_experts, k_routed, cfg.norm_eps, cfg.residual_scale, cfg.dense_residual_scale, H**-0.5,
+            cfg.swiglu_beta, cfg.swiglu_limit)
+
+    nbytes = _lib.lib.lyra_decode_step_scratch(step(0, 0))
+    if nbytes == 0:
+        return None
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)  # (the allocator's, on this stream: reused when this call's launches are done)
+    with _lib.on_device(dev):
+        rc = _lib.lib.lyra_decode_step(step(scratch.data_ptr(), nbytes), stream)
+    if rc == _lib.E_UNSUPPORTED:
+        if len(_NATIVE_REFUSED) < 4096:
+            _NATIVE_REFUSED.add(shape)
+        return None
+    _lib.check(rc, "lyra_decode_step")
+    return out
+
+
 def model_apply_fused(tokens: torch.Tensor, model: ModelWeights, cache: ModelCache, cfg: ModelConfig, hidden_out: list | None = None,
                       groups_out: list | None = None, advance: bool = True):
     from lyra_amd.kernels import decode_fused as F
 
-    # int32 token ids are gathered by the first norm kernel (one launch fewer, and a sampler can write them in place)
-    h = TokenRows(model.emb, tokens) if tokens.dtype == torch.int32 and tokens.is_contiguous() else model.emb[tokens]
     cos_t, sin_t = _rope_tables(cfg, model.emb.device)
-    pos = cache.pos
-    for idx, layer in enumerate(model.layers):
-        h, _ = attention_apply_fused(h, layer.attn, idx, pos, cos_t, sin_t, cache.layers[idx], cfg)
-        h = moe_apply_fused(h, layer.mlp, cfg, groups_out) if isinstance(layer.mlp, MoEWeights) else dense_mlp_apply_fused(h, layer.mlp, cfg)
-    normed = F.rmsnorm_proj(h, model.norm_scale, cfg.norm_eps)
-    if hidden_out is not None:  # the residual stream after the last layer (the norm kernel completes it on its way)
-        hidden_out.append(normed[2] if len(normed) > 2 else h)
-    h = normed[0]
+    native = (_NATIVE_STEP and _ROWS_PROJ and _TILED_ACTIVATIONS and not (_SEPARATE_COMBINE or _SEPARATE_QKV_POST) and hidden_out is None
+              and groups_out is None)
+    normed = None
+    if native:
+        try:
+            normed = _layers_native(tokens, model, cache, cfg, cos_t, sin_t)
+        except _NotNative:
+            pass
+    if normed is None:
+        # int32 token ids are gathered by the first norm kernel (one launch fewer, and a sampler can write them in place)
+        h = TokenRows(model.emb, tokens) if tokens.dtype == torch.int32 and tokens.is_contiguous() else model.emb[tokens]
+        pos = cache.pos
+        for idx, layer in enumerate(model.layers):
+            h, _ = attention_apply_fused(h, layer.attn, idx, pos, cos_t, sin_t, cache.layers[idx], cfg)
+            h = moe_apply_fused(h, layer.mlp, cfg, groups_out) if isinstance(layer.mlp, MoEWeights) else dense_mlp_apply_fused(h, layer.mlp, cfg)
+        normed = F.rmsnorm_proj(h, model.norm_scale, cfg.norm_eps)
+        if hidden_out is not None:  # the residual stream after the last layer (the norm kernel completes it on its way)
+            hidden_out.append(normed[2] if len(normed) > 2 else h)
+        normed = normed[0]
+    h = normed
     # The LM head also leaves the maximum of every 128-column tile of the logits; they travel with the tensor (with the
     # version it had when they were taken) and `sample_token` hands them to a sampler that reads a few tiles per row instead
     # of the whole vocabulary - unless the logits have been written to since.
