@@ -63,3 +63,31 @@ def test_slices_summed_in_the_launch(M, K, N, kind):
     ws = [v for k, v in _lib._WORKSPACES.items() if k[0] == "gemm"]
     torch.cuda.synchronize()
     assert all(int(b[:65536].view(torch.int32).abs().sum()) == 0 for b in ws)
+
+
+# a plan of more than one round of workgroups becomes one round of longer slices: 192 workgroups of one slice, 192 of two, 160
+# of one in bf16 (2880 rows, not a multiple of the refilled register sets), scale blocks along K; and its neighbours that keep
+# the shorter slices (a light last row block; more tiles than one round holds)
+@pytest.mark.parametrize("M,K,N,kind,splits", [(128, 4096, 12288, "channel", 1), (192, 6144, 4096, "channel", 2), (256, 2880, 5120, "bf16", 1),
+                                               (97, 4096, 12288, "block", 1), (96, 4096, 12288, "channel", 2), (129, 6144, 4096, "channel", 3),
+                                               (256, 4096, 12288, "channel", 2)])
+def test_one_round_of_longer_slices(M, K, N, kind, splits):
+    from lyra_amd import _lib
+    from lyra_amd.kernels import decode_fused as F
+    from lyra_amd.nn.quant import quantize
+
+    print(f"dense plan M={M} K={K} N={N} {kind}", file=sys.stderr, flush=True)
+    dev, gen = U.dev(), torch.Generator(device=U.dev()).manual_seed(M + K)
+    w = (torch.randn(1, K, N, device=dev, generator=gen) * 0.05).to(torch.bfloat16)
+    x = torch.randn(M, K, device=dev, generator=gen).to(torch.bfloat16)
+    if kind == "bf16":
+        ref = w[0].double()
+    else:
+        w = quantize(w, torch.float8_e4m3fn, (K, 1) if kind == "channel" else (256, 256))
+        s = w.scale[0].double().repeat_interleave(w.block[0], 0).repeat_interleave(w.block[1], 1)
+        ref = w.qval[0].float().double() * s
+    got = F.gemm_unsummed(x, w, _lib.row_count(M, dev)).partials
+    assert got.shape == (splits, M, N)
+    err = (got.double().sum(0) - x.double() @ ref).abs()
+    # exact products of bf16 operands, float32 sums of K / 128 matrix instructions per wavefront and of 4 wavefronts
+    assert (err <= 2.0**-18 * (x.double().abs() @ ref.abs())).all()
