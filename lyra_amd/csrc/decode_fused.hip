@@ -1062,8 +1062,12 @@ namespace lyra {
 static int launch_rmsnorm_proj(const NormProjParams& p0, int B, lyra_stream_t stream) {
     NormProjParams p = p0;
     const size_t lds = ((size_t)p.C + 16) * sizeof(float);
-    static const int shares_env = [] { const char* e = getenv("LYRA_NORM_SHARES"); return e ? atoi(e) : 4; }();  // tuning override
-    const int shares = (p.proj_t && p.n >= 8 && B <= 256) ? std::max(1, std::min(shares_env, p.n)) : 1;
+    // 4 workgroups per row, fewer where that is more than one per compute unit: with 16 wavefronts each, a second one on a unit
+    // costs more than a share saves (lyra-small steps at 64 / 70 / 128 / 250 rows: 4 shares 1142 / 1400 / 1486 / 2252 us, 3 - /
+    // 1359 / - / 2245, 2 1152 / 1358 / 1455 / 2183, 1 1175 / 1374 / 1480 / 2121; lyra-medium at 128: 1939, with 2 1912).
+    static const int shares_env = [] { const char* e = getenv("LYRA_NORM_SHARES"); return e ? atoi(e) : 0; }();  // tuning override
+    const int most = shares_env > 0 ? shares_env : std::min(4, 256 / B);
+    const int shares = (p.proj_t && p.n >= 8 && B <= 256) ? std::max(1, std::min(most, p.n)) : 1;
     p.per_share = (p.n + shares - 1) / shares;
     if (p.comb_rows) hipLaunchKernelGGL(rmsnorm_proj_kernel<true>, dim3(B, shares), dim3(kNormThreads), lds, (hipStream_t)stream, p);
     else hipLaunchKernelGGL(rmsnorm_proj_kernel<false>, dim3(B, shares), dim3(kNormThreads), lds, (hipStream_t)stream, p);
