@@ -69,3 +69,23 @@ def test_whole_pairs_and_a_chunked_remainder(B, K, N, S, H, fp8):
 @pytest.mark.parametrize("B,N,K,S", [(65, 16, 4, 600), (33, 32, 8, 1100), (23, 16, 4, 1100)])
 def test_front_step_in_a_launch_of_uneven_pairs(B, N, K, S):
     front_step(B, N, K, S, 128, True, True, 0, True, "full")
+
+
+# windows that begin at every offset from a tile and from 16 bytes of scales, at the end of caches whose length is and is not a
+# multiple of 4; windows that are and are not whole tiles, one chunked
+@pytest.mark.parametrize("S,sw", [(520, 128), (517, 128), (520, 100), (519, 33), (520, 1), (904, 300)])
+@pytest.mark.parametrize("fp8", [True, False])
+def test_windows_at_every_offset(S, sw, fp8):
+    from lyra_amd.kernels.decode_attention import decode_attention
+
+    print(f"attention window S={S} sw={sw} fp8={fp8}", file=sys.stderr, flush=True)
+    B, N, K, H = 40, 8, 2, 64
+    case = U.attention_case(S + sw, B, N, K, S, H, fp8=fp8)
+    q, k, v, sinks = U.attention_torch_inputs(case)
+    first = np.concatenate([np.arange(S - 36, S), [0, 1, sw - 1, sw]]).astype(np.int32)
+    got = decode_attention(q, k, v, sinks, H**-0.5, sw, torch.from_numpy(first).to(U.dev()), implementation="pallas")
+    want = O.decode_attention_reference(case["q"], case["k"], case["v"], case["sinks"], H**-0.5, sw, first)
+    U.assert_close(U.to_np(got), want, what="windows")
+    for i in (0, 5, 34, 35):  # (one position for the batch: the same launch as a step's)
+        one = decode_attention(q, k, v, sinks, H**-0.5, sw, torch.tensor(int(first[i]), dtype=torch.int32, device=U.dev()), implementation="pallas")
+        assert torch.equal(one[i], got[i])
