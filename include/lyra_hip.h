@@ -137,19 +137,6 @@ int lyra_decode_attention_qkv_bias(const void* qkv, const float* partials, int s
                                    int out_dtype, lyra_stream_t stream);
 
 /*
- * The same behind lyra_rows_proj_norm: every element of the projection is factor * (sum of its slices) with the row's
- * factor = rsqrt(sum(sq[0..n_sq-1][row]) / sq_width + sq_eps), before it is rounded to bf16; and the output gate is
- * bf16(2 * sigmoid(factor * sum_s gate_part[s][row][n])), gate_part [gate_splits,B,N] (null: no gate).
- * n_sq <= 64, gate_splits <= 16 (LYRA_E_UNSUPPORTED otherwise).
- */
-int lyra_decode_attention_rows(const float* partials, int splits, const float* qkv_bias, const float* sq, int n_sq, int sq_width,
-                               float sq_eps, const float* gate_part, int gate_splits, const float* qnorm, const float* knorm,
-                               const float* cos_t, const float* sin_t, int rope_rows, float eps, void* k, void* v, float* k_scale,
-                               float* v_scale, const float* sinks, const int32_t* position, int position_stride, void* out,
-                               void* workspace, size_t workspace_bytes, int B, int N, int K, int S, int H, float sm_scale,
-                               int sliding_window, int kv_dtype, int out_dtype, lyra_stream_t stream);
-
-/*
  * Ragged batches, rows dealt out by length (an extension of the boundary, like position_stride 1: the reference passes one
  * position for the whole batch, lyra/kernels/decode_attention.py:364-375).  With more (row, kv head) pairs than compute
  * units, which workgroup takes which pair decides how long a launch lasts.  The order of the rows by length changes
@@ -301,30 +288,20 @@ int lyra_decode_gemm_partials(const void* lhs, const void* rhs, const float* rhs
                               int rhs_dtype, lyra_stream_t stream);
 
 /*
- * The same projections for at most 8 rows, fed by the unsummed slices of the projection before: what stands between
- * the two - residual update and RMS norm (lyra/model.py:371-374, 631-636, 189-191), or SwiGLU - happens inside the launch.
- *   lyra_rows_proj_sums    number n_sq of partial sums of squares per row of lyra_rows_proj_norm for (M, K, N, bk); 0 = these
- *                          launches do not exist for the shape (shape only, like lyra_decode_gemm_splits)
- *   lyra_rows_proj_norm    x_out [M,K] as lyra_rmsnorm_proj_sum_bias forms it from sums [splits,M,K]; partials [s] of
- *                          bf16(x_out * norm_scale) @ rhs.  The factor rsqrt(mean(x^2) + eps) of every row is left to the
- *                          consumer, which gets sq_out [n_sq,M], sums of x^2 over parts of the row: the product is
- *                          factor * sum of slices.  gate_t [gate_n,K] float32 (or gate_n 0): gate_part [splits,M,gate_n]
- *                          holds the slices of the same rows' narrow projection, the factor likewise left out.
- *                          x_out must not overlap the inputs.
- *   lyra_rows_proj_swiglu  partials of bf16(swiglu(gate, linear)) @ rhs, gate and linear the two halves of
- *                          factor * (sum of sums [splits,M,2K]) + bias ([2K] float32 or null), factor from sq as above with
- *                          sq_width columns per row.
- * partials as in lyra_decode_gemm_partials; rhs_dtype bf16, e4m3fn or e5m2, optionally LYRA_RHS_SPAN_MAJOR.  sums and gate_t
- * 16-byte aligned, residual and x_out 8-byte aligned, gate_n <= 16 (LYRA_E_UNSUPPORTED otherwise).
+ * A down projection of at most 16 rows behind an up projection that was left in K slices: the SwiGLU between the two happens
+ * inside the launch.
+ *   lyra_rows_proj_swiglu_exists  1 where the launch exists for (M, K, N, bk) - shape only, like lyra_decode_gemm_splits
+ *   lyra_rows_proj_swiglu         partials of bf16(swiglu(gate, linear)) @ rhs, gate and linear the two halves of the sum of
+ *                                 sums [splits,M,2K] + bias ([2K] float32 or null): what lyra_decode_gemm_ex with fused_swiglu
+ *                                 and lyra_decode_gemm_partials behind it leave (the operand bit for bit, the slices up to
+ *                                 the order of their sums).
+ * partials as in lyra_decode_gemm_partials; rhs_dtype bf16, e4m3fn or e5m2, optionally LYRA_RHS_SPAN_MAJOR.  sums is 16-byte
+ * aligned (LYRA_E_UNSUPPORTED otherwise).
  */
-int lyra_rows_proj_sums(int M, int K, int N, int bk);
-int lyra_rows_proj_norm(const float* sums, int splits, const float* sum_bias, const void* residual, float out_scale,
-                        const float* norm_scale, void* x_out, float* sq_out, const float* gate_t, int gate_n, float* gate_part,
-                        const void* rhs, const float* rhs_scale, int bk, int bn, float* partials, size_t partials_bytes, int M,
-                        int K, int N, int rhs_dtype, lyra_stream_t stream);
-int lyra_rows_proj_swiglu(const float* sums, int splits, const float* bias, const float* sq, int n_sq, int sq_width, float eps,
-                          float beta, float limit, const void* rhs, const float* rhs_scale, int bk, int bn, float* partials,
-                          size_t partials_bytes, int M, int K, int N, int rhs_dtype, lyra_stream_t stream);
+int lyra_rows_proj_swiglu_exists(int M, int K, int N, int bk);
+int lyra_rows_proj_swiglu(const float* sums, int splits, const float* bias, float beta, float limit, const void* rhs,
+                          const float* rhs_scale, int bk, int bn, float* partials, size_t partials_bytes, int M, int K, int N,
+                          int rhs_dtype, lyra_stream_t stream);
 
 /*
  * The elementwise steps of a decode layer between the two kernels above, one launch each.  They follow the

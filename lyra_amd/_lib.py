@@ -85,22 +85,11 @@ SIGNATURES = {
         _c.c_int,
         [_c.c_void_p] * 3 + [_c.c_int] * 2 + [_c.c_void_p] * 2 + [_c.c_size_t] + [_c.c_int] * 4 + [_c.c_void_p],
     ),
-    "lyra_rows_proj_sums": (_c.c_int, [_c.c_int] * 4),
-    "lyra_rows_proj_norm": (
-        _c.c_int,
-        [_c.c_void_p, _c.c_int] + [_c.c_void_p] * 2 + [_c.c_float] + [_c.c_void_p] * 4 + [_c.c_int] + [_c.c_void_p] * 3 + [_c.c_int] * 2
-        + [_c.c_void_p, _c.c_size_t] + [_c.c_int] * 4 + [_c.c_void_p],
-    ),
+    "lyra_rows_proj_swiglu_exists": (_c.c_int, [_c.c_int] * 4),
     "lyra_rows_proj_swiglu": (
         _c.c_int,
-        [_c.c_void_p, _c.c_int] + [_c.c_void_p] * 2 + [_c.c_int] * 2 + [_c.c_float] * 3 + [_c.c_void_p] * 2 + [_c.c_int] * 2
-        + [_c.c_void_p, _c.c_size_t] + [_c.c_int] * 4 + [_c.c_void_p],
-    ),
-    "lyra_decode_attention_rows": (
-        _c.c_int,
-        [_c.c_void_p, _c.c_int] + [_c.c_void_p] * 2 + [_c.c_int] * 2 + [_c.c_float, _c.c_void_p, _c.c_int] + [_c.c_void_p] * 4
-        + [_c.c_int, _c.c_float] + [_c.c_void_p] * 6 + [_c.c_int] + [_c.c_void_p] * 2 + [_c.c_size_t] + [_c.c_int] * 5 + [_c.c_float]
-        + [_c.c_int] * 3 + [_c.c_void_p],
+        [_c.c_void_p, _c.c_int, _c.c_void_p] + [_c.c_float] * 2 + [_c.c_void_p] * 2 + [_c.c_int] * 2 + [_c.c_void_p, _c.c_size_t]
+        + [_c.c_int] * 4 + [_c.c_void_p],
     ),
     "lyra_rmsnorm_proj_sum": (
         _c.c_int,
@@ -198,7 +187,7 @@ def workspace(kind: str, device, stream_ptr: int, nbytes: int):
 attention_workspace = functools.lru_cache(maxsize=4096)(lib.lyra_decode_attention_workspace)
 gemm_workspace = functools.lru_cache(maxsize=4096)(lib.lyra_decode_gemm_workspace)
 gemm_splits = functools.lru_cache(maxsize=4096)(lib.lyra_decode_gemm_splits)
-rows_proj_sums = functools.lru_cache(maxsize=4096)(lib.lyra_rows_proj_sums)
+rows_proj_swiglu_exists = functools.lru_cache(maxsize=4096)(lib.lyra_rows_proj_swiglu_exists)
 
 
 def raw_stream(device) -> int:

@@ -64,14 +64,6 @@ struct AttnParams {
     const float* sin_t;
     int rope_rows;
     float norm_eps;
-    // lyra_decode_attention_rows: the slices still lack their row's factor rsqrt(sum of row_sq / sq_width + sq_eps), and the
-    // output gate comes as slices of its projection
-    const float* row_sq;  // [n_sq, B] or null
-    int n_sq, sq_width;
-    float sq_eps;
-    const float* gate_part;  // [gate_splits, B, N] or null (with row_sq only)
-    int gate_splits;
-    int has_gate;  // gate or gate_part
     // lyra_decode_attention_ranked: batch rows from longest to shortest ([B]), or null.  With it the unchunked launch deals
     // its (row, kv head) pairs out so that the workgroups that share a compute unit hold a long and a short row.
     const int32_t* row_order;
@@ -102,18 +94,18 @@ __device__ __forceinline__ Range visible_range(int pos, int sw, int S) {
 // multiplication, as "t *= gate.astype(dtype)" does on a bf16 array (lyra/model.py:347).
 __device__ __forceinline__ void store_out(const AttnParams& p, size_t idx, float val, float gate) {
     if (p.out_f32) {
-        ((float*)p.out)[idx] = p.has_gate ? val * gate : val;
+        ((float*)p.out)[idx] = p.gate ? val * gate : val;
     } else {
-        if (p.has_gate) val = bf16_bits_to_f32(f32_to_bf16_bits(val)) * gate;
+        if (p.gate) val = bf16_bits_to_f32(f32_to_bf16_bits(val)) * gate;
         ((uint16_t*)p.out)[idx] = f32_to_bf16_bits(val);
     }
 }
 
 // The value the output gate leaves, as the JAX code holds it: a bf16 output is rounded before and after the multiplication.
 __device__ __forceinline__ float gated(const AttnParams& p, float val, float gate) {
-    if (p.out_f32) return p.has_gate ? val * gate : val;
+    if (p.out_f32) return p.gate ? val * gate : val;
     val = bf16_bits_to_f32(f32_to_bf16_bits(val));
-    return p.has_gate ? bf16_bits_to_f32(f32_to_bf16_bits(val * gate)) : val;
+    return p.gate ? bf16_bits_to_f32(f32_to_bf16_bits(val * gate)) : val;
 }
 
 // Learned exclusive self attention on the G finished heads of one (batch row, kv head) (lyra/model.py:351-363):
@@ -434,7 +426,7 @@ __device__ __forceinline__ void request_head(const AttnParams& p, __amdgpu_buffe
 // The projection's bf16 output for this lane's two elements of head hd: the slices added in slice order, then rounded.
 template <int H>
 __device__ __forceinline__ void sum_head(const AttnParams& p, __amdgpu_buffer_rsrc_t part_rsrc, int b, int hd, int lane,
-                                         const HeadSlices& hs, float factor, float& a, float& c) {
+                                         const HeadSlices& hs, float& a, float& c) {
     constexpr int half = H / 2;
     if (!p.qkv_partials) {
         a = bf16_bits_to_f32(hs.qa);
@@ -459,8 +451,8 @@ __device__ __forceinline__ void sum_head(const AttnParams& p, __amdgpu_buffer_rs
             c += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(part_rsrc, off, half * 4, 0));
         }
     }
-    a = bf16r(a * factor);  // (the literal 1 where the slices are complete)
-    c = bf16r(c * factor);
+    a = bf16r(a);
+    c = bf16r(c);
     if (p.qkv_bias) {
         // lyra/model.py:310-313: the bias is added to the projection's bf16 result, in bf16.  Fetched here, in the one
         // branch of the front step that holds loads: launches without a bias (every lyra variant) skip it, and two more
@@ -519,9 +511,8 @@ __device__ __forceinline__ void append_staged(const Slab& sl, const uint8_t* sta
     }
 }
 
-// QKV: the launch also does the step in front of the attention (lyra_decode_attention_qkv); 2: from slices that still lack
-// their row's factor (lyra_decode_attention_rows: its requests cost every launch that does not need them 0.3 us).
-template <int H, int FP8, bool VEC4, int WAVES, bool EARLY, int DEPTH, int QKV = 0>
+// QKV: the launch also does the step in front of the attention (lyra_decode_attention_qkv).
+template <int H, int FP8, bool VEC4, int WAVES, bool EARLY, int DEPTH, bool QKV = false>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(DEPTH > 1 ? 2 : (WAVES >= 8 ? 4 : 3))))
 void decode_attention_kernel(AttnParams p) {
     static_assert(!QKV || DEPTH == 1, "the fused front step knows one register set per wavefront");
@@ -590,8 +581,6 @@ void decode_attention_kernel(AttnParams p) {
         p.qkv_partials, p.qkv_partials ? (uint32_t)p.qkv_splits * (uint32_t)p.B * (uint32_t)qkv_heads * (uint32_t)H * 4u : 0u);
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t qkv_rsrc =
         make_rsrc(p.qkv, (QKV && !p.qkv_partials) ? (uint32_t)p.B * (uint32_t)qkv_heads * (uint32_t)H * 2u : 0u);
-    [[maybe_unused]] float row_factor = 1.f;
-    [[maybe_unused]] __shared__ float sm_gq[16];  // gates that were summed here, for the merge of the chunks
     [[maybe_unused]] HeadSlices hq, hkv;  // QKV: the projection slices of this wavefront's first query head (head `wave` of the G)
     [[maybe_unused]] float qn_a = 0.f, qn_c = 0.f, kn_a = 0.f, kn_c = 0.f;
     if constexpr (!QKV) {
@@ -602,19 +591,7 @@ void decode_attention_kernel(AttnParams p) {
     const float sink_raw = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(srsrc, x * 4, 0, 0));
     // ... and the output gates of these heads (an absent gate reads as zeros and is replaced by 1 below)
     const __amdgpu_buffer_rsrc_t grsrc = make_rsrc(p.gate ? p.gate + (size_t)b * p.N + kh * G : nullptr, p.gate ? (uint32_t)(G * 2) : 0u);
-    uint16_t gate_raw = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(grsrc, x * 2, 0, 0);
-    // ... or what the row's factor and its gates are summed from (lyra_decode_attention_rows), the gates 4 slices of a head per
-    // lane: requested here and not where they are summed, behind the cache tiles
-    [[maybe_unused]] float sq_raw = 0.f, gate_slices[4];
-    if constexpr (QKV == 2) {
-        const __amdgpu_buffer_rsrc_t sqrsrc = make_rsrc(p.row_sq, (uint32_t)(p.n_sq * p.B) * 4u);
-        const __amdgpu_buffer_rsrc_t gprsrc = make_rsrc(p.gate_part, p.gate_part ? (uint32_t)(p.gate_splits * p.B * p.N) * 4u : 0u);
-        sq_raw = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(sqrsrc, lane < p.n_sq ? (lane * p.B + b) * 4 : kNoLoad, 0, 0));
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            gate_slices[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                gprsrc, x < G && 4 * j + kb < p.gate_splits ? (((4 * j + kb) * p.B + b) * p.N + kh * G + x) * 4 : kNoLoad, 0, 0));
-    }
+    const uint16_t gate_raw = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(grsrc, x * 2, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
 
     // First tile of this wavefront: requested next.  Without a sliding window the chunk starts at a
@@ -667,7 +644,7 @@ void decode_attention_kernel(AttnParams p) {
     // QKV: this workgroup appends the new token's key and value when its chunk holds them, through the wavefront that
     // reads that key's tile (kv_wave); when the tile is that wavefront's first, it is requested a second time after the
     // rows have been written (`redo`).
-    [[maybe_unused]] const bool owner = QKV != 0 && pos >= 0 && pos < p.S && pos >= c_lo && pos < c_lo + chunk;
+    [[maybe_unused]] const bool owner = QKV && pos >= 0 && pos < p.S && pos >= c_lo && pos < c_lo + chunk;
     [[maybe_unused]] const int kv_wave = owner ? ((pos - c_lo) / kTile) % WAVES : -1;
     [[maybe_unused]] const bool redo = owner && wave == kv_wave && (pos - c_lo) / kTile < WAVES;
     [[maybe_unused]] float rope_cs = 0.f, rope_sn = 0.f;
@@ -685,14 +662,6 @@ void decode_attention_kernel(AttnParams p) {
     uint16_t* sm_q = (uint16_t*)smem;
     static_assert(WAVES * 64 >= 16 * (H / 8), "one q piece per thread");
     if constexpr (QKV) {
-        if constexpr (QKV == 2) {
-            row_factor = rsqrtf(wave_sum(sq_raw) / (float)p.sq_width + p.sq_eps);
-            if (p.gate_part) {
-                const float g = group4_sum((gate_slices[0] + gate_slices[1]) + (gate_slices[2] + gate_slices[3])) * row_factor;
-                gate_raw = f32_to_bf16_bits(2.f / (1.f + __expf(-g)));
-                if (wave == 0 && kb == 0) sm_gq[x] = bf16_bits_to_f32(gate_raw);
-            }
-        }
         if (q_row >= G) *(u32x4*)(sm_q + q_row * QP + q_piece * 8) = q_raw;  // zeros
         constexpr int half = H / 2;
         if (p.qkv_splits > kFirstSlices) {  // (projections of few rows are cut into more slices)
@@ -715,7 +684,7 @@ void decode_attention_kernel(AttnParams p) {
                 request_head<H, kFirstSlices>(p, part_rsrc, qkv_rsrc, b, kh * G + t, true, lane, hq);
             }
             float a, c;
-            sum_head<H>(p, part_rsrc, b, kh * G + t, lane, hq, row_factor, a, c);
+            sum_head<H>(p, part_rsrc, b, kh * G + t, lane, hq, a, c);
             head_norm_rope(a, c, p.qnorm != nullptr, qn_a, qn_c, rope_cs, rope_sn, p.norm_eps, H);
             if (lane < half) {
                 sm_q[t * QP + lane] = f32_to_bf16_bits(a);
@@ -726,7 +695,7 @@ void decode_attention_kernel(AttnParams p) {
             uint8_t* stage = (uint8_t*)(smem + p.xsa_lds);
             const bool is_k = wave == WAVES - 1;
             float a, c;
-            sum_head<H>(p, part_rsrc, b, is_k ? p.N + kh : p.N + p.K + kh, lane, hkv, row_factor, a, c);
+            sum_head<H>(p, part_rsrc, b, is_k ? p.N + kh : p.N + p.K + kh, lane, hkv, a, c);
             if (is_k) head_norm_rope(a, c, p.knorm != nullptr, kn_a, kn_c, rope_cs, rope_sn, p.norm_eps, H);
             stage_row<H, FP8>(stage, is_k ? 0 : 1, lane, a, c);
         }
@@ -808,7 +777,7 @@ void decode_attention_kernel(AttnParams p) {
     float* sm_gate = sm_sink + 16;                  // [16] loop below then reads no global memory between its stores
     if (wave == 0 && kb == 0 && x < G) {
         sm_sink[x] = sink2;
-        sm_gate[x] = p.has_gate ? bf16_bits_to_f32(gate_raw) : 1.f;
+        sm_gate[x] = p.gate ? bf16_bits_to_f32(gate_raw) : 1.f;
     }
     if (x < G) {
         float* dst = sm_o + ((size_t)wave * G + x) * HP;
@@ -909,7 +878,7 @@ void decode_attention_kernel(AttnParams p) {
                 for (int u = 0; u < 8; ++u)
                     if (c0 + u < n_valid) o += v[u] * sm_w[(c0 + u) * G + g];
             }
-            const float gate = p.gate ? bf16_bits_to_f32(p.gate[(size_t)b * p.N + n]) : (QKV == 2 && p.gate_part ? sm_gq[g] : 1.f);
+            const float gate = p.gate ? bf16_bits_to_f32(p.gate[(size_t)b * p.N + n]) : 1.f;
             if (p.xsa_v) smem[p.xsa_lds + idx] = gated(p, o / sm_den[g], gate);
             else store_out(p, ((size_t)b * p.N + n) * H + col, o / sm_den[g], gate);
         }
@@ -930,7 +899,7 @@ void decode_attention_kernel(AttnParams p) {
             den += load_agent(ml + 1) * f;
             o += load_agent(p.part_o + ((item0 + c) * G + g) * H + col) * f;
         }
-        const float gate = p.gate ? bf16_bits_to_f32(p.gate[(size_t)b * p.N + n]) : (QKV == 2 && p.gate_part ? sm_gq[g] : 1.f);
+        const float gate = p.gate ? bf16_bits_to_f32(p.gate[(size_t)b * p.N + n]) : 1.f;
         if (p.xsa_v) smem[p.xsa_lds + idx] = gated(p, o / den, gate);
         else store_out(p, ((size_t)b * p.N + n) * H + col, o / den, gate);
     }
@@ -1249,12 +1218,6 @@ struct QkvFront {
     const float *qnorm, *knorm, *cos_t, *sin_t;
     int rope_rows;
     float eps;
-    // lyra_decode_attention_rows
-    const float* row_sq = nullptr;
-    int n_sq = 0, sq_width = 1;
-    float sq_eps = 0.f;
-    const float* gate_part = nullptr;
-    int gate_splits = 0;
 };
 
 static int run_attention(const void* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
@@ -1336,11 +1299,6 @@ static int run_attention(const void* q, const void* k, const void* v, const floa
     p.qnorm = p.knorm = p.cos_t = p.sin_t = nullptr;
     p.rope_rows = 0;
     p.norm_eps = 0.f;
-    p.row_sq = p.gate_part = nullptr;
-    p.n_sq = p.gate_splits = 0;
-    p.sq_width = 1;
-    p.sq_eps = 0.f;
-    p.has_gate = gate != nullptr;
     if (front) {
         p.qkv_partials = front->partials;
         p.qkv = (const uint16_t*)front->qkv;
@@ -1352,13 +1310,6 @@ static int run_attention(const void* q, const void* k, const void* v, const floa
         p.sin_t = front->sin_t;
         p.rope_rows = front->rope_rows;
         p.norm_eps = front->eps;
-        p.row_sq = front->row_sq;
-        p.n_sq = front->n_sq;
-        p.sq_width = front->sq_width;
-        p.sq_eps = front->sq_eps;
-        p.gate_part = front->gate_part;
-        p.gate_splits = front->gate_splits;
-        if (p.gate_part) p.has_gate = 1;
     }
     p.arrivals = nullptr;
     if (pl.n_chunks > 1) {
@@ -1444,10 +1395,8 @@ static int run_attention(const void* q, const void* k, const void* v, const floa
 #define LYRA_LAUNCH_ATTN(HH, F, V)                              \
     do {                                                        \
         if (front) {                                            \
-            if (p.row_sq && sliding_window == 0) hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, 4, true, 1, 2>), grid, block, lds, st, p); \
-            else if (p.row_sq) hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, 4, false, 1, 2>), grid, block, lds, st, p); \
-            else if (sliding_window == 0) hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, 4, true, 1, 1>), grid, block, lds, st, p); \
-            else hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, 4, false, 1, 1>), grid, block, lds, st, p); \
+            if (sliding_window == 0) hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, 4, true, 1, true>), grid, block, lds, st, p); \
+            else hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, 4, false, 1, true>), grid, block, lds, st, p); \
         } else if (pl.waves == 4) LYRA_LAUNCH_ATTN_W(HH, F, V, 4); \
         else if (pl.waves == 8) LYRA_LAUNCH_ATTN_W(HH, F, V, 8); \
         else LYRA_LAUNCH_ATTN_W(HH, F, V, 16);                  \
@@ -1516,27 +1465,6 @@ extern "C" int lyra_decode_attention_qkv_bias(const void* qkv, const float* part
     if (qkv_bias && !partials) return LYRA_E_BADARG;  // (a summed projection already carries its bias)
     const lyra::QkvFront front{qkv, partials, splits, qkv_bias, qnorm, knorm, cos_t, sin_t, rope_rows, eps};
     return lyra::run_attention(nullptr, k, v, k_scale, v_scale, sinks, position, position_stride, gate, out, workspace,
-                               workspace_bytes, LYRA_E_WORKSPACE, false, nullptr, nullptr, B, N, K, S, H, sm_scale,
-                               sliding_window, kv_dtype, out_dtype, stream, &front);
-}
-
-extern "C" int lyra_decode_attention_rows(const float* partials, int splits, const float* qkv_bias, const float* sq, int n_sq,
-                                          int sq_width, float sq_eps, const float* gate_part, int gate_splits, const float* qnorm,
-                                          const float* knorm, const float* cos_t, const float* sin_t, int rope_rows, float eps,
-                                          void* k, void* v, float* k_scale, float* v_scale, const float* sinks,
-                                          const int32_t* position, int position_stride, void* out, void* workspace,
-                                          size_t workspace_bytes, int B, int N, int K, int S, int H, float sm_scale,
-                                          int sliding_window, int kv_dtype, int out_dtype, lyra_stream_t stream) {
-    if (!partials || !sq || n_sq <= 0 || sq_width <= 0 || (gate_part && gate_splits <= 0)) return LYRA_E_BADARG;
-    if (n_sq > 64 || gate_splits > 16) return LYRA_E_UNSUPPORTED;
-    lyra::QkvFront front{nullptr, partials, splits, qkv_bias, qnorm, knorm, cos_t, sin_t, rope_rows, eps};
-    front.row_sq = sq;
-    front.n_sq = n_sq;
-    front.sq_width = sq_width;
-    front.sq_eps = sq_eps;
-    front.gate_part = gate_part;
-    front.gate_splits = gate_splits;
-    return lyra::run_attention(nullptr, k, v, k_scale, v_scale, sinks, position, position_stride, nullptr, out, workspace,
                                workspace_bytes, LYRA_E_WORKSPACE, false, nullptr, nullptr, B, N, K, S, H, sm_scale,
                                sliding_window, kv_dtype, out_dtype, stream, &front);
 }

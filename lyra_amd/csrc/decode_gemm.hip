@@ -1301,46 +1301,29 @@ __device__ __forceinline__ f32x4 load_f32x4_at(__amdgpu_buffer_rsrc_t rsrc, int 
 }
 
 // ---- K-split projections of a few rows that finish their own input ------------------------------------------------
-// With 8 rows or fewer the launches between two projections - the sum of the slices with the RMS norm, or with the SwiGLU -
-// cost more than what they do (4-5 us each, three per dense layer), so the projection behind them does it: each workgroup
-// sums its K columns of the rows while its weights come from memory, and keeps the result in LDS as the matrix operand.
-//   front 1  x = bf16(residual + bf16(bf16(sum) * out_scale)); operand bf16(x * norm_scale).  The norm's factor of a row
-//            needs the whole row and is one number per row, so it is left to the consumer of the product: the workgroups
-//            of span 0 write x and their columns' sum of x^2.  One more workgroup per K slice forms the slice of a narrow
-//            float32 projection of the same operand (the output gate).
-//   front 2  operand bf16(swiglu(factor * sum(gate) + bias, factor * sum(linear) + bias)), factor from those sums of squares.
-// What bounds it is what a compute unit takes in: every span's workgroups repeat the sums of their K slice, at 8 rows 65-131 KB
-// from L2 beside 32-128 KB of weights.  lyra-small, us per dense layer (q/k/v, up and down projection with the norms and the
-// finish launch in front of them, in the captured step): 1 row 27.0 -> 19.2, 8 rows 30.4 -> 22.7, 16 rows 30.8 -> 30.6 and the
-// whole step 1008 -> 1052, hence the limit.  8 wavefronts instead of 4: 0.7-0.9 us slower per launch of 256-row slices, 0.9 us
-// faster for the 512-row slices of the up projection.
-constexpr int kRowsMax = 8;
+// A down projection of a few rows whose operand is the SwiGLU of an up projection left in K slices: each workgroup sums its K
+// columns of the rows' slices, applies bias and SwiGLU as the finish kernel does, element for element in its order, and keeps
+// the bf16 result in LDS as the matrix operand.  The launch that would do it in between costs 3-4 us for little work; here the
+// sums arrive while the weights come from memory.  What bounds it is what a compute unit takes in: every span's workgroups
+// repeat the sums of their K slice, at 8 rows 65 KB from L2 beside 32 KB of weights (lyra-small in FP8, us in the captured step:
+// finish 3.0 + down 4.9 -> 5.7 at 1 row, 4.0 + 4.9 -> 6.2 at 8, 4.0 + 4.6 -> 7.8 at 16; beyond that the sums outgrow the launch).
+// (The RMS norm went the same way, its row factor left to the consumer of the product: 3-4 us less per norm at up to 8 rows.
+// Taken back: the operand then skips one of the reference's roundings, and 2 of 100 single-sequence steps sent a token to
+// another expert.)
+constexpr int kRowsMax = 16;
 constexpr int kRowsWaves = 4;
-constexpr int kRowsSlices = 12;  // slices (front 2: half as many pairs) requested at once per item; further ones one by one
-constexpr int kRowsGates = 4 * kRowsWaves;   // outputs of the narrow projection: 16 lanes each
-constexpr int kRowsSqMax = 64;   // partial sums of squares of a row: one per lane
+constexpr int kRowsSlices = 6;  // slices of both halves requested at once per item; further ones one by one
 
 struct RowsFront {
-    const float* sums;  // [splits, M, K] (front 2: [splits, M, 2 K], gate columns first)
+    const float* sums;  // [splits, M, 2 K], gate columns first
     int splits;
-    const float* sum_bias;     // front 1: [K], added to the bf16 sum in bf16; front 2: [2 K], added to the float32 product; or null
-    const uint16_t* residual;  // front 1: [M, K]
-    float out_scale;
-    const float* norm_scale;  // front 1: [K]
-    uint16_t* x_out;          // front 1: [M, K]
-    float* sq_out;            // front 1: [n_sq, M] sums of x^2 over 256 columns each (fewer at the end of a slice)
-    const float* gate_w;      // front 1: [gate_n, K] or null
-    int gate_n;
-    float* gate_part;  // [ksplit, M, gate_n], gate_n <= kRowsGates
-    const float* sq;   // front 2: [n_sq, M]
-    int n_sq, sq_width;
-    float eps;
-    float beta, limit;  // front 2
+    const float* bias;  // [2 K] or null
+    float beta, limit;
 };
 
 #if LYRA_GEMM_HAS_SPLITK
 // ITEMS: how many items of sums a wavefront requests at once.
-template <int FP8, int DEPTH, int STEP_SCALES, int FRONT, int ITEMS>
+template <int FP8, int DEPTH, int STEP_SCALES, int ITEMS>
 __global__ __launch_bounds__(kRowsWaves * 64) void decode_gemm_rows_kernel(GemmParams p, RowsFront f) {
     constexpr int ES = FP8 ? 1 : 2;
     extern __shared__ float sm_part[];  // [kRowsWaves][16][kSplitPitch], then the operand: [4 * DEPTH steps][4][16 rows][8] bf16
@@ -1349,8 +1332,7 @@ __global__ __launch_bounds__(kRowsWaves * 64) void decode_gemm_rows_kernel(GemmP
     const int x = lane & 15, kb = lane >> 4;
     // (K slices vary fastest: the workgroups of an XCD, every eighth, then share few slices' sums in their L2)
     const int span = blockIdx.y, ks = blockIdx.x;
-    const bool gate_wg = FRONT == 1 && f.gate_n > 0 && span == (int)gridDim.y - 1;
-    const bool cols = !gate_wg && span * 128 + 8 * x < p.N;
+    const bool cols = span * 128 + 8 * x < p.N;
     const int ncol = cols ? span * 128 + 8 * x : 0;
     const int k0 = ks * p.kpart, k1 = min(p.K, k0 + p.kpart);
     const int steps = (k1 - k0) >> 5;
@@ -1359,36 +1341,22 @@ __global__ __launch_bounds__(kRowsWaves * 64) void decode_gemm_rows_kernel(GemmP
 
     // ---- the sums: item = (row, 256 columns of the slice), 4 columns per lane; a wavefront takes every fourth, ITEMS at a time
     const int nch = (p.kpart + 255) >> 8, n_items = p.M * nch;
-    const int width = FRONT == 2 ? 2 * p.K : p.K;
+    const int width = 2 * p.K;
     const __amdgpu_buffer_rsrc_t srsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float*>(f.sums), 0, (uint32_t)f.splits * (uint32_t)p.M * (uint32_t)width * 4u, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rrsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(f.residual), 0, FRONT == 1 ? (uint32_t)p.M * (uint32_t)p.K * 2u : 0u, 0x00020000);
-    const __amdgpu_buffer_rsrc_t nrsrc =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(f.norm_scale), 0, FRONT == 1 ? (uint32_t)p.K * 4u : 0u, 0x00020000);
-    const __amdgpu_buffer_rsrc_t qrsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float*>(f.sq), 0, FRONT == 2 ? (uint32_t)f.n_sq * (uint32_t)p.M * 4u : 0u, 0x00020000);
     const int slab = p.M * width * 4;
-    f32x4 u[ITEMS][kRowsSlices], gs[ITEMS];
-    u32x2 res[ITEMS];
-    float sq[ITEMS];
+    f32x4 u[ITEMS][2 * kRowsSlices];
     auto row_of = [&](int item) { return item / nch; };
     auto col_of = [&](int item) { return k0 + (item - row_of(item) * nch) * 256 + lane * 4; };
     auto request = [&](int i, int item) {
         const int row = row_of(item), c = col_of(item);
         const bool live = item < n_items && c < k1;
         const int off = live ? (row * width + c) * 4 : kNoLoad;
-        if constexpr (FRONT == 2) sq[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(qrsrc, item < n_items && lane < f.n_sq ? (lane * p.M + row) * 4 : kNoLoad, 0, 0));
-        constexpr int per = FRONT == 2 ? kRowsSlices / 2 : kRowsSlices;
 #pragma unroll
-        for (int s = 0; s < per; ++s) {
+        for (int s = 0; s < kRowsSlices; ++s) {
             const int soff = __builtin_amdgcn_readfirstlane(s < f.splits ? s * slab : 0), voff = s < f.splits ? off : kNoLoad;
             u[i][s] = load_f32x4_at(srsrc, voff, soff);
-            if constexpr (FRONT == 2) u[i][per + s] = load_f32x4_at(srsrc, voff == kNoLoad ? kNoLoad : voff + p.K * 4, soff);
-        }
-        if constexpr (FRONT == 1) {
-            gs[i] = load_f32x4_at(nrsrc, live ? c * 4 : kNoLoad, 0);
-            res[i] = __builtin_amdgcn_raw_buffer_load_b64(rrsrc, live ? (row * p.K + c) * 2 : kNoLoad, 0, 0);
+            u[i][kRowsSlices + s] = load_f32x4_at(srsrc, voff == kNoLoad ? kNoLoad : voff + p.K * 4, soff);
         }
     };
 #pragma unroll
@@ -1396,24 +1364,10 @@ __global__ __launch_bounds__(kRowsWaves * 64) void decode_gemm_rows_kernel(GemmP
     __builtin_amdgcn_sched_barrier(0);
 
     // ---- the weights of the whole slice, requested behind the sums (loads return in order) ----
-    // (the narrow projection's workgroup instead: 16 lanes hold the slice of one output)
-    constexpr int kGateLoads = DEPTH * kRowsWaves / 2;  // 64 columns each
-    [[maybe_unused]] f32x4 gw[kGateLoads];
-    if constexpr (FRONT == 1) {
-        const __amdgpu_buffer_rsrc_t gwrsrc = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<float*>(f.gate_w), 0, gate_wg ? (uint32_t)f.gate_n * (uint32_t)p.K * 4u : 0u, 0x00020000);
-        if (gate_wg) {
-#pragma unroll
-            for (int i = 0; i < kGateLoads; ++i) {
-                const int j = threadIdx.x >> 4, c = k0 + (i * 16 + x) * 4;
-                gw[i] = load_f32x4_at(gwrsrc, j < f.gate_n && c < k1 ? (j * p.K + c) * 4 : kNoLoad, 0);
-            }
-        }
-    }
     const int row_bytes = p.packed ? 128 * ES : p.N * ES;
     const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(p.rhs) + (p.packed && !gate_wg ? (size_t)span * p.K * row_bytes : (size_t)0), 0,
-        gate_wg ? 0u : (uint32_t)p.K * (uint32_t)row_bytes, 0x00020000);
+        const_cast<uint8_t*>(p.rhs) + (p.packed ? (size_t)span * p.K * row_bytes : (size_t)0), 0,
+        (uint32_t)p.K * (uint32_t)row_bytes, 0x00020000);
     const int wvoff = cols ? 8 * kb * row_bytes + (p.packed ? 8 * x : ncol) * ES : kNoLoad;
     RawW<FP8> w[DEPTH];
 #pragma unroll
@@ -1447,63 +1401,37 @@ __global__ __launch_bounds__(kRowsWaves * 64) void decode_gemm_rows_kernel(GemmP
 
     auto finish = [&](int i, int item) {
         const int row = row_of(item), c = col_of(item);
-        constexpr int per = FRONT == 2 ? kRowsSlices / 2 : kRowsSlices;
         f32x4 t = f32x4{0.f, 0.f, 0.f, 0.f}, l = t;
 #pragma unroll
-        for (int s = 0; s < per; ++s) {
+        for (int s = 0; s < kRowsSlices; ++s) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 t[e] += u[i][s][e];
-                if constexpr (FRONT == 2) l[e] += u[i][per + s][e];
+                l[e] += u[i][kRowsSlices + s][e];
             }
         }
         const bool live = item < n_items && c < k1;
-        for (int s = per; s < f.splits; ++s) {
+        for (int s = kRowsSlices; s < f.splits; ++s) {
             const int off = live ? (row * width + c) * 4 : kNoLoad, soff = __builtin_amdgcn_readfirstlane(s * slab);
-            const f32x4 a = load_f32x4_at(srsrc, off, soff);
-            [[maybe_unused]] f32x4 b;
-            if constexpr (FRONT == 2) b = load_f32x4_at(srsrc, live ? off + p.K * 4 : kNoLoad, soff);
+            const f32x4 a = load_f32x4_at(srsrc, off, soff), b = load_f32x4_at(srsrc, live ? off + p.K * 4 : kNoLoad, soff);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 t[e] += a[e];
-                if constexpr (FRONT == 2) l[e] += b[e];
+                l[e] += b[e];
             }
         }
-        u32x2 a;
-        if constexpr (FRONT == 1) {
-            if (f.sum_bias) {
+        float o[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) t[e] = round_bf16(round_bf16(t[e]) + (live ? f.sum_bias[c + e] : 0.f));
+        for (int e = 0; e < 4; ++e) {
+            if (f.bias) {
+                t[e] += live ? f.bias[c + e] : 0.f;
+                l[e] += live ? f.bias[p.K + c + e] : 0.f;
             }
-            const float r[4] = {__uint_as_float(res[i][0] << 16), __uint_as_float(res[i][0] & 0xFFFF0000u),
-                                __uint_as_float(res[i][1] << 16), __uint_as_float(res[i][1] & 0xFFFF0000u)};
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = round_bf16(r[e] + round_bf16(round_bf16(t[e]) * f.out_scale));
-            float ss = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
-            ss = wave_sum(ss);
-            if (span == 0 && item < n_items) {  // (the same in every lane)
-                if (live) store_through((void*)f.x_out, ((size_t)row * p.K + c) * 2, u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])});
-                if (lane == 0) store_through(f.sq_out + (size_t)(ks * nch + item - row * nch) * p.M + row, ss);
-            }
-            a = u32x2{pack_bf16(v[0] * gs[i][0], v[1] * gs[i][1]), pack_bf16(v[2] * gs[i][2], v[3] * gs[i][3])};
-        } else {
-            const float factor = rsqrtf(wave_sum(sq[i]) / (float)f.sq_width + f.eps);
-            float o[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float g = t[e] * factor, n = l[e] * factor;
-                if (f.sum_bias) {
-                    g += live ? f.sum_bias[c + e] : 0.f;
-                    n += live ? f.sum_bias[p.K + c + e] : 0.f;
-                }
-                o[e] = swiglu_one(g, n, f.beta, f.limit);
-            }
-            a = u32x2{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
+            o[e] = swiglu_one(t[e], l[e], f.beta, f.limit);
         }
         if (live) {
             const int at = c - k0;
-            *(u32x2*)(sm_a + ((((at >> 5) * 4 + ((at >> 3) & 3)) * 16 + row) * 8 + (at & 7)) * 2) = a;
+            *(u32x2*)(sm_a + ((((at >> 5) * 4 + ((at >> 3) & 3)) * 16 + row) * 8 + (at & 7)) * 2) = u32x2{pack_bf16(o[0], o[1]), pack_bf16(o[2], o[3])};
         }
     };
     for (int item = wave;;) {
@@ -1515,29 +1443,6 @@ __global__ __launch_bounds__(kRowsWaves * 64) void decode_gemm_rows_kernel(GemmP
         for (int i = 0; i < ITEMS; ++i) request(i, item + i * kRowsWaves);
     }
     lds_barrier();  // (the weights stay in flight)
-
-    if constexpr (FRONT == 1) {
-        if (gate_wg) {  // 16 lanes per output: their columns of every row, then the sum over the lanes
-            const int j = threadIdx.x >> 4;
-            for (int row = 0; row < p.M; ++row) {
-                float acc = 0.f;
-#pragma unroll
-                for (int i = 0; i < kGateLoads; ++i) {
-                    const int c = (i * 16 + x) * 4;
-                    const u32x2 a = *(const u32x2*)(sm_a + ((((c >> 5) * 4 + ((c >> 3) & 3)) * 16 + row) * 8 + (c & 7)) * 2);
-                    const float s = __uint_as_float(a[0] << 16) * gw[i][0] + __uint_as_float(a[0] & 0xFFFF0000u) * gw[i][1] +
-                                    __uint_as_float(a[1] << 16) * gw[i][2] + __uint_as_float(a[1] & 0xFFFF0000u) * gw[i][3];
-                    acc += k0 + c < k1 ? s : 0.f;  // (what lies behind the slice in LDS was not written)
-                }
-                acc += dpp_row<0xB1>(acc);
-                acc += dpp_row<0x4E>(acc);
-                acc += dpp_row<0x141>(acc);
-                acc += dpp_row<0x140>(acc);
-                if (x == 0 && j < f.gate_n) store_through(f.gate_part + ((size_t)ks * p.M + row) * f.gate_n + j, acc);
-            }
-            return;
-        }
-    }
 
     f32x4 acc[8];
 #pragma unroll
@@ -2437,9 +2342,9 @@ static GemmPlan plan_gemm(int M, int G, int K, int N, int bk, int fused_swiglu, 
 // receives [ksplit, M, N] float32 slices.
 template <int WT>
 int launch_split_k_fmt(const GemmParams& p, const GemmPlan& pl, hipStream_t st);
-// ... the same for the kernel that finishes its own input (front 1 or 2).
+// ... the same for the kernel that finishes its own input.
 template <int WT>
-int launch_rows_fmt(const GemmParams& p, const RowsFront& f, int front, const GemmPlan& pl, hipStream_t st);
+int launch_rows_fmt(const GemmParams& p, const RowsFront& f, const GemmPlan& pl, hipStream_t st);
 // Sums the K slices in p.part and applies the epilogue (the finish kernel lives in the pass with the entry points).
 int launch_finish(const GemmParams& p, hipStream_t st);
 
@@ -2498,49 +2403,43 @@ int launch_split_k_fmt(const GemmParams& p, const GemmPlan& pl, hipStream_t st) 
 }
 
 template <int WT>
-int launch_rows_fmt(const GemmParams& p, const RowsFront& f, int front, const GemmPlan& pl, hipStream_t st) {
+int launch_rows_fmt(const GemmParams& p, const RowsFront& f, const GemmPlan& pl, hipStream_t st) {
     const int depth = pl.kpart <= 2 * kRowsWaves * 32 ? 2 : 4, items = (p.M * ((pl.kpart + 255) / 256) + kRowsWaves - 1) / kRowsWaves;
     const int step_scales = !(WT != 0 && p.scale_mode == 1 && p.bk < p.K) ? 0 : (p.bk % (32 * depth) == 0 ? 1 : 2);
-    const dim3 grid(pl.ksplit, pl.spans + (front == 1 && f.gate_n > 0 ? 1 : 0)), block(kRowsWaves * 64);
+    const dim3 grid(pl.ksplit, pl.spans), block(kRowsWaves * 64);
     // (more than half of a compute unit's 160 KB: workgroups are spread one per unit)
     const size_t lds = (size_t)88 * 1024;
     static_assert(kRowsWaves * 16 * kSplitPitch * sizeof(float) + 4 * kRowsWaves * 1024 <= 88 * 1024, "partial tiles and the operand");
-#define LYRA_ROWS(D, S, F, I)                                                                                          \
+#define LYRA_ROWS(...)                                                                                                 \
     do {                                                                                                              \
-        static const hipError_t attr = hipFuncSetAttribute((const void*)decode_gemm_rows_kernel<WT, D, S, F, I>,       \
+        static const hipError_t attr = hipFuncSetAttribute((const void*)decode_gemm_rows_kernel<WT, __VA_ARGS__>,      \
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);     \
         if (attr != hipSuccess) return LYRA_E_LAUNCH;                                                                 \
-        hipLaunchKernelGGL((decode_gemm_rows_kernel<WT, D, S, F, I>), grid, block, lds, st, p, f);                     \
+        hipLaunchKernelGGL((decode_gemm_rows_kernel<WT, __VA_ARGS__>), grid, block, lds, st, p, f);                    \
     } while (0)
-#define LYRA_ROWS_I(D, S, F)                \
-    do {                                    \
-        if (items <= 1) LYRA_ROWS(D, S, F, 1); \
-        else LYRA_ROWS(D, S, F, 2);         \
-    } while (0)
-#define LYRA_ROWS_S(D, F)                      \
-    do {                                       \
-        if (WT == 0 || step_scales == 0) LYRA_ROWS_I(D, 0, F); \
-        else if (step_scales == 1) LYRA_ROWS_I(D, (WT ? 1 : 0), F); \
-        else LYRA_ROWS_I(D, (WT ? 2 : 0), F);  \
-    } while (0)
-#define LYRA_ROWS_F(F)                        \
+#define LYRA_ROWS_I(D, S)                     \
     do {                                      \
-        if (depth == 2) LYRA_ROWS_S(2, F);    \
-        else LYRA_ROWS_S(4, F);               \
+        if (items <= 1) LYRA_ROWS(D, S, 1);   \
+        else LYRA_ROWS(D, S, 2);              \
     } while (0)
-    if (front == 1) LYRA_ROWS_F(1);
-    else LYRA_ROWS_F(2);
-#undef LYRA_ROWS_F
+#define LYRA_ROWS_S(D)                                                      \
+    do {                                                                    \
+        if (WT == 0 || step_scales == 0) LYRA_ROWS_I(D, 0);                 \
+        else if (step_scales == 1) LYRA_ROWS_I(D, (WT ? 1 : 0));            \
+        else LYRA_ROWS_I(D, (WT ? 2 : 0));                                  \
+    } while (0)
+    if (depth == 2) LYRA_ROWS_S(2);
+    else LYRA_ROWS_S(4);
 #undef LYRA_ROWS_S
 #undef LYRA_ROWS_I
 #undef LYRA_ROWS
     return hipGetLastError() == hipSuccess ? LYRA_OK : LYRA_E_LAUNCH;
 }
 #if LYRA_GEMM_PART == 2
-template int launch_rows_fmt<0>(const GemmParams&, const RowsFront&, int, const GemmPlan&, hipStream_t);
-template int launch_rows_fmt<1>(const GemmParams&, const RowsFront&, int, const GemmPlan&, hipStream_t);
+template int launch_rows_fmt<0>(const GemmParams&, const RowsFront&, const GemmPlan&, hipStream_t);
+template int launch_rows_fmt<1>(const GemmParams&, const RowsFront&, const GemmPlan&, hipStream_t);
 #elif LYRA_GEMM_PART == 4
-template int launch_rows_fmt<2>(const GemmParams&, const RowsFront&, int, const GemmPlan&, hipStream_t);
+template int launch_rows_fmt<2>(const GemmParams&, const RowsFront&, const GemmPlan&, hipStream_t);
 #endif
 #if LYRA_GEMM_PART == 2
 template int launch_split_k_fmt<0>(const GemmParams&, const GemmPlan&, hipStream_t);
@@ -3012,30 +2911,10 @@ static int partials_params(const void* lhs, const void* rhs, const float* rhs_sc
     return LYRA_OK;
 }
 
-// Partial sums of squares per row that front 1 writes for a plan: 0 where the kernel that finishes its own input does not exist
-// (more rows than one matrix tile holds, slices longer than its registers).
-static int rows_sums(const GemmPlan& pl, int M, int K) {
-    if (!pl.split_k || M > kRowsMax || pl.row_block != 16 || pl.kpart > 4 * kRowsWaves * 32 || K % 4) return 0;
-    const int n = pl.ksplit * ((pl.kpart + 255) / 256);
-    return n <= kRowsSqMax ? n : 0;
-}
-
-static int run_rows(const RowsFront& f, int front, const void* rhs, const float* rhs_scale, int bk, int bn, float* partials,
-                    size_t partials_bytes, int M, int K, int N, int rhs_dtype, lyra_stream_t stream) {
-    GemmParams p;
-    GemmPlan pl;
-    if (rhs_dtype & LYRA_LHS_TILED16) return LYRA_E_UNSUPPORTED;  // (there is no lhs)
-    const int rc = partials_params(f.sums, rhs, rhs_scale, bk, bn, (const int32_t*)f.sums, partials, partials_bytes, M, K, N, rhs_dtype, p, pl);
-    if (rc != LYRA_OK) return rc;
-    if (rows_sums(pl, M, K) == 0) return LYRA_E_UNSUPPORTED;
-    const size_t width = front == 2 ? 2 * (size_t)K : (size_t)K;
-    if ((size_t)f.splits * M * width * 4 >= (1ull << 31)) return LYRA_E_UNSUPPORTED;
-    p.lhs = nullptr;
-    p.group_sizes = nullptr;
-    const int fmt = rhs_dtype & ~LYRA_RHS_SPAN_MAJOR;
-    if (fmt == LYRA_DTYPE_E5M2) return launch_rows_fmt<2>(p, f, front, pl, (hipStream_t)stream);
-    return fmt == LYRA_DTYPE_E4M3FN ? launch_rows_fmt<1>(p, f, front, pl, (hipStream_t)stream)
-                                    : launch_rows_fmt<0>(p, f, front, pl, (hipStream_t)stream);
+// Whether the kernel that finishes its own input takes a plan: no more rows than one matrix tile holds, no longer slices than
+// its registers.
+static bool rows_exists(const GemmPlan& pl, int M, int K) {
+    return pl.split_k && M <= kRowsMax && pl.row_block == 16 && pl.kpart <= 4 * kRowsWaves * 32 && K % 4 == 0;
 }
 }  // namespace lyra
 
@@ -3052,39 +2931,27 @@ extern "C" int lyra_decode_gemm_partials(const void* lhs, const void* rhs, const
     return one_byte_format(rhs_dtype) ? launch_split_k_fmt<1>(p, pl, (hipStream_t)stream) : launch_split_k_fmt<0>(p, pl, (hipStream_t)stream);
 }
 
-extern "C" int lyra_rows_proj_sums(int M, int K, int N, int bk) {
+extern "C" int lyra_rows_proj_swiglu_exists(int M, int K, int N, int bk) {
     if (M <= 0 || K <= 0 || N <= 0 || K % 32 || N % 8) return 0;
-    return lyra::rows_sums(lyra::plan_gemm(M, 1, K, N, bk, 0), M, K);
+    return lyra::rows_exists(lyra::plan_gemm(M, 1, K, N, bk, 0), M, K) ? 1 : 0;
 }
 
-extern "C" int lyra_rows_proj_norm(const float* sums, int splits, const float* sum_bias, const void* residual, float out_scale,
-                                   const float* norm_scale, void* x_out, float* sq_out, const float* gate_t, int gate_n,
-                                   float* gate_part, const void* rhs, const float* rhs_scale, int bk, int bn, float* partials,
-                                   size_t partials_bytes, int M, int K, int N, int rhs_dtype, lyra_stream_t stream) {
-    if (!sums || splits <= 0 || !residual || !norm_scale || !x_out || !sq_out || gate_n < 0) return LYRA_E_BADARG;
-    if (gate_n > 0 && (!gate_t || !gate_part)) return LYRA_E_BADARG;
-    if (gate_n > lyra::kRowsGates || (size_t)gate_n * K * 4 >= (1ull << 31)) return LYRA_E_UNSUPPORTED;
-    if (((uintptr_t)sums | (uintptr_t)gate_t) % 16 || ((uintptr_t)residual | (uintptr_t)x_out) % 8) return LYRA_E_UNSUPPORTED;
-    lyra::RowsFront f = {};
-    f.sums = sums; f.splits = splits; f.sum_bias = sum_bias;
-    f.residual = (const uint16_t*)residual;
-    f.out_scale = out_scale;
-    f.norm_scale = norm_scale;
-    f.x_out = (uint16_t*)x_out;
-    f.sq_out = sq_out;
-    f.gate_w = gate_t; f.gate_n = gate_n; f.gate_part = gate_part;
-    return lyra::run_rows(f, 1, rhs, rhs_scale, bk, bn, partials, partials_bytes, M, K, N, rhs_dtype, stream);
-}
-
-extern "C" int lyra_rows_proj_swiglu(const float* sums, int splits, const float* bias, const float* sq, int n_sq, int sq_width,
-                                     float eps, float beta, float limit, const void* rhs, const float* rhs_scale, int bk, int bn,
-                                     float* partials, size_t partials_bytes, int M, int K, int N, int rhs_dtype, lyra_stream_t stream) {
-    if (!sums || splits <= 0 || !sq || n_sq <= 0 || sq_width <= 0) return LYRA_E_BADARG;
-    if (n_sq > lyra::kRowsSqMax || (uintptr_t)sums % 16) return LYRA_E_UNSUPPORTED;
-    lyra::RowsFront f = {};
-    f.sums = sums; f.splits = splits; f.sum_bias = bias;
-    f.sq = sq; f.n_sq = n_sq; f.sq_width = sq_width; f.eps = eps;
-    f.beta = beta; f.limit = limit;
-    return lyra::run_rows(f, 2, rhs, rhs_scale, bk, bn, partials, partials_bytes, M, K, N, rhs_dtype, stream);
+extern "C" int lyra_rows_proj_swiglu(const float* sums, int splits, const float* bias, float beta, float limit, const void* rhs,
+                                     const float* rhs_scale, int bk, int bn, float* partials, size_t partials_bytes, int M, int K,
+                                     int N, int rhs_dtype, lyra_stream_t stream) {
+    using namespace lyra;
+    if (!sums || splits <= 0) return LYRA_E_BADARG;
+    if ((rhs_dtype & LYRA_LHS_TILED16) || (uintptr_t)sums % 16) return LYRA_E_UNSUPPORTED;  // (there is no lhs)
+    GemmParams p;
+    GemmPlan pl;
+    const int rc = partials_params(sums, rhs, rhs_scale, bk, bn, (const int32_t*)sums, partials, partials_bytes, M, K, N, rhs_dtype, p, pl);
+    if (rc != LYRA_OK) return rc;
+    if (!rows_exists(pl, M, K) || (size_t)splits * M * 2 * K * 4 >= (1ull << 31)) return LYRA_E_UNSUPPORTED;
+    p.lhs = nullptr;
+    p.group_sizes = nullptr;
+    const RowsFront f = {sums, splits, bias, beta, limit};
+    const int fmt = rhs_dtype & ~LYRA_RHS_SPAN_MAJOR;
+    if (fmt == LYRA_DTYPE_E5M2) return launch_rows_fmt<2>(p, f, pl, (hipStream_t)stream);
+    return fmt == LYRA_DTYPE_E4M3FN ? launch_rows_fmt<1>(p, f, pl, (hipStream_t)stream) : launch_rows_fmt<0>(p, f, pl, (hipStream_t)stream);
 }
 #endif  // LYRA_GEMM_HAS_ENTRY

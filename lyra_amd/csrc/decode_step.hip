@@ -37,8 +37,6 @@ struct Stream {
     const int32_t* dest = nullptr;
 };
 
-constexpr int kNarrowest = 1024;  // columns from which the norm runs inside the projection behind it (as the Python driver has it)
-
 struct Step {
     const lyra_step_t& s;
     bool dry;  // sizes only: nothing is launched
@@ -86,50 +84,23 @@ struct Step {
     int attention(const lyra_layer_t& l, Stream& t) {
         const int W = (s.N + 2 * s.K) * s.H, heads = s.N * s.H;
         const int splits = lyra_decode_gemm_splits(s.B, s.C, W, l.qkv.scale ? l.qkv.bk : 0);
-        void* out = nullptr;
-        const void* x = nullptr;
-        // (16 gates and 16 slices of them are what the launches take)
-        const bool rows = t.kind == Stream::kSlices && s.C >= kNarrowest && (!l.gate_t || (s.N <= 16 && splits <= 16));
-        const int n_sq = rows ? lyra_rows_proj_sums(s.B, s.C, W, l.qkv.scale ? l.qkv.bk : 0) : 0;
-        if (n_sq > 0) {
-            void* x_out = mem.take(bf16(s.B, s.C));
-            float* part = mem.take<float>(f32((size_t)splits * s.B * W));
-            float* sq = mem.take<float>(f32((size_t)n_sq * s.B));
-            float* gp = l.gate_t ? mem.take<float>(f32((size_t)splits * s.B * s.N)) : nullptr;
-            out = mem.take(bf16(s.B, heads));
-            if (mem.over) return LYRA_E_WORKSPACE;
-            if (!dry) {
-                int rc = lyra_rows_proj_norm(t.slices, t.splits, t.bias, t.x, t.scale, l.attn_norm, x_out, sq, l.gate_t, l.gate_t ? s.N : 0,
-                                             gp, l.qkv.data, l.qkv.scale, l.qkv.bk, l.qkv.bn, part, f32((size_t)splits * s.B * W), s.B,
-                                             s.C, W, l.qkv.dtype, st);
-                if (rc != LYRA_OK) return rc;
-                rc = lyra_decode_attention_rows(part, splits, l.qkv_bias, sq, n_sq, s.C, s.eps, gp, gp ? splits : 0, l.qnorm, l.knorm,
-                                                s.cos_t, s.sin_t, s.rope_rows, s.eps, l.k, l.v, l.ks, l.vs, l.sinks, s.position, 0, out,
+        void* h = mem.take(tiled(s.C));
+        void* gate = l.gate_t ? mem.take(bf16(s.B, s.N)) : nullptr;
+        int rc = norm(t, l.attn_norm, h, l.gate_t, nullptr, gate, l.gate_t ? s.N : 0, 1 | 4);
+        if (rc != LYRA_OK) return rc;
+        float* part = splits > 0 ? mem.take<float>(f32((size_t)splits * s.B * W)) : nullptr;
+        void* qkv = splits > 0 ? nullptr : mem.take(bf16(s.B, W));
+        void* out = mem.take(bf16(s.B, heads));
+        rc = splits > 0 ? partials(h, true, l.qkv, s.C, W, splits, part)
+                        : gemm(h, true, l.qkv, s.C, W, l.qkv_bias, l.qkv_bias ? 2 : 0, nullptr, 1.f, qkv);
+        if (rc != LYRA_OK) return rc;
+        if (!dry)
+            rc = lyra_decode_attention_qkv_bias(qkv, part, splits, splits > 0 ? l.qkv_bias : nullptr, l.qnorm, l.knorm, s.cos_t, s.sin_t,
+                                                s.rope_rows, s.eps, l.k, l.v, l.ks, l.vs, l.sinks, s.position, 0, gate, out,
                                                 s.attn_ws, s.attn_ws_bytes, s.B, s.N, s.K, l.S, s.H, s.sm_scale, l.sliding_window,
                                                 s.kv_dtype, LYRA_DTYPE_BF16, st);
-                if (rc != LYRA_OK) return rc;
-            }
-            x = x_out;
-        } else {
-            void* h = mem.take(tiled(s.C));
-            void* gate = l.gate_t ? mem.take(bf16(s.B, s.N)) : nullptr;
-            int rc = norm(t, l.attn_norm, h, l.gate_t, nullptr, gate, l.gate_t ? s.N : 0, 1 | 4);
-            if (rc != LYRA_OK) return rc;
-            x = t.x;
-            float* part = splits > 0 ? mem.take<float>(f32((size_t)splits * s.B * W)) : nullptr;
-            void* qkv = splits > 0 ? nullptr : mem.take(bf16(s.B, W));
-            out = mem.take(bf16(s.B, heads));
-            rc = splits > 0 ? partials(h, true, l.qkv, s.C, W, splits, part)
-                            : gemm(h, true, l.qkv, s.C, W, l.qkv_bias, l.qkv_bias ? 2 : 0, nullptr, 1.f, qkv);
-            if (rc != LYRA_OK) return rc;
-            if (!dry)
-                rc = lyra_decode_attention_qkv_bias(qkv, part, splits, splits > 0 ? l.qkv_bias : nullptr, l.qnorm, l.knorm, s.cos_t, s.sin_t,
-                                                    s.rope_rows, s.eps, l.k, l.v, l.ks, l.vs, l.sinks, s.position, 0, gate, out,
-                                                    s.attn_ws, s.attn_ws_bytes, s.B, s.N, s.K, l.S, s.H, s.sm_scale, l.sliding_window,
-                                                    s.kv_dtype, LYRA_DTYPE_BF16, st);
-            if (rc != LYRA_OK) return rc;
-        }
-        return leave(t, out, false, l.out, heads, l.out_bias, s.residual_scale, x);
+        if (rc != LYRA_OK) return rc;
+        return leave(t, out, false, l.out, heads, l.out_bias, s.residual_scale, t.x);
     }
 
     // one-group product summed by the launch itself; post: bits of lyra_decode_gemm_ex's post_scale
@@ -160,33 +131,27 @@ struct Step {
     }
 
     int dense(const lyra_layer_t& l, Stream& t) {
-        const int Hd = s.dense_hidden, bk_up = l.up.scale ? l.up.bk : 0, bk_down = l.down.scale ? l.down.bk : 0;
-        const int n_sq = t.kind == Stream::kSlices && s.C >= kNarrowest && lyra_rows_proj_sums(s.B, Hd, s.C, bk_down) > 0
-                             ? lyra_rows_proj_sums(s.B, s.C, 2 * Hd, bk_up) : 0;
-        if (n_sq > 0) {
-            const int up = lyra_decode_gemm_splits(s.B, s.C, 2 * Hd, bk_up), down = lyra_decode_gemm_splits(s.B, Hd, s.C, bk_down);
-            void* x = mem.take(bf16(s.B, s.C));
-            float* part = mem.take<float>(f32((size_t)up * s.B * 2 * Hd));
-            float* sq = mem.take<float>(f32((size_t)n_sq * s.B));
-            float* dpart = mem.take<float>(f32((size_t)down * s.B * s.C));
-            if (mem.over) return LYRA_E_WORKSPACE;
-            if (!dry) {
-                int rc = lyra_rows_proj_norm(t.slices, t.splits, t.bias, t.x, t.scale, l.mlp_norm, x, sq, nullptr, 0, nullptr, l.up.data,
-                                             l.up.scale, l.up.bk, l.up.bn, part, f32((size_t)up * s.B * 2 * Hd), s.B, s.C, 2 * Hd,
-                                             l.up.dtype, st);
-                if (rc != LYRA_OK) return rc;
-                rc = lyra_rows_proj_swiglu(part, up, l.up_bias, sq, n_sq, s.C, s.eps, s.beta, s.limit, l.down.data, l.down.scale, l.down.bk,
-                                           l.down.bn, dpart, f32((size_t)down * s.B * s.C), s.B, Hd, s.C, l.down.dtype, st);
-                if (rc != LYRA_OK) return rc;
-            }
-            t = Stream{};
-            t.kind = Stream::kSlices;
-            t.x = x; t.slices = dpart; t.splits = down; t.bias = l.down_bias; t.scale = s.dense_residual_scale;
-            return LYRA_OK;
-        }
+        const int Hd = s.dense_hidden;
         void* h = mem.take(tiled(s.C));
         void* act = mem.take(tiled(Hd));
         int rc = norm(t, l.mlp_norm, h, nullptr, nullptr, nullptr, 0, 2 | 4);
+        const int bk_down = l.down.scale ? l.down.bk : 0;
+        const int up = lyra_rows_proj_swiglu_exists(s.B, Hd, s.C, bk_down) ? lyra_decode_gemm_splits(s.B, s.C, 2 * Hd, l.up.scale ? l.up.bk : 0) : 0;
+        if (rc == LYRA_OK && up > 0) {  // a few rows: SwiGLU inside the down projection's launch
+            const int down = lyra_decode_gemm_splits(s.B, Hd, s.C, bk_down);
+            float* part = mem.take<float>(f32((size_t)up * s.B * 2 * Hd));
+            float* dpart = mem.take<float>(f32((size_t)down * s.B * s.C));
+            rc = partials(h, true, l.up, s.C, 2 * Hd, up, part);
+            if (rc == LYRA_OK && !dry)
+                rc = lyra_rows_proj_swiglu(part, up, l.up_bias, s.beta, s.limit, l.down.data, l.down.scale, l.down.bk, l.down.bn, dpart,
+                                           f32((size_t)down * s.B * s.C), s.B, Hd, s.C, l.down.dtype, st);
+            const void* x = t.x;
+            t = Stream{};
+            t.kind = Stream::kSlices;
+            t.x = x; t.slices = dpart; t.splits = down; t.bias = l.down_bias; t.scale = s.dense_residual_scale;
+            return rc;
+        }
+        if (rc == LYRA_OK && mem.over) rc = LYRA_E_WORKSPACE;
         if (rc == LYRA_OK && !dry)
             rc = lyra_decode_gemm_ex(h, nullptr, l.up.data, l.up.scale, l.up.bk, l.up.bn, one, l.up_bias, nullptr, 1.f, 0, act, s.gemm_ws,
                                      s.gemm_ws_bytes, s.B, 1, s.C, 2 * Hd, l.up.dtype | LYRA_LHS_TILED16 | LYRA_OUT_TILED16,

@@ -46,24 +46,13 @@ class Unsummed:
     follows it (``residual`` [M, N] bf16 and ``scale``), to be applied by the kernel that consumes it.  ``bias``: the
     projection's own bias [N] (float32 holding bf16 values), which the consumer adds to the bf16-rounded sum in bf16
     (lyra/model.py:310-313, 367-368, 629-630); the attention launch with the front step and the norm kernel take it,
-    ``qkv_post`` does not.  ``factor``: the slices lack their rows' norm factor, which the consumer forms from this
-    ``RowFactor`` (what ``rows_proj_norm`` returns; only ``rows_proj_swiglu`` and ``attention_qkv`` take it)."""
+    ``qkv_post`` does not."""
 
-    __slots__ = ("partials", "residual", "scale", "bias", "factor")
+    __slots__ = ("partials", "residual", "scale", "bias")
 
     def __init__(self, partials: torch.Tensor, residual: torch.Tensor | None = None, scale: float = 1.0,
-                 bias: torch.Tensor | None = None, factor: RowFactor | None = None):
-        self.partials, self.residual, self.scale, self.bias, self.factor = partials, residual, scale, bias, factor
-
-
-class RowFactor:
-    """rsqrt(mean(x^2) + eps) of every row, not formed yet: ``sq`` [n, M] float32 sums of x^2 over parts of a row of ``width``
-    columns.  ``gate``: slices [splits, M, heads] of the rows' output-gate projection, which lack the factor too."""
-
-    __slots__ = ("sq", "width", "eps", "gate")
-
-    def __init__(self, sq: torch.Tensor, width: int, eps: float, gate: torch.Tensor | None):
-        self.sq, self.width, self.eps, self.gate = sq, width, eps, gate
+                 bias: torch.Tensor | None = None):
+        self.partials, self.residual, self.scale, self.bias = partials, residual, scale, bias
 
 
 class Uncombined:
@@ -203,50 +192,18 @@ def gemm_unsummed(lhs: torch.Tensor, rhs, group_sizes: torch.Tensor) -> Unsummed
     return Unsummed(part)
 
 
-ROWS_PROJ_MAX = 8  # rows that the launches below take
-
-
-def rows_proj_norm(x: Unsummed, scale: torch.Tensor, eps: float, rhs, gate: torch.Tensor | None = None):
-    """``rmsnorm_proj`` of an ``Unsummed`` projection with its residual and the projection ``rhs`` behind it in one launch
-    (lyra_rows_proj_norm), for a few rows.  Returns (the new projection's slices, still without the rows' factors, and the
-    completed rows x), or None where the launch does not exist.  ``gate`` [C, heads] float32: the output-gate projection."""
-    splits, M, C = x.partials.shape
-    rv, rs, bk, bn, rd, (G, K, N) = _rhs_args(rhs)
-    if M > ROWS_PROJ_MAX or G != 1 or K != C or N % 8 or (isinstance(rhs, SpanMajor) and rhs.layout != 1) or x.factor is not None:
-        return None
-    n_sq = _lib.rows_proj_sums(M, K, N, bk)
-    if n_sq <= 0:
-        return None
-    assert x.residual is not None and x.residual.dtype == torch.bfloat16 and x.residual.is_contiguous()
-    assert x.bias is None or (x.bias.dtype == torch.float32 and x.bias.is_contiguous() and x.bias.numel() == C)
-    dev = x.partials.device
-    out_splits, heads = _lib.gemm_splits(M, K, N, bk), 0 if gate is None else gate.shape[1]
-    part = torch.empty((out_splits, M, N), dtype=torch.float32, device=dev)
-    sq = torch.empty((n_sq, M), dtype=torch.float32, device=dev)
-    gp = torch.empty((out_splits, M, heads), dtype=torch.float32, device=dev) if heads else None
-    x_out = torch.empty_like(x.residual)
-    rc = _L.lyra_rows_proj_norm(x.partials.data_ptr(), splits, _ptr(x.bias), x.residual.data_ptr(), float(x.scale), _f32(scale).data_ptr(),
-                                x_out.data_ptr(), sq.data_ptr(), _ptr(None if gate is None else _f32(_transposed(gate))), heads, _ptr(gp),
-                                rv.data_ptr(), _ptr(rs), bk, bn, part.data_ptr(), part.numel() * 4, M, K, N, rd, _stream(dev))
-    if rc == _lib.E_UNSUPPORTED:
-        return None
-    _lib.check(rc, "lyra_rows_proj_norm")
-    return Unsummed(part, factor=RowFactor(sq, C, eps, gp)), x_out
-
-
 def rows_proj_swiglu(x: Unsummed, rhs, beta: float, limit: float, bias: torch.Tensor | None = None) -> Unsummed | None:
-    """SwiGLU of the up projection that ``rows_proj_norm`` left, and the down projection ``rhs`` behind it, in one launch
-    (lyra_rows_proj_swiglu).  ``bias`` [2K] float32 of the up projection.  None where the launch does not exist."""
+    """SwiGLU of an up projection left in slices, and the down projection ``rhs`` behind it, in one launch
+    (lyra_rows_proj_swiglu), for a few rows.  ``bias`` [2K] float32 of the up projection.  None where the launch does not exist."""
     splits, M, width = x.partials.shape
     rv, rs, bk, bn, rd, (G, K, N) = _rhs_args(rhs)
-    if not rows_proj_swiglu_exists(M, rhs) or width != 2 * K or x.factor is None:
+    if not rows_proj_swiglu_exists(M, rhs) or width != 2 * K:
         return None
     assert bias is None or (bias.dtype == torch.float32 and bias.is_contiguous() and bias.numel() == width)
-    dev, f = x.partials.device, x.factor
+    dev = x.partials.device
     part = torch.empty((_lib.gemm_splits(M, K, N, bk), M, N), dtype=torch.float32, device=dev)
-    rc = _L.lyra_rows_proj_swiglu(x.partials.data_ptr(), splits, _ptr(bias), f.sq.data_ptr(), f.sq.shape[0], f.width, float(f.eps),
-                                  float(beta), float(limit), rv.data_ptr(), _ptr(rs), bk, bn, part.data_ptr(), part.numel() * 4, M, K, N,
-                                  rd, _stream(dev))
+    rc = _L.lyra_rows_proj_swiglu(x.partials.data_ptr(), splits, _ptr(bias), float(beta), float(limit), rv.data_ptr(), _ptr(rs), bk, bn,
+                                  part.data_ptr(), part.numel() * 4, M, K, N, rd, _stream(dev))
     if rc == _lib.E_UNSUPPORTED:
         return None
     _lib.check(rc, "lyra_rows_proj_swiglu")
@@ -255,8 +212,7 @@ def rows_proj_swiglu(x: Unsummed, rhs, beta: float, limit: float, bias: torch.Te
 
 def rows_proj_swiglu_exists(M: int, rhs) -> bool:
     _, _, bk, _, _, (G, K, N) = _rhs_args(rhs)
-    return (M <= ROWS_PROJ_MAX and G == 1 and N % 8 == 0 and not (isinstance(rhs, SpanMajor) and rhs.layout != 1)
-            and _lib.rows_proj_sums(M, K, N, bk) > 0)
+    return G == 1 and N % 8 == 0 and not (isinstance(rhs, SpanMajor) and rhs.layout != 1) and _lib.rows_proj_swiglu_exists(M, K, N, bk) == 1
 
 
 def rmsnorm_proj(x, scale: torch.Tensor, eps: float, proj: torch.Tensor | None = None,
@@ -289,7 +245,7 @@ def rmsnorm_proj(x, scale: torch.Tensor, eps: float, proj: torch.Tensor | None =
     if isinstance(x, Unsummed):
         u = x
         splits, B, C = u.partials.shape
-        assert u.residual is not None and u.residual.dtype == torch.bfloat16 and u.residual.is_contiguous() and u.factor is None
+        assert u.residual is not None and u.residual.dtype == torch.bfloat16 and u.residual.is_contiguous()
         x_out = torch.empty_like(u.residual)
         h_obj, h, mode = _norm_out(u.residual, tiled, gate)
         y, n = None, 0
@@ -358,7 +314,7 @@ def qkv_post(qkv, qnorm, knorm, cos_t: torch.Tensor, sin_t: torch.Tensor, pos: t
     N, K, H = n_heads, n_kv_heads, head_dim
     unsummed = isinstance(qkv, Unsummed)
     if unsummed:  # the projection arrives as K slices; they are summed while reading
-        assert qkv.factor is None and qkv.bias is None, "a projection with a bias comes summed (gemm with bias_after_cast) to qkv_post"
+        assert qkv.bias is None, "a projection with a bias comes summed (gemm with bias_after_cast) to qkv_post"
         part = qkv.partials
         splits, B, width = part.shape
         assert width == (N + 2 * K) * H and qkv.residual is None
@@ -430,20 +386,6 @@ def attention_qkv(qkv, qnorm, knorm, cos_t: torch.Tensor, sin_t: torch.Tensor, p
     qkv_bias = qkv.bias if unsummed else None
     if qkv_bias is not None:
         assert qkv_bias.dtype == torch.float32 and qkv_bias.is_contiguous() and qkv_bias.numel() == (N + 2 * K) * H
-    if unsummed and qkv.factor is not None:  # (its own gate slices; the caller passes no gate)
-        f = qkv.factor
-        assert gate is None and f.sq.shape[1] == B and (f.gate is None or tuple(f.gate.shape[1:]) == (B, N))
-        rc = _L.lyra_decode_attention_rows(part.data_ptr(), splits, _ptr(qkv_bias), f.sq.data_ptr(), f.sq.shape[0], f.width, float(f.eps),
-                                           _ptr(f.gate), 0 if f.gate is None else f.gate.shape[0], _ptr(qnorm), _ptr(knorm),
-                                           _f32(cos_t).data_ptr(), _f32(sin_t).data_ptr(), cos_t.shape[0], float(eps), kq.data_ptr(),
-                                           vq.data_ptr(), _ptr(ks), _ptr(vs), sinks.data_ptr(), pos.data_ptr(),
-                                           0 if pos.numel() == 1 else 1, out.data_ptr(), ws.data_ptr(), ws.numel(), B, N, K, S, H,
-                                           float(sm_scale), int(sliding_window), _lib.fp8_code(kq.dtype) if fp8 else _lib.DTYPE_BF16,
-                                           _lib.DTYPE_F32 if out_dtype == torch.float32 else _lib.DTYPE_BF16, stream)
-        if rc == _lib.E_UNSUPPORTED:
-            return None
-        _lib.check(rc, "lyra_decode_attention_rows")
-        return out
     rc = _L.lyra_decode_attention_qkv_bias(None if unsummed else qkv.data_ptr(), part.data_ptr() if unsummed else None,
                                       splits if unsummed else 0, _ptr(qkv_bias), _ptr(qnorm), _ptr(knorm), _f32(cos_t).data_ptr(),
                                       _f32(sin_t).data_ptr(), cos_t.shape[0], float(eps), kq.data_ptr(), vq.data_ptr(), _ptr(ks),

@@ -457,7 +457,7 @@ _LOGIT_TILE_MAX = os.environ.get("LYRA_NO_LOGIT_TILE_MAX") is None  # tuning ove
 # a K-split workgroup then reads one contiguous run per wavefront instead of pieces a weight row apart (0.2-0.3 us of each
 # 5-10 us launch).  Expert weights keep the reference's array unless their rows straddle cache lines (the copy costs the
 # expert kernel more than it gains there).  LYRA_SPAN_MAJOR_DENSE=0: the alignment rule for every array.
-_ROWS_PROJ = os.environ.get("LYRA_NO_ROWS_PROJ") is None  # tuning override: norm and SwiGLU in launches of their own at every batch
+_ROWS_PROJ = os.environ.get("LYRA_NO_ROWS_PROJ") is None  # tuning override: SwiGLU in a launch of its own at every batch
 _DENSE_SPAN_MAJOR = os.environ.get("LYRA_SPAN_MAJOR_DENSE", "1") != "0"
 
 
@@ -482,17 +482,6 @@ def _bf16_bias(bias, groups: int = 1):
     return kept[1]
 
 
-def _norm_in_projection(x) -> bool:
-    """Whether the norm of ``x`` runs inside the launch of the projection behind it: slices of a few rows (beyond that the sums,
-    which every column span repeats, cost more than the norm's launch), of 1024 columns or more.  The operand there is bf16(x *
-    scale) with the row's factor applied to the float32 product, so it skips one of the reference's roundings to bf16: closer
-    to the exact product, but where a router's two best experts are within that rounding of each other a token may go to the
-    other one.  Narrower models are held to the reference's own roundings, launch by launch."""
-    from lyra_amd.kernels import decode_fused as F
-
-    return _ROWS_PROJ and isinstance(x, F.Unsummed) and x.partials.shape[1] <= F.ROWS_PROJ_MAX and x.partials.shape[2] >= 1024
-
-
 def attention_apply_fused(x, w: AttentionWeights, idx: int, pos, cos_t, sin_t, cache: LayerCache, cfg: ModelConfig):
     """attention_apply as 4 launches: norm(+gate) | qkv matmul | QK norm + RoPE + cache append + attention | output matmul.
     ``x`` is the residual stream or an ``Unsummed`` projection that still has to be added to it; the return value likewise
@@ -506,16 +495,6 @@ def attention_apply_fused(x, w: AttentionWeights, idx: int, pos, cos_t, sin_t, c
     front_step = w.xsa_alpha is None and not _SEPARATE_QKV_POST
     w_qkv, w_out = F.span_major(w.qkv, always=_DENSE_SPAN_MAJOR), F.span_major(w.out, always=_DENSE_SPAN_MAJOR)
     t = None
-    if front_step and pos.numel() == 1 and _norm_in_projection(x):
-        # a few rows: the norm inside the projection's launch
-        rows = F.rows_proj_norm(x, w.norm_scale, cfg.norm_eps, w_qkv, gate=w.sdpa_gate)
-        if rows is not None:
-            qkv, x_done = rows
-            qkv.bias = None if w.qkv_bias is None else _bf16_bias(w.qkv_bias).reshape(-1)
-            t = F.attention_qkv(qkv, w.qnorm_scale, w.knorm_scale, cos_t, sin_t, pos, cache.k, cache.v, w.sinks, H**-0.5,
-                                sliding_window, N, K, H, cfg.norm_eps)
-            if t is not None:
-                return _attention_out(t, w_out, x_done, w, cfg), cache
     if isinstance(x, TokenRows):  # first layer of a step: the embedding rows are gathered by the norm kernel
         h, gate, x = F.embed_rmsnorm_proj(x.table, x.tokens, w.norm_scale, cfg.norm_eps, w.sdpa_gate, None, gate=True, tiled=tiled)
     elif isinstance(x, (F.Unsummed, F.Uncombined)):
@@ -599,20 +578,18 @@ def dense_mlp_apply_fused(x, w: DenseMLPWeights, cfg: ModelConfig):
 
     tiled = _TILED_ACTIVATIONS and cfg.n_embd % 32 == 0 and cfg.dense_hidden % 32 == 0
     w_up, w_down = F.span_major(w.mlp_up, always=_DENSE_SPAN_MAJOR), F.span_major(w.mlp_down, always=_DENSE_SPAN_MAJOR)
-    if _norm_in_projection(x) and F.rows_proj_swiglu_exists(x.partials.shape[1], w_down):
-        # a few rows: norm and SwiGLU inside the launches of the projections behind them
-        rows = F.rows_proj_norm(x, w.norm_scale, cfg.norm_eps, w_up)
-        if rows is not None:
-            down = F.rows_proj_swiglu(rows[0], w_down, cfg.swiglu_beta, cfg.swiglu_limit, bias=_flat(_bf16_bias(w.mlp_up_bias)))
-            if down is not None:
-                down.residual, down.scale = rows[1], cfg.dense_residual_scale
-                down.bias = _flat(_bf16_bias(w.mlp_down_bias))
-                return down
     if isinstance(x, (F.Unsummed, F.Uncombined)):
         t, _, x = F.rmsnorm_proj(x, w.norm_scale, cfg.norm_eps, tiled=tiled)
     else:
         t, _ = F.rmsnorm_proj(x, w.norm_scale, cfg.norm_eps, tiled=tiled)
     one = _one_group(x.shape[0], x.device)
+    if _ROWS_PROJ and F.rows_proj_swiglu_exists(x.shape[0], w_down):  # a few rows: SwiGLU inside the down projection's launch
+        up = F.gemm_unsummed(t, w_up, one)
+        down = None if up is None else F.rows_proj_swiglu(up, w_down, cfg.swiglu_beta, cfg.swiglu_limit, bias=_flat(_bf16_bias(w.mlp_up_bias)))
+        if down is not None:
+            down.residual, down.scale = x, cfg.dense_residual_scale
+            down.bias = _flat(_bf16_bias(w.mlp_down_bias))
+            return down
     t = F.gemm(t, w_up, one, fused_swiglu=True, swiglu_beta=cfg.swiglu_beta, swiglu_limit=cfg.swiglu_limit,
                bias=_bf16_bias(w.mlp_up_bias), out_tiled=tiled)
     # :628-636: projection, + bias, * residual scale, + residual, each a bf16 result - left to the norm that sums the slices

@@ -25,7 +25,7 @@ def _cfg(name):
         "small-e5m2": replace(apply_inference_overrides(small, fp8=True, fp8_attn=True), gemm_dtype=torch.float8_e5m2),
         "biases": gpt,
         "dense-only": replace(small, mlp_map=("dense",) * 3, use_sdpa_output_gate=False),
-        "wide-gate": replace(small, n_attn_heads=32, head_dim=64),  # more gates than the launches of a few rows take
+        "wide-gate": replace(small, n_attn_heads=32, head_dim=64),
     }[name]
 
 
