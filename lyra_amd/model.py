@@ -649,15 +649,19 @@ def _layers_native(tokens: torch.Tensor, model: ModelWeights, cache: ModelCache,
     if pos.device != dev or tokens.device != dev or model.emb.dtype != torch.bfloat16 or not model.emb.is_contiguous():
         return None
 
+    keep = []  # (converted copies are kept per weight tensor, one at a time: those of this step stay alive until it is launched)
+
     def f32(t, n=None):
         if t is None:
             return 0
         _need(t.dtype == torch.float32 and t.is_contiguous() and t.device == dev and (n is None or t.numel() == n))
+        keep.append(t)
         return t.data_ptr()
 
     def matrix(rhs, groups, k, n):
         data, scale, bk, bn, dtype, dims = F._rhs_args(rhs)
         _need(dims == (groups, k, n) and data.device == dev)
+        keep.extend((data, scale))
         return data.data_ptr(), 0 if scale is None else scale.data_ptr(), bk, bn, dtype, 0
 
     width, heads, E, k_routed = (N + 2 * K) * H, N * H, cfg.n_experts, cfg.n_active_routed_experts

@@ -79,6 +79,21 @@ def test_one_call_equals_the_launches_one_by_one(name, B, monkeypatch):
         assert torch.equal(a, b)
 
 
+def test_layers_that_share_a_parameters_memory():
+    """One copy of a converted parameter is kept per address: the copies that two layers make of the same memory through tensors of
+    their own have to outlive the results allocated after them."""
+    import lyra_amd.model as M
+
+    cfg, dev = _cfg("small-bf16"), U.dev()
+    model = M.init_weights(cfg, dev, seed=4)
+    first, last = model.layers[0].attn, model.layers[2].attn
+    last.sdpa_gate = first.sdpa_gate.view(first.sdpa_gate.shape)
+    tokens = torch.arange(8, dtype=torch.int32, device=dev)
+    want = _logits(model, M.init_cache(cfg, 8, 64, dev), tokens, cfg, False)
+    for _ in range(3):
+        assert torch.equal(_logits(model, M.init_cache(cfg, 8, 64, dev), tokens, cfg, True), want)
+
+
 def test_steps_that_the_call_does_not_cover_run_from_python(monkeypatch):
     import lyra_amd.model as M
 
