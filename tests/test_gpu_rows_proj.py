@@ -35,8 +35,7 @@ def test_swiglu_inside_the_down_projection(M, K, N, kind, splits, with_bias, pac
     sums = 3 * rand(splits, M, 2 * K)
     bias = rand(2 * K).to(torch.bfloat16).float() if with_bias else None
     got = F.rows_proj_swiglu(F.Unsummed(sums), F.pack_weights(w) if packed else w, 1.702, 7.0, bias=bias)
-    # the operand: slices added in slice order, bias, SwiGLU, one rounding to bf16 - formed here with the up projection's own
-    # finish step, which a product with the identity of the summed slices reaches
+    # the operand: slices added in slice order, bias, SwiGLU, one rounding to bf16
     total = torch.zeros(M, 2 * K, device=dev)
     for part in sums:
         total = total + part
