@@ -512,7 +512,7 @@ __device__ __forceinline__ void append_staged(const Slab& sl, const uint8_t* sta
 }
 
 // QKV: the launch also does the step in front of the attention (lyra_decode_attention_qkv).
-template <int H, int FP8, bool VEC4, int WAVES, bool EARLY, int DEPTH, bool QKV = false>
+template <int H, int FP8, bool VEC4, int WAVES, bool EARLY, int DEPTH, bool QKV = false, bool WHOLE = false>
 __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(DEPTH > 1 ? 2 : (WAVES >= 8 ? 4 : 3))))
 void decode_attention_kernel(AttnParams p) {
     static_assert(!QKV || DEPTH == 1, "the fused front step knows one register set per wavefront");
@@ -527,7 +527,8 @@ void decode_attention_kernel(AttnParams p) {
     int c_idx = blockIdx.x, n_chunks = p.n_chunks, chunk = p.chunk;
     int kh = blockIdx.y, b = blockIdx.z;
     const int G = p.G;
-    if (EARLY && __builtin_expect(p.whole > 0, 0)) {  // (out of the way: falling through costs the others nothing)
+    // (an instantiation of its own: as a branch on p.whole it cost the even launches 0.15 us - 64 x 4 x 4096 FP8 43.7 -> 43.8)
+    if constexpr (WHOLE) {
         int pair = (int)blockIdx.x;
         if (pair < p.whole) {
             c_idx = 0;
@@ -811,7 +812,7 @@ void decode_attention_kernel(AttnParams p) {
             if (p.xsa_v) smem[p.xsa_lds + idx] = gated(p, o / den, sm_gate[g]);
             else store_out(p, ((size_t)b * p.N + n) * H + col, o / den, sm_gate[g]);
         } else {
-            const size_t item = (size_t)(b * p.K + kh - p.whole) * n_chunks + c_idx;
+            const size_t item = (size_t)(b * p.K + kh - (WHOLE ? p.whole : 0)) * n_chunks + c_idx;
             store_agent(p.part_o + (item * G + g) * H + col, o);
             if (col == 0) {
                 store_agent(p.part_ml + (item * G + g) * 2, mm);
@@ -838,7 +839,7 @@ void decode_attention_kernel(AttnParams p) {
     if (!sm_last) return;
     // weights of the chunks: every thread fetches one (max, sum) pair, then LDS holds exp2(m_c - m*) and the
     // denominator per head; the output columns are then gathered with all loads of a thread in flight at once
-    const size_t item0 = (size_t)(b * p.K + kh - p.whole) * n_chunks;
+    const size_t item0 = (size_t)(b * p.K + kh - (WHOLE ? p.whole : 0)) * n_chunks;
     float* sm_w = smem;                 // [n_valid][G] weight of chunk c for head g
     float* sm_den = smem + 1024;        // [G]
     float* sm_cm = smem + 1024 + 16;    // [n_valid][G] chunk maxima
@@ -1389,13 +1390,15 @@ static int run_attention(const void* q, const void* k, const void* v, const floa
     }
 #define LYRA_LAUNCH_ATTN_W(HH, F, V, W)                                                                        \
     do {                                                                                                      \
-        if (sliding_window == 0) hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, W, true, 1>), grid, block, lds, st, p); \
+        if (pl.whole > 0) hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, W, true, 1, false, true>), grid, block, lds, st, p); \
+        else if (sliding_window == 0) hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, W, true, 1>), grid, block, lds, st, p); \
         else hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, W, false, 1>), grid, block, lds, st, p);      \
     } while (0)
 #define LYRA_LAUNCH_ATTN(HH, F, V)                              \
     do {                                                        \
         if (front) {                                            \
-            if (sliding_window == 0) hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, 4, true, 1, true>), grid, block, lds, st, p); \
+            if (pl.whole > 0) hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, 4, true, 1, true, true>), grid, block, lds, st, p); \
+            else if (sliding_window == 0) hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, 4, true, 1, true>), grid, block, lds, st, p); \
             else hipLaunchKernelGGL((decode_attention_kernel<HH, F, V, 4, false, 1, true>), grid, block, lds, st, p); \
         } else if (pl.waves == 4) LYRA_LAUNCH_ATTN_W(HH, F, V, 4); \
         else if (pl.waves == 8) LYRA_LAUNCH_ATTN_W(HH, F, V, 8); \
