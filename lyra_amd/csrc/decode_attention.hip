@@ -76,17 +76,13 @@ constexpr int kMergeStageFloats = 3 * 1024 + 16;  // LDS floats used when the la
 // Visible key range of one batch row; bit-exact restatement of the mask
 // (key <= pos) & (key > pos - sw)   (decode_attention.py:285-286, :338-340).
 struct Range {
-    int lo, hi, start;  // [lo, hi] visible; start: first key of the first tile
+    int lo, hi, start;  // [lo, hi] visible, start = lo rounded down to a tile
 };
 __device__ __forceinline__ Range visible_range(int pos, int sw, int S) {
     Range r;
     r.hi = min(pos, S - 1);
     r.lo = sw > 0 ? max(0, pos - sw + 1) : 0;
-    // Tiles start at the first visible key, wherever that is: from a multiple of 32 a window of 128 keys was 5 tiles for 4
-    // wavefronts at 31 of 32 positions (1 x 4 x 1000 bf16 5.8 -> 4.8 us, 64 x 4 x 4001 FP8 6.3 -> 5.3, 128 x 8 x 1501 17.6 -> 13.5).
-    // The 16-byte loads of scales then start at any multiple of 4 bytes, which buffer loads take, each dword checked by itself
-    // against the end of the slab.
-    r.start = r.lo;
+    r.start = r.lo & ~(kTile - 1);
     return r;
 }
 
@@ -1126,7 +1122,7 @@ static void cut_chunks(AttnPlan& pl, int span, long n) {
 static AttnPlan plan_attention(int B, int K, int S, int sliding_window) {
     static const long target_env = env_long("LYRA_ATTN_TARGET_WGS");  // tuning overrides, read once
     static const long waves_env = env_long("LYRA_ATTN_WAVES");
-    int span = S;  // longest visible range (a window: and as many keys as tiles that start at multiples of 32 would add)
+    int span = S;  // longest visible range, measured from its tile-aligned start
     if (sliding_window > 0) span = std::min(S, sliding_window + kTile - 1);
     const long pairs = (long)B * K;
     AttnPlan pl;

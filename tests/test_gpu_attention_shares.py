@@ -89,3 +89,26 @@ def test_windows_at_every_offset(S, sw, fp8):
     for i in (0, 5, 34, 35):  # (one position for the batch: the same launch as a step's)
         one = decode_attention(q, k, v, sinks, H**-0.5, sw, torch.tensor(int(first[i]), dtype=torch.int32, device=U.dev()), implementation="pallas")
         assert torch.equal(one[i], got[i])
+
+
+# a window's sums are those of a global layer over the keys from the last multiple of 32 before it, bit for bit: the order of its
+# sums does not move with the position inside a tile
+@pytest.mark.parametrize("pos", [127, 128, 140, 158, 159, 160, 299])
+def test_window_adds_in_the_order_of_tiles_at_multiples_of_32(pos):
+    from lyra_amd.kernels.decode_attention import decode_attention
+
+    print(f"attention window tiles pos={pos}", file=sys.stderr, flush=True)
+    B, N, K, S, H, sw = 64, 8, 4, 300, 64, 128
+    gen = torch.Generator(device=U.dev()).manual_seed(pos)
+    q, k, v = (torch.randn(*s, device=U.dev(), generator=gen).to(torch.bfloat16) for s in ((B, N, 1, H), (B, K, S, H), (B, K, S, H)))
+    sinks = torch.randn(N, device=U.dev(), generator=gen)
+    q[..., 0], k[..., 0] = 1.0, 0.0
+    at = lambda p: torch.tensor(p, dtype=torch.int32, device=U.dev())  # noqa: E731
+    got = decode_attention(q, k, v, sinks, H**-0.5, sw, at(pos), implementation="pallas")
+    lo = max(0, pos - sw + 1)
+    a = lo // 32 * 32
+    kk, vv = k[:, :, a : pos + 1].contiguous(), v[:, :, a : pos + 1].contiguous()
+    kk[:, :, : lo - a] = 0.0
+    kk[:, :, : lo - a, 0] = -30000.0  # (exp2 of it is exactly zero: these keys add nothing, in their place)
+    want = decode_attention(q, kk, vv, sinks, H**-0.5, 0, at(pos - a), implementation="pallas")
+    assert torch.equal(got, want)
