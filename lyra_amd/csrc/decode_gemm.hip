@@ -2297,15 +2297,6 @@ static GemmPlan plan_gemm(int M, int G, int K, int N, int bk, int fused_swiglu, 
         int kpart = (int)((K + want - 1) / want);
         // up to 512 rows per slice everything is requested at once; longer slices (larger matrices) refill 4 register sets
         kpart = std::min(2048, (kpart + unit - 1) / unit * unit);
-        // More than one round of workgroups (a compute unit holds one) for the sake of that limit: slices as long as one round
-        // needs instead, where the last row block is not a light one that fills the gaps anyway (us with the sum, FP8, 2048 rows
-        // against one round: 4096 x 12288 at 128 rows 52.5 / 44.1, at 96 46.3 / 46.1, at 65 41.6 / 45.7; 6144 x 4096 at 192 and 256
-        // rows 49.0 / 34.1 and 50.8 / 34.5, at 129 30.2 / 34.5; 4096 x 6144 at 256 51.5 / 42.0; 2880 x 5120 bf16 at 256 45.2 / 37.5).
-        const long tiles = (long)pl.spans * pl.row_par;
-        if (tiles <= 256 && tiles * ((K + kpart - 1) / kpart) > 256 && (M - 1) % 64 >= 32 && pl.row_block == 64) {
-            const int longer = ((K + (int)want - 1) / (int)want + unit - 1) / unit * unit;
-            if (longer <= 4096 && tiles * ((K + longer - 1) / longer) <= 256 && !(bk > 0 && bk < K && longer % bk)) kpart = longer;
-        }
         if (unit > 512 || (bk > 0 && bk < K && kpart % bk)) pl.split_k = false;  // scale blocks that do not tile a slice
         pl.kpart = kpart;
         pl.ksplit = (K + kpart - 1) / kpart;
