@@ -2684,11 +2684,19 @@ extern "C" int lyra_gemm_pack(const void* rhs, void* packed, int G, int K, int N
 extern "C" size_t lyra_decode_gemm_workspace(int M, int G, int K, int N, int fused_swiglu) {
     if (M <= 0 || G <= 0 || K <= 0 || N <= 0) return 0;
     // The scale block is not known here and decides both which kernel runs (a block that does not tile a K slice sends a
-    // small projection to the general kernel) and how many K slices it writes; a coarser block only ever lowers the slice
-    // count of either kernel, so the larger of the two plans without a block covers every block.
-    const lyra::GemmPlan with_split = lyra::plan_gemm(M, G, K, N, 0, fused_swiglu, true);
-    const lyra::GemmPlan general = lyra::plan_gemm(M, G, K, N, 0, fused_swiglu, false);
-    return lyra::kGemmCounterBytes + std::max(lyra::gemm_partial_bytes(with_split, M, N), lyra::gemm_partial_bytes(general, M, N));
+    // small projection to the general kernel) and how many K slices it writes, more of them too: 384 rows rounded up to whole
+    // blocks stay 384 with blocks of 384, and become 512 without (64 x 6144 x 2048: 16 slices and 12).  So every block that
+    // divides K is asked for.
+    size_t most = 0;
+    auto cover = [&](int bk) { most = std::max(most, lyra::gemm_partial_bytes(lyra::plan_gemm(M, G, K, N, bk, fused_swiglu), M, N)); };
+    cover(0);
+    for (int d = 1; d <= K / d; ++d)
+        if (K % d == 0) {
+            cover(d);
+            cover(K / d);
+        }
+    most = std::max(most, lyra::gemm_partial_bytes(lyra::plan_gemm(M, G, K, N, 0, fused_swiglu, false), M, N));
+    return lyra::kGemmCounterBytes + most;
 }
 
 extern "C" size_t lyra_decode_gemm_workspace_for(int M, int G, int K, int N, int bk, int fused_swiglu) {

@@ -112,3 +112,20 @@ def test_matmul_workspace_covers_the_launched_plan_for_every_scale_block():
     for (M, K, N, bk, slices) in ((16, 8192, 8192, 1024, 8), (128, 2048, 32768, 1024, 2), (16, 12288, 8192, 96, 32)):
         assert L.lyra_decode_gemm_splits(M, K, N, bk) == 0
         assert L.lyra_decode_gemm_workspace_for(M, 1, K, N, bk, 0) == 65536 + slices * M * N * 4
+
+
+def test_matmul_workspace_covers_scale_blocks_that_are_no_power_of_two():
+    from lyra_amd import _lib
+
+    L = _lib.lib
+    more = 0
+    for M in (1, 17, 64, 128, 300):
+        for K in (1536, 2720, 2880, 3456, 5760, 6144, 18432, 41472):
+            for N in (200, 1024, 2048, 6144):
+                for swiglu in (0, 1) if N % 16 == 0 else (0,):
+                    cover = L.lyra_decode_gemm_workspace(M, 1, K, N, swiglu)
+                    for bk in (d for d in range(1, K + 1) if K % d == 0):
+                        need = L.lyra_decode_gemm_workspace_for(M, 1, K, N, bk, swiglu)
+                        assert need <= cover, (M, K, N, swiglu, bk, need, cover)
+                        more += bk == 384 and need > L.lyra_decode_gemm_workspace_for(M, 1, K, N, 0, swiglu)
+    assert more > 0  # blocks of 384 rows do need more than the plan without a block
