@@ -1144,6 +1144,12 @@ static AttnPlan plan_attention(int B, int K, int S, int sliding_window) {
 // (2-3 us), so pairs are only cut where that saves the streaming of 128 KB or more (64 KB where only part of the device is
 // busy, which streams faster per unit): 33 x 8 x 1000 FP8 21.9 -> 18.0 us, 16 x 8 x 1000 in 2 chunks 12.5, whole 13.9; but
 // 45 x 8 x 300 10.6 whole, 13.4 cut.
+// The count follows from the cache's length and holds at every position in it: FP8 at S / 4, S / 2, 3 S / 4 and S, cut finer and as
+// here, 33 x 4 x 4096 24.0 / 38.8 / 40.1 / 41.7 and 14.6 / 22.0 / 30.7 / 38.5; 17 x 4 x 2000 15.0 / 15.7 / 16.2 / 16.9 and 11.1 / 13.4 /
+// 13.8 / 14.4; 30 x 4 x 2000 11.7 / 17.0 / 20.5 / 21.7 and 11.7 / 16.8 / 16.6 / 17.0 (an empty chunk still takes a turn on a unit).
+// Only the first quarter of a long cache is slower in a few (12 x 4 x 4096 13.1 / 17.8 / 20.9 / 21.2 and 14.3 / 15.1 / 15.9 / 16.3).
+// Fewer than 4 rows keep the finer cut, which differs for them only in caches of a few hundred keys (3 x 4 x 300 8.3 us, whole 6.6):
+// another order of the same sums sends a row in 70 to another expert further on, and there one row is the result.
 // Rows with a position each leave more than 256 pairs whole (the whole-row kernel takes those).  key_bytes: of one key and its
 // value.  Its parts may need more room than those of the plan above; a caller's workspace is held to that plan, and gets it
 // when it is too small for this one.
@@ -1151,7 +1157,7 @@ static AttnPlan plan_shares(int B, int K, int S, int key_bytes, int sliding_wind
     AttnPlan pl = plan_attention(B, K, S, sliding_window);
     static const bool off = env_long("LYRA_ATTN_TARGET_WGS") > 0;  // (the override states the number of chunks)
     const long pairs = (long)B * K, left = pairs % 256;
-    if (off || sliding_window > 0 || left == 0 || pairs > kMaxSplitPairs || (pairs > 256 && !one_position)) return pl;
+    if (off || B < 4 || sliding_window > 0 || left == 0 || pairs > kMaxSplitPairs || (pairs > 256 && !one_position)) return pl;
     long want = std::min(256 / left, ((long)S + pl.waves * kTile - 1) / (pl.waves * kTile));
     if ((double)S * key_bytes * (want - 1) < (pairs > 256 ? 131072.0 : 65536.0) * want) want = 1;
     cut_chunks(pl, S, want);

@@ -112,3 +112,24 @@ def test_window_adds_in_the_order_of_tiles_at_multiples_of_32(pos):
     kk[:, :, : lo - a, 0] = -30000.0  # (exp2 of it is exactly zero: these keys add nothing, in their place)
     want = decode_attention(q, kk, vv, sinks, H**-0.5, 0, at(pos - a), implementation="pallas")
     assert torch.equal(got, want)
+
+
+# up to 3 rows a short cache is cut into chunks whatever its format (from 4 rows on, one of FP8 this short stays whole): codes
+# with unit scales and the same numbers in bf16 then give the same bits.  (Small whole numbers in q and k: exact in any order.)
+@pytest.mark.parametrize("B,K,S", [(1, 4, 300), (2, 4, 300), (3, 4, 300), (3, 8, 300), (1, 1, 330)])
+def test_few_rows_keep_their_chunks(B, K, S):
+    from lyra_amd.kernels.decode_attention import decode_attention
+    from lyra_amd.nn.quant import QArray
+
+    print(f"attention few rows B={B} K={K} S={S}", file=sys.stderr, flush=True)
+    H, gen = 128, torch.Generator(device=U.dev()).manual_seed(B + K)
+    q = torch.randint(-3, 4, (B, 4 * K, 1, H), device=U.dev(), generator=gen).to(torch.bfloat16)
+    k = torch.randint(-3, 4, (B, K, S, H), device=U.dev(), generator=gen).float().to(torch.float8_e4m3fn)
+    v = torch.randn(B, K, S, H, device=U.dev(), generator=gen).to(torch.float8_e4m3fn)
+    one = torch.ones(B, K, S, 1, device=U.dev())
+    sinks = torch.randn(4 * K, device=U.dev(), generator=gen)
+    for pos in (S - 1, S // 2):
+        at = torch.tensor(pos, dtype=torch.int32, device=U.dev())
+        codes = decode_attention(q, QArray(k, one, (1, H)), QArray(v, one, (1, H)), sinks, H**-0.5, 0, at, implementation="pallas")
+        plain = decode_attention(q, k.to(torch.bfloat16), v.to(torch.bfloat16), sinks, H**-0.5, 0, at, implementation="pallas")
+        assert torch.equal(codes, plain)
