@@ -448,7 +448,8 @@ int lyra_sample_topk_tiles(const float* x, const float* tile_max, const float* u
  *   lyra_step_t    table [table_rows,C] bf16, tokens [B] int32; out [B,C] bf16: the normalised rows behind the last layer;
  *                  gemm_ws / attn_ws: workspaces large enough for every launch; scratch: lyra_decode_step_scratch bytes, 256-byte
  *                  aligned, for the results between the launches (contents irrelevant)
- * lyra_decode_step_scratch answers 0 for a step that lyra_decode_step refuses by its sizes.  A launch that refuses its shape ends
+ * lyra_decode_step_scratch answers 0 for a step that lyra_decode_step refuses by its sizes; scratch_bytes below its answer is refused
+ * (LYRA_E_WORKSPACE) before anything is launched.  A launch that refuses its shape ends
  * the call with that launch's code; nothing but the caches' rows at the position, out and the workspaces has been written then.
  */
 typedef struct {

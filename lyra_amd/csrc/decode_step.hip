@@ -12,13 +12,11 @@ namespace {
 // Results of a layer live in one of two halves of the caller's scratch memory; the next layer writes the other one.
 struct Carve {
     char* base = nullptr;
-    size_t used = 0, cap = 0;
-    bool over = false;
+    size_t used = 0;
     template <typename T = void>
     T* take(size_t bytes) {
         char* p = base ? base + used : nullptr;
         used += (bytes + 255) / 256 * 256;
-        if (base && used > cap) over = true;
         return (T*)p;
     }
 };
@@ -57,7 +55,6 @@ struct Step {
             return rc;
         }
         void* x = mem.take(xbytes);
-        if (mem.over) return LYRA_E_WORKSPACE;
         if (!dry) {
             if (t.kind == Stream::kTokens)
                 rc = lyra_rmsnorm_proj_embed(s.table, s.tokens, s.table_rows, x, scale, h, proj, bias, y, s.B, s.C, n, mode, s.eps, st);
@@ -75,7 +72,6 @@ struct Step {
 
     // lhs @ w as K slices (splits > 0), rows: lhs holds B rows of K
     int partials(const void* lhs, bool lhs_tiled, const lyra_matrix_t& w, int K, int N, int splits, float* out) {
-        if (mem.over) return LYRA_E_WORKSPACE;
         if (dry) return LYRA_OK;
         return lyra_decode_gemm_partials(lhs, w.data, w.scale, w.bk, w.bn, one, out, f32((size_t)splits * s.B * N), s.B, K, N,
                                          w.dtype | (lhs_tiled ? LYRA_LHS_TILED16 : 0), st);
@@ -106,7 +102,6 @@ struct Step {
     // one-group product summed by the launch itself; post: bits of lyra_decode_gemm_ex's post_scale
     int gemm(const void* lhs, bool lhs_tiled, const lyra_matrix_t& w, int K, int N, const float* bias, int post, const void* residual,
              float scale, void* out) {
-        if (mem.over) return LYRA_E_WORKSPACE;
         if (dry) return LYRA_OK;
         return lyra_decode_gemm_ex(lhs, nullptr, w.data, w.scale, w.bk, w.bn, one, bias, residual, scale, post, out, s.gemm_ws,
                                    s.gemm_ws_bytes, s.B, 1, K, N, w.dtype | (lhs_tiled ? LYRA_LHS_TILED16 : 0), LYRA_DTYPE_BF16, 0, s.beta,
@@ -151,7 +146,6 @@ struct Step {
             t.x = x; t.slices = dpart; t.splits = down; t.bias = l.down_bias; t.scale = s.dense_residual_scale;
             return rc;
         }
-        if (rc == LYRA_OK && mem.over) rc = LYRA_E_WORKSPACE;
         if (rc == LYRA_OK && !dry)
             rc = lyra_decode_gemm_ex(h, nullptr, l.up.data, l.up.scale, l.up.bk, l.up.bn, one, l.up_bias, nullptr, 1.f, 0, act, s.gemm_ws,
                                      s.gemm_ws_bytes, s.B, 1, s.C, 2 * Hd, l.up.dtype | LYRA_LHS_TILED16 | LYRA_OUT_TILED16,
@@ -172,7 +166,6 @@ struct Step {
         int32_t* dest = mem.take<int32_t>(f32(M));
         void* act = mem.take(((size_t)M + 15) / 16 * 16 * Hd * 2);
         void* rows = mem.take(bf16(M, s.C));
-        if (mem.over) return LYRA_E_WORKSPACE;
         if (!dry) {
             rc = lyra_moe_route(logits, scores, groups, row_map, dest, s.B, s.n_routed, s.n_shared, s.k_routed, st);
             if (rc != LYRA_OK) return rc;
@@ -199,7 +192,6 @@ struct Step {
         for (int i = 0; i <= s.n_layers; ++i) {
             mem.used = 0;
             mem.base = dry ? nullptr : (char*)s.scratch + (i & 1) * half;
-            mem.cap = half;
             int rc;
             if (i < s.n_layers) {
                 const lyra_layer_t& l = s.layers[i];
@@ -245,10 +237,14 @@ extern "C" int lyra_decode_step(const lyra_step_t* step, lyra_stream_t stream) {
     if (rc != LYRA_OK) return rc;
     if (!step->table || !step->tokens || !step->cos_t || !step->sin_t || !step->position || !step->final_norm || !step->out || !step->scratch)
         return LYRA_E_BADARG;
+    // all of the scratch memory is there before anything is launched (the pass that counts it takes a microsecond)
+    lyra::Step count{*step, true, {}, nullptr, nullptr};
+    size_t half = 0;
+    const int fits = count.run(half);
+    if (fits != LYRA_OK) return fits;
+    if ((uintptr_t)step->scratch % 256 || step->scratch_bytes / 2 < half) return LYRA_E_WORKSPACE;
     const int32_t* counts = (const int32_t*)lyra_row_counts();
     if (!counts) return LYRA_E_LAUNCH;
-    if ((uintptr_t)step->scratch % 256) return LYRA_E_WORKSPACE;
     lyra::Step run{*step, false, {}, counts + step->B, stream};
-    size_t half = step->scratch_bytes / 512 * 256;
     return run.run(half);
 }

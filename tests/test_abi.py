@@ -129,3 +129,22 @@ def test_matmul_workspace_covers_scale_blocks_that_are_no_power_of_two():
                         assert need <= cover, (M, K, N, swiglu, bk, need, cover)
                         more += bk == 384 and need > L.lyra_decode_gemm_workspace_for(M, 1, K, N, 0, swiglu)
     assert more > 0  # blocks of 384 rows do need more than the plan without a block
+
+
+@pytest.mark.parametrize("rows", [4, 300])  # (more than 256 rows: no projection runs split over K, norms read complete rows)
+@pytest.mark.parametrize("experts", [False, True])
+def test_decode_step_refuses_scratch_that_is_too_small_before_any_launch(rows, experts):
+    import lyra_amd.model as M
+    from lyra_amd import _lib
+
+    L, at = _lib.lib, [256]
+    layer = M._LAYER.pack(256, *([256, 0, 0, 0, 0, 0] * 2), *at * 10, 64, 0, 256, *([256, 0, 0, 0, 0, 0] * 2), 0, 0, *(at * 2 if experts else (0, 0)))
+    layers = ctypes.create_string_buffer(layer * 3, 3 * len(layer))
+    step = lambda nbytes, scratch=256: M._STEP.pack(  # noqa: E731
+        ctypes.addressof(layers), *at * 11, scratch, nbytes, 3, rows, 256, 2, 1, 64, 0, 10, 10, 384, 384, 8, 1, 2, 1e-5, 1.0, 1.0, 1.0, 1.0, 1.0)
+    need = L.lyra_decode_step_scratch(step(0))
+    assert need > 0 and need % 512 == 0
+    # (none of these addresses is ever used: without a device no launch could work either)
+    for nbytes in [*range(0, need, 256), need - 1]:
+        assert L.lyra_decode_step(step(nbytes), None) == -3, nbytes
+    assert L.lyra_decode_step(step(need, scratch=128), None) == -3
