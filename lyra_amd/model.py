@@ -645,6 +645,8 @@ def _layers_native(tokens: torch.Tensor, model: ModelWeights, cache: ModelCache,
     if (cfg.use_learned_xsa or pos.numel() != 1 or pos.dtype != torch.int32 or tokens.dtype != torch.int32 or not tokens.is_contiguous()
             or not 0 < B <= 256 or shape in _NATIVE_REFUSED):
         return None
+    # (fewer caches than layers, or a table of another width: the Python loop says so)
+    _need(len(cache.layers) >= len(model.layers) and tuple(model.emb.shape[1:]) == (C,))
     dev = model.emb.device
     if pos.device != dev or tokens.device != dev or model.emb.dtype != torch.bfloat16 or not model.emb.is_contiguous():
         return None

@@ -115,6 +115,18 @@ def test_steps_that_the_call_does_not_cover_run_from_python(monkeypatch):
     assert torch.equal(_logits(model, fresh(), tokens, cfg, True), want)
 
 
+def test_fewer_caches_than_layers_are_an_error():
+    import lyra_amd.model as M
+
+    cfg, dev = _cfg("dev"), U.dev()
+    model, tokens = M.init_weights(cfg, dev, seed=2), torch.arange(4, dtype=torch.int32, device=dev)
+    for native in (True, False):
+        cache = M.init_cache(cfg, 4, 64, dev)
+        cache.layers.pop()
+        with pytest.raises(IndexError):
+            _logits(model, cache, tokens, cfg, native)
+
+
 def test_arguments_and_scratch_are_checked_before_any_launch():
     import ctypes
 
