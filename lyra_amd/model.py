@@ -620,7 +620,7 @@ _MATRIX = "QQiiii"
 _LAYER = struct.Struct("=Q" + 2 * _MATRIX + 10 * "Q" + "iiQ" + 2 * _MATRIX + 4 * "Q")
 _STEP = struct.Struct("=14Q14i6f")
 _NATIVE_STEP = os.environ.get("LYRA_NO_NATIVE_STEP") is None  # tuning override: every launch of a step from Python
-_NATIVE_REFUSED: set = set()  # shapes that a launch refused (a plan without a kernel for them): their steps run from Python
+_NATIVE_REFUSED: set = set()  # steps that a launch refused (a plan without a kernel for them), by `_native_key`: they run from Python
 
 
 class _NotNative(Exception):
@@ -632,6 +632,17 @@ def _need(ok: bool) -> None:
         raise _NotNative
 
 
+def _native_key(B: int, model: ModelWeights, cache: ModelCache, cfg: ModelConfig) -> tuple:
+    """What a launch can refuse a step for: its sizes, and every layer's formats, scale blocks and cache length."""
+    def fmt(t):
+        return (t.dtype, t.block) if isinstance(t, QArray) else t.dtype
+
+    return (B, cfg.n_embd, cfg.n_attn_heads, cfg.n_kv_heads, cfg.head_dim, cfg.dense_hidden, cfg.expert_hidden, cfg.n_routed_experts,
+            cfg.n_active_routed_experts, cfg.n_shared_experts, cfg.mlp_map,
+            tuple((fmt(layer.attn.qkv), fmt(layer.attn.out), fmt(layer.mlp.mlp_up), fmt(layer.mlp.mlp_down), fmt(c.k), c.k.shape[2])
+                  for layer, c in zip(model.layers, cache.layers)))
+
+
 def _layers_native(tokens: torch.Tensor, model: ModelWeights, cache: ModelCache, cfg: ModelConfig, cos_t, sin_t) -> torch.Tensor | None:
     """All layers and the final norm in one call of the library (lyra_decode_step): the launches of ``attention_apply_fused``,
     ``moe_apply_fused`` and ``dense_mlp_apply_fused`` issued from native code, where one costs the host 2.5 us instead of 8-12.
@@ -640,13 +651,14 @@ def _layers_native(tokens: torch.Tensor, model: ModelWeights, cache: ModelCache,
     from lyra_amd.kernels import decode_fused as F
 
     B, C, N, K, H = tokens.shape[0], cfg.n_embd, cfg.n_attn_heads, cfg.n_kv_heads, cfg.head_dim
-    shape = (B, C, N, K, H, cfg.dense_hidden, cfg.expert_hidden, cfg.n_routed_experts, cfg.n_shared_experts, cfg.mlp_map)
     pos = cache.pos
     if (cfg.use_learned_xsa or pos.numel() != 1 or pos.dtype != torch.int32 or tokens.dtype != torch.int32 or not tokens.is_contiguous()
-            or not 0 < B <= 256 or shape in _NATIVE_REFUSED):
+            or not 0 < B <= 256):
         return None
     # (fewer caches than layers, or a table of another width: the Python loop says so)
     _need(len(cache.layers) >= len(model.layers) and tuple(model.emb.shape[1:]) == (C,))
+    if _NATIVE_REFUSED and _native_key(B, model, cache, cfg) in _NATIVE_REFUSED:
+        return None
     dev = model.emb.device
     if pos.device != dev or tokens.device != dev or model.emb.dtype != torch.bfloat16 or not model.emb.is_contiguous():
         return None
@@ -712,14 +724,16 @@ def _layers_native(tokens: torch.Tensor, model: ModelWeights, cache: ModelCache,
             cfg.swiglu_beta, cfg.swiglu_limit)
 
     nbytes = _lib.lib.lyra_decode_step_scratch(step(0, 0))
-    if nbytes == 0:
+    if nbytes == 0:  # (sizes that the call refuses)
+        if len(_NATIVE_REFUSED) < 4096:
+            _NATIVE_REFUSED.add(_native_key(B, model, cache, cfg))
         return None
     scratch = torch.empty(nbytes, dtype=torch.uint8, device=dev)  # (the allocator's, on this stream: reused when this call's launches are done)
     with _lib.on_device(dev):
         rc = _lib.lib.lyra_decode_step(step(scratch.data_ptr(), nbytes), stream)
     if rc == _lib.E_UNSUPPORTED:
         if len(_NATIVE_REFUSED) < 4096:
-            _NATIVE_REFUSED.add(shape)
+            _NATIVE_REFUSED.add(_native_key(B, model, cache, cfg))
         return None
     _lib.check(rc, "lyra_decode_step")
     return out

@@ -102,17 +102,38 @@ def test_steps_that_the_call_does_not_cover_run_from_python(monkeypatch):
     tokens = torch.arange(4, dtype=torch.int32, device=dev)
     fresh = lambda: M.init_cache(cfg, 4, 64, dev)  # noqa: E731
     want = _logits(model, fresh(), tokens, cfg, False)
-    # 64-bit token ids; a position per row; a bias that is not float32 falls back, too
+    # 64-bit token ids; a position per row
     assert torch.equal(_logits(model, fresh(), tokens.long(), cfg, True), want)
     cache = fresh()
     cache.pos = torch.zeros(4, dtype=torch.int32, device=dev)
     U.assert_close(U.to_np(_logits(model, cache, tokens, cfg, True))[:, : cfg.vocab_size], U.to_np(want)[:, : cfg.vocab_size])
-    # what a launch refuses: remembered by shape, and the step is the Python loop's
+    # what a launch refuses: remembered, and the step is the Python loop's
     monkeypatch.setattr(M, "_NATIVE_REFUSED", set())
     monkeypatch.setattr(M._lib.lib, "lyra_decode_step", lambda *a: M._lib.E_UNSUPPORTED)
     assert torch.equal(_logits(model, fresh(), tokens, cfg, True), want) and len(M._NATIVE_REFUSED) == 1
     monkeypatch.setattr(M._lib.lib, "lyra_decode_step", lambda *a: pytest.fail("asked again"))
     assert torch.equal(_logits(model, fresh(), tokens, cfg, True), want)
+
+
+@pytest.mark.parametrize("refused", ["lyra_decode_step", "lyra_decode_step_scratch"])
+def test_a_refusal_is_remembered_for_its_formats_and_cache_length_only(refused, monkeypatch):
+    import lyra_amd.model as M
+
+    dev, tokens = U.dev(), torch.arange(4, dtype=torch.int32, device=U.dev())
+    step = lambda m, cfg, S: _logits(m, M.init_cache(cfg, 4, S, dev), tokens, cfg, True)  # noqa: E731
+    bf16, block, channel = _cfg("small-bf16"), _cfg("small-serve"), _cfg("small-fp8")  # (the same widths)
+    models = [M.init_weights(cfg, dev, seed=2) for cfg in (bf16, block, channel)]
+    monkeypatch.setattr(M, "_NATIVE_REFUSED", set())
+    asked, inner = [], getattr(M._lib.lib, refused)
+    answer = {"lyra_decode_step": M._lib.E_UNSUPPORTED, "lyra_decode_step_scratch": 0}[refused]
+    monkeypatch.setattr(M._lib.lib, refused, lambda *a: asked.append(a) or (answer if len(asked) == 1 else inner(*a)))
+    step(models[1], block, 64)
+    step(models[1], block, 64)
+    assert len(asked) == 1 and len(M._NATIVE_REFUSED) == 1
+    step(models[0], bf16, 64)
+    step(models[2], channel, 64)
+    step(models[1], block, 96)
+    assert len(asked) == 4 and len(M._NATIVE_REFUSED) == 1
 
 
 def test_fewer_caches_than_layers_are_an_error():
