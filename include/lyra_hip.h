@@ -77,6 +77,9 @@ const char* lyra_strerror(int code);
  *                   zero again when it ends: zero the buffer once after allocating it (lyra_workspace_init
  *                   or any memset) and it can be reused by every later call, of any shape, on the same stream,
  *                   as long as nothing else writes to it in between.
+ *                   Launches that keep every pair whole need none (null); of these, the ones with one position
+ *                   for the batch, no window and more than 256 (row, kv head) pairs may cut some of them when they are
+ *                   given one of the full size: the same sums in another order.
  * Supported: H in {64,128}; 1 <= N/K <= 16; any B, S >= 1.
  */
 int lyra_decode_attention(const void* q, const void* k, const void* v, const float* k_scale, const float* v_scale,
@@ -157,7 +160,10 @@ int lyra_decode_attention_ranked(const void* q, const void* k, const void* v, co
 /*
  * lyra_decode_attention for callers that cannot allocate device memory or hand over a workspace (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  It has no counterpart in the reference.
- * Same arguments, same kernels and bit-identical results as lyra_decode_attention, minus the workspace: split partials
+ * Same arguments and same kernels as lyra_decode_attention, minus the workspace, and bit-identical results but for one kind
+ * of launch: one position for the batch, no window, and more than 256 (row, kv head) pairs that are no multiple of 256.
+ * lyra_decode_attention with a full workspace may cut the pairs that no whole round over the compute units takes; here
+ * every pair stays whole, as it does there without a workspace, and the same sums are added in another order.  Split partials
  * and arrival counters live in a device array of LYRA_STATIC_SCRATCH_BYTES that is part of the library's code object
  * (every GPU the library runs on holds one copy until the process ends).  The call allocates and frees nothing; the
  * first call on a device looks up the array's device address, so make that call outside a capture.  A launch that is

@@ -13,7 +13,7 @@ from tests import gpu_util as U
 pytestmark = pytest.mark.gpu
 
 
-def _call(case, B, N, K, S, H, pos, sw, static, gate=None):
+def _call(case, B, N, K, S, H, pos, sw, static, gate=None, workspace=True):
     from lyra_amd import _lib
 
     L = _lib.lib
@@ -24,13 +24,13 @@ def _call(case, B, N, K, S, H, pos, sw, static, gate=None):
     g = None if gate is None else U.t_bf16(gate)
     stream = torch.cuda.current_stream().cuda_stream
     head = (q.data_ptr(), k.qval.data_ptr(), v.qval.data_ptr(), k.scale.data_ptr(), v.scale.data_ptr(), sinks.data_ptr(),
-            p.data_ptr(), 1, g.data_ptr() if g is not None else None, out.data_ptr())
+            p.data_ptr(), p.dim(), g.data_ptr() if g is not None else None, out.data_ptr())
     tail = (B, N, K, S, H, H**-0.5, sw, _lib.DTYPE_E4M3FN, _lib.DTYPE_BF16, stream)
     if static:
         rc = L.lyra_decode_attention_static(*head, *tail)
     else:
         ws = torch.zeros(max(L.lyra_decode_attention_workspace(B, N, K, S, H, sw), 256), dtype=torch.uint8, device=dev)
-        rc = L.lyra_decode_attention(*head, ws.data_ptr(), ws.numel(), *tail)
+        rc = L.lyra_decode_attention(*head, *((ws.data_ptr(), ws.numel()) if workspace else (None, 0)), *tail)
     _lib.check(rc, "static" if static else "workspace")
     torch.cuda.synchronize()
     return out
@@ -93,3 +93,22 @@ def test_static_scratch_entry_point_at_drawn_shapes(seed):
     ref = _call(case, B, K * G, K, S, H, pos, sw, static=False)
     got = _call(case, B, K * G, K, S, H, pos, sw, static=True)
     assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
+# one position for the batch: shares of fewer than 256 pairs (both cut, or both whole), whole rounds, a remainder too small to be
+# cut, a window - and pairs beyond 256 whose remainder a full workspace lets the other entry point cut
+@pytest.mark.parametrize("B,N,K,S,sw,cut", [(17, 16, 4, 1500, 0, False), (40, 16, 4, 700, 0, False), (64, 16, 4, 500, 0, False),
+                                            (73, 16, 4, 200, 0, False), (65, 16, 4, 700, 128, False), (65, 16, 4, 700, 0, True),
+                                            (33, 32, 8, 1100, 0, True)])
+def test_static_scratch_entry_point_with_one_position(B, N, K, S, sw, cut):
+    print(f"static scratch one position B={B} N={N} K={K} S={S} sw={sw}", file=sys.stderr, flush=True)
+    case = U.attention_case(B + S, B, N, K, S, 128, fp8=True)
+    for pos in (S - 1, S // 2):
+        got = _call(case, B, N, K, S, 128, pos, sw, static=True)
+        ref = _call(case, B, N, K, S, 128, pos, sw, static=False)
+        same = torch.equal(got.view(torch.int16), ref.view(torch.int16))
+        assert same != cut
+        if cut:  # (no more than the order of the sums: what the call gives without a workspace)
+            whole = _call(case, B, N, K, S, 128, pos, sw, static=False, workspace=False)
+            assert torch.equal(got.view(torch.int16), whole.view(torch.int16))
+            U.assert_close(U.to_np(got), U.to_np(ref))
