@@ -9,6 +9,7 @@ import torch
 from oracle import clib
 from oracle import lyra_oracle as O
 from tests import gpu_util as U
+from tests.test_gpu_attention import test_learned_exclusive_self_attention_in_the_epilogue as exclusive_self_attention
 from tests.test_gpu_fused import test_attention_with_the_front_step_equals_the_two_launches as front_step
 
 pytestmark = pytest.mark.gpu
@@ -69,6 +70,28 @@ def test_whole_pairs_and_a_chunked_remainder(B, K, N, S, H, fp8):
 @pytest.mark.parametrize("B,N,K,S", [(65, 16, 4, 600), (33, 32, 8, 1100), (23, 16, 4, 1100)])
 def test_front_step_in_a_launch_of_uneven_pairs(B, N, K, S):
     front_step(B, N, K, S, 128, True, True, 0, True, "full")
+
+
+# whole pairs and a chunked remainder (65 x 4, 33 x 8 as lyra-medium's heads at 33 rows, 64-wide heads), chunks only (23 x 4)
+@pytest.mark.parametrize("B,N,K,S,H", [(65, 16, 4, 700, 128), (33, 32, 8, 1025, 128), (33, 64, 8, 1100, 64), (23, 16, 4, 1100, 128)])
+def test_exclusive_self_attention_in_a_launch_of_uneven_pairs(B, N, K, S, H):
+    exclusive_self_attention(B, N, K, S, H, 0, False)
+
+
+@pytest.mark.parametrize("B,K,N,S,H", [(65, 4, 16, 700, 128), (33, 8, 32, 1025, 64)])
+def test_whole_pairs_and_a_chunked_remainder_in_e5m2(B, K, N, S, H):
+    from lyra_amd.kernels.decode_attention import decode_attention
+
+    print(f"attention shares e5m2 B={B} N={N} K={K} S={S} H={H}", file=sys.stderr, flush=True)
+    case = U.attention_case(B + S, B, N, K, S, H, fp8=True, fmt=2)
+    q, k, v, sinks = U.attention_torch_inputs(case)
+    (kq, ks), (vq, vs) = case["k"], case["v"]
+    for pos in (S - 1, S // 2):
+        at = torch.tensor(pos, dtype=torch.int32, device=U.dev())
+        got = decode_attention(q, k, v, sinks, H**-0.5, 0, at, dtype=torch.float32, implementation="pallas")
+        want = clib.decode_attention(O.bf16_bits(case["q"]), kq, vq, ks[..., 0], vs[..., 0], case["sinks"], np.full(B, pos, np.int32), None,
+                                     H**-0.5, 0, fp8_format=2)
+        U.assert_close(U.to_np(got), want, what=f"e5m2 shares pos={pos}")
 
 
 # windows that begin at every offset from a tile and from 16 bytes of scales, at the end of caches whose length is and is not a

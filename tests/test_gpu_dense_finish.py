@@ -31,7 +31,7 @@ def test_slices_summed_in_the_launch(M, K, N, kind):
     rand = lambda *s: torch.randn(*s, device=dev, generator=gen)  # noqa: E731
     w = (rand(1, K, N) * 0.05).to(torch.bfloat16)
     if kind != "bf16":
-        w = quantize(w, torch.float8_e4m3fn, (K, 1) if kind == "channel" else (256, 256))
+        w = quantize(w, torch.float8_e5m2 if kind == "e5m2" else torch.float8_e4m3fn, (256, 256) if kind == "block" else (K, 1))
     x, bias, res = rand(M, K).to(torch.bfloat16), rand(1, N).to(torch.bfloat16).float(), rand(M, N).to(torch.bfloat16)
     one = _lib.row_count(M, dev)
     sums = _slices_in_order(F.gemm_unsummed(x, w, one).partials)
@@ -63,6 +63,18 @@ def test_slices_summed_in_the_launch(M, K, N, kind):
     ws = [v for k, v in _lib._WORKSPACES.items() if k[0] == "gemm"]
     torch.cuda.synchronize()
     assert all(int(b[:65536].view(torch.int32).abs().sum()) == 0 for b in ws)
+
+
+# slices longer than a wavefront's register sets hold at once (1024, 2048 and 768 rows: the middle variant's projections), the sum
+# inside the launch up to 8 rows, with more than 8 only without SwiGLU
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("K,N,kind", [(4096, 6144, "bf16"), (4096, 6144, "block"), (4096, 12288, "channel"), (6144, 4096, "channel"),
+                                      (6144, 4096, "e5m2")])
+def test_long_slices_summed_in_the_launch(M, K, N, kind):
+    from lyra_amd import _lib
+
+    assert K / _lib.gemm_splits(M, K, N, 0 if kind == "bf16" else (256 if kind == "block" else K)) > 512
+    test_slices_summed_in_the_launch(M, K, N, kind)
 
 
 # slices of at most 2048 rows, also where that makes a second round of workgroups: longer ones add up more terms in a row

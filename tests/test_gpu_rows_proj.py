@@ -12,11 +12,14 @@ pytestmark = pytest.mark.gpu
 FP8 = torch.float8_e4m3fn
 
 
-# one row and the most rows, one slice of the up projection and more than are requested at once (6), slices of 256, 384 and 512
-# rows, a last span that the columns do not fill, every scale layout
+# one row and the most rows, one slice of the up projection and more than are requested at once (6), slices of 128, 256, 384 and
+# 512 rows, a last span that the columns do not fill; scales per column, one block along all of K, and blocks along K that hold a
+# wavefront's rows (128 and 256) or change within them (32 and 64)
 @pytest.mark.parametrize("M,K,N,kind,splits,with_bias", [
     (1, 256, 512, "bf16", 2, False), (16, 3072, 2048, "channel", 4, False), (5, 2048, 6144, "block", 6, True), (9, 512, 136, "bf16", 13, True),
-    (3, 2880, 5120, "channel", 7, False), (8, 1024, 2048, "e5m2", 1, False), (16, 768, 4096, "block", 3, True)])
+    (3, 2880, 5120, "channel", 7, False), (8, 1024, 2048, "e5m2", 1, False), (16, 768, 4096, "block", 3, True),
+    (4, 1024, 2048, "b32", 3, False), (7, 2048, 6144, "b64", 2, True), (13, 2048, 6144, "b32", 4, False), (6, 2048, 2048, "column", 4, False),
+    (10, 3456, 3584, "b128", 3, False), (2, 2880, 2816, "bf16", 4, True)])
 @pytest.mark.parametrize("packed", [False, True])
 def test_swiglu_inside_the_down_projection(M, K, N, kind, splits, with_bias, packed):
     from lyra_amd import _lib
@@ -29,7 +32,8 @@ def test_swiglu_inside_the_down_projection(M, K, N, kind, splits, with_bias, pac
     w = (rand(1, K, N) * 0.05).to(torch.bfloat16)
     w_abs = w[0].abs().double()
     if kind != "bf16":
-        w = quantize(w, torch.float8_e5m2 if kind == "e5m2" else FP8, (256, 256) if kind == "block" else (K, 1))
+        block = {"block": (256, 256), "b32": (32, 32), "b64": (64, 64), "b128": (128, 128), "column": (K, 128)}.get(kind, (K, 1))
+        w = quantize(w, torch.float8_e5m2 if kind == "e5m2" else FP8, block)
         s = w.scale[0].double().repeat_interleave(w.block[0], 0).repeat_interleave(w.block[1], 1)
         w_abs = (w.qval[0].float().double() * s).abs()
     sums = 3 * rand(splits, M, 2 * K)
