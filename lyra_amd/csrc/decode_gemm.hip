@@ -2535,10 +2535,14 @@ int launch_planned(GemmParams p, const GemmPlan& pl, int layout, int fused_swigl
     }
     if (pl.split_k) {
         // The sum of the slices inside the launch, by the last workgroup of a tile to arrive, for a few rows: one launch less on
-        // the host (3 us a call, which is what bounds a call from Python: lyra-small q/k/v at 5 rows 18.3 -> 15.1 us) and no slower
-        // on the device (8.6 -> 8.1 us, MLP up 9.5 -> 9.1, gpt-oss-20b out 9.6 -> 8.7, all in a graph).  With more rows the few
-        // workgroups that finish take longer than a launch of the whole device (16 rows: 12 slices 9.0 -> 11.0 us, SwiGLU 10.2 ->
-        // 10.7, 8 slices 9.3 -> 9.5; 64 rows 12.4 -> 14.0).
+        // the host, which is what bounds a call from Python at every shape (2048 x 3072 at 1 to 16 rows 17.4 -> 14.8 us, 3072 x 2048
+        // FP8 19.7 -> 17.1).  The device gains with it up to 8 slices or 1024 columns (us in a graph at 1 / 8 rows: 2048 x 1024 bf16, 8
+        // slices, 6.7 / 7.2 -> 6.2 / 6.8; 2880 x 328, 23 slices, 7.5 / 8.1 -> 6.6 / 7.3; 8192 x 256, 32, 9.5 / 10.3 -> 7.6 / 8.7; 4096 x 6144,
+        // 4, 12.1 / 12.7 -> 11.7 / 12.2) and loses with more of both (3072 x 2048 FP8, 12 slices, 7.2 / 7.9 -> 7.8 / 9.0; 4096 x 2048, 16, 7.9 /
+        // 8.5 -> 8.8 / 9.5): a captured call pays that, one from Python is faster all the same, and a decode step takes the slices as they
+        // are.  With more rows the few workgroups that finish take longer than a launch of the whole device: 9 to 16 rows cost
+        // 0.4-0.8 us up to 8 slices (2048 x 3072 at 16 8.6 -> 9.4), under the 2.5 us of host time; 2 us with 12, 0.5 with SwiGLU, 1.6 at
+        // 64 rows: two launches there.
         p.finish_in_launch = (M <= 8 || (M <= 16 && !fused_swiglu && pl.ksplit <= 8)) && (!fused_swiglu || N % 256 == 0) &&
                              (size_t)pl.spans * pl.row_par * sizeof(int) <= kGemmCounterBytes;
         const int rc = launch_split_k_fmt<WT>(p, pl, st);
