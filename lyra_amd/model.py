@@ -490,11 +490,6 @@ def attention_apply_fused(x, w: AttentionWeights, idx: int, pos, cos_t, sin_t, c
 
     H, N, K = cfg.head_dim, cfg.n_attn_heads, cfg.n_kv_heads
     tiled = _TILED_ACTIVATIONS and cfg.n_embd % 32 == 0  # (the normalised rows only feed the q/k/v projection: 16 x 32 tiles)
-    sliding_window = cfg.sliding_window if idx % 2 == 0 else 0
-    # (learned exclusive self attention needs the value rows that a launch of its own hands over)
-    front_step = w.xsa_alpha is None and not _SEPARATE_QKV_POST
-    w_qkv, w_out = F.span_major(w.qkv, always=_DENSE_SPAN_MAJOR), F.span_major(w.out, always=_DENSE_SPAN_MAJOR)
-    t = None
     if isinstance(x, TokenRows):  # first layer of a step: the embedding rows are gathered by the norm kernel
         h, gate, x = F.embed_rmsnorm_proj(x.table, x.tokens, w.norm_scale, cfg.norm_eps, w.sdpa_gate, None, gate=True, tiled=tiled)
     elif isinstance(x, (F.Unsummed, F.Uncombined)):
@@ -503,14 +498,18 @@ def attention_apply_fused(x, w: AttentionWeights, idx: int, pos, cos_t, sin_t, c
         h, gate = F.rmsnorm_proj(x, w.norm_scale, cfg.norm_eps, w.sdpa_gate, None, gate=True, tiled=tiled)
     B = x.shape[0]
     one = _one_group(B, x.device)
+    w_qkv, w_out = F.span_major(w.qkv, always=_DENSE_SPAN_MAJOR), F.span_major(w.out, always=_DENSE_SPAN_MAJOR)
     # (:310-313: a bias is added to the projection's bf16 result, in bf16: by the attention launch that sums the slices when
     # that launch is certain to take them - one position for the batch, no learned exclusive self attention - else inside
     # the matmul's epilogue, which costs the launch that sums the slices)
+    front_step = w.xsa_alpha is None and not _SEPARATE_QKV_POST
     qkv = F.gemm_unsummed(h, w_qkv, one) if (w.qkv_bias is None or (front_step and pos.numel() == 1)) else None
     if qkv is not None and w.qkv_bias is not None:
         qkv.bias = _bf16_bias(w.qkv_bias).reshape(-1)
     if qkv is None:
         qkv = F.gemm(h, w_qkv, one, bias=_bf16_bias(w.qkv_bias), bias_after_cast=w.qkv_bias is not None)
+    sliding_window = cfg.sliding_window if idx % 2 == 0 else 0
+    t = None
     if front_step:  # QK norm + RoPE + cache append inside the attention launch
         t = F.attention_qkv(qkv, w.qnorm_scale, w.knorm_scale, cos_t, sin_t, pos, cache.k, cache.v, w.sinks, H**-0.5,
                             sliding_window, N, K, H, cfg.norm_eps, gate=gate)
@@ -525,22 +524,14 @@ def attention_apply_fused(x, w: AttentionWeights, idx: int, pos, cos_t, sin_t, c
         attn = attn_op(cfg.mode, cfg.implementation)
         t = attn(q[:, :, None, :], cache.k, cache.v, w.sinks, H**-0.5, sliding_window, pos, gate=gate, xsa_v=xsa_v,
                  xsa_alpha=w.xsa_alpha).reshape(B, N * H)
-    return _attention_out(t, w_out, x, w, cfg), cache
-
-
-def _attention_out(t, w_out, x, w: AttentionWeights, cfg: ModelConfig):
-    """lyra/model.py:366-373: projection, + bias, * residual scale, + residual, each a bf16 result - left to the norm that sums
-    the slices, where there are slices."""
-    from lyra_amd.kernels import decode_fused as F
-
-    one = _one_group(t.shape[0], t.device)
+    # :366-373: projection, + bias, * residual scale, + residual, each a bf16 result - left to the norm that sums the slices
     out = F.gemm_unsummed(t, w_out, one)
     if out is None:
         return F.gemm(t, w_out, one, bias=_bf16_bias(w.out_bias), bias_after_cast=w.out_bias is not None, residual=x,
-                      out_scale=cfg.residual_scale)
+                      out_scale=cfg.residual_scale), cache
     out.residual, out.scale = x, cfg.residual_scale
     out.bias = None if w.out_bias is None else _bf16_bias(w.out_bias).reshape(-1)
-    return out
+    return out, cache
 
 
 def moe_apply_fused(x, w: MoEWeights, cfg: ModelConfig, groups_out: list | None = None):
