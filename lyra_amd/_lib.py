@@ -138,7 +138,7 @@ class LyraHipError(RuntimeError):
 def _load() -> ctypes.CDLL:
     if not os.path.exists(LIB_PATH):
         raise LyraHipError(
-            f"{LIB_PATH} is missing: build it with `python -m lyra_amd.build` (hipcc, gfx950). "
+            f"{LIB_PATH} is missing: build it with `python {os.path.join(PKG_DIR, 'build.py')}` (hipcc, gfx950). "
             "lyra_amd has no non-HIP code path."
         )
     lib = ctypes.CDLL(LIB_PATH)

@@ -148,3 +148,19 @@ def test_decode_step_refuses_scratch_that_is_too_small_before_any_launch(rows, e
     for nbytes in [*range(0, need, 256), need - 1]:
         assert L.lyra_decode_step(step(nbytes), None) == -3, nbytes
     assert L.lyra_decode_step(step(need, scratch=128), None) == -3
+
+
+def test_a_missing_library_names_a_command_that_runs_without_it(tmp_path):
+    import shutil
+    import subprocess
+    import sys
+
+    copy = tmp_path / "lyra_amd"
+    shutil.copytree(os.path.join(ROOT, "lyra_amd"), copy, ignore=shutil.ignore_patterns("*.so", "__pycache__"))
+    run = lambda *args: subprocess.run([sys.executable, *args], cwd=tmp_path, capture_output=True, text=True, timeout=300)  # noqa: E731
+    err = run("-c", "import lyra_amd").stderr
+    command = re.search(r"build it with `python (.+?)`", err).group(1)
+    assert command == str(copy / "build.py")
+    # (up to the compiler: one that always fails)
+    tried = subprocess.run([sys.executable, command], cwd=tmp_path, capture_output=True, text=True, timeout=300, env={**os.environ, "HIPCC": "false"})
+    assert "hipcc failed" in tried.stderr
