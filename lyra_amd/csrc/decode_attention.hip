@@ -1147,7 +1147,9 @@ static AttnPlan plan_attention(int B, int K, int S, int sliding_window) {
 // The count follows from the cache's length and holds at every position in it: FP8 at S / 4, S / 2, 3 S / 4 and S, cut finer and as
 // here, 33 x 4 x 4096 24.0 / 38.8 / 40.1 / 41.7 and 14.6 / 22.0 / 30.7 / 38.5; 17 x 4 x 2000 15.0 / 15.7 / 16.2 / 16.9 and 11.1 / 13.4 /
 // 13.8 / 14.4; 30 x 4 x 2000 11.7 / 17.0 / 20.5 / 21.7 and 11.7 / 16.8 / 16.6 / 17.0 (an empty chunk still takes a turn on a unit).
-// Only the first quarter of a long cache is slower in a few (12 x 4 x 4096 13.1 / 17.8 / 20.9 / 21.2 and 14.3 / 15.1 / 15.9 / 16.3).
+// Of 68 shapes 6 are slower somewhere by more than 4 %: the first quarter of a long cache where a count just over 256 becomes one
+// below it (12 x 4 x 4096 13.1 / 17.8 / 20.9 / 21.2 and 14.3 / 15.1 / 15.9 / 16.3; 10 x 4 x 4096, 12 x 4 x 2000 and bf16 5 x 8 x 4096
+// alike), and two of 64-wide heads (15 x 8 x 4096 at the half, 16.2 and 18.6; 23 x 8 x 4096 at the end, 26.1 and 27.9).
 // Fewer than 4 rows keep the finer cut, which differs for them only in caches of a few hundred keys (3 x 4 x 300 8.3 us, whole 6.6):
 // another order of the same sums sends a row in 70 to another expert further on, and there one row is the result.
 // Rows with a position each leave more than 256 pairs whole (the whole-row kernel takes those).  key_bytes: of one key and its
