@@ -70,6 +70,7 @@ struct AttnParams {
 };
 
 constexpr int kTile = 32;
+constexpr int kCutSaves = 104 * 1024;  // bytes of keys and values that cutting a pair behind whole ones has to save (plan_shares)
 constexpr int kMaxRankedRows = 256;  // batch rows the whole-row kernel can rank by length (one per thread)
 constexpr int kMergeStageFloats = 3 * 1024 + 16;  // LDS floats used when the last workgroup merges chunks
 
@@ -625,6 +626,16 @@ void decode_attention_kernel(AttnParams p) {
 
     const int pos = __builtin_amdgcn_readfirstlane((int)pos_raw);  // (waited for here, with everything above in flight)
     const Range rg = visible_range(pos, p.sw, p.S);
+    if constexpr (WHOLE) {  // a part-filled cache: a pair whose cut saves less than its merge costs stays whole, with its first workgroup
+        if (n_chunks > 1 && (long)(rg.hi + 1 - chunk) * (2 * H * ES) < kCutSaves) {
+            if (c_idx > 0) {
+                wait_all_memory();
+                return;
+            }
+            n_chunks = 1;
+            chunk = p.S;
+        }
+    }
     const int c_lo = rg.start + c_idx * chunk;
     if (c_lo > rg.hi) {  // chunk holds no visible key (whole workgroup leaves together)
         // First chunk empty = no chunk of this row holds a key (position < 0): only the sink is attended and its value is
@@ -1138,18 +1149,21 @@ static AttnPlan plan_attention(int B, int K, int S, int sliding_window) {
 
 // The plan above in even shares: as many whole pairs on each compute unit as there are full rounds of them, and the pairs left
 // over (all, when there are fewer than 256) cut into as many chunks each as still make one workgroup per unit.  A unit that
-// gets a second pair, or a chunk more than the others, sets the launch's time: 65 rows x 4 heads x 2000 keys in FP8 took
-// 39.2 us, with the 4 left-over pairs in chunks 27.5; 37 x 8 x 1777 in bf16 62.7 and 48.5; 48 x 8 x 3001 at H = 64 34.2 and
-// 31.3; 23 x 4 x 2000 in 3 chunks 20.6, in 2 16.4; 50 x 4 x 2000 in 2 chunks 27.3, whole 22.9.  A chunk costs its merge
-// (2-3 us), so pairs are only cut where that saves the streaming of 128 KB or more (64 KB where only part of the device is
-// busy, which streams faster per unit): 33 x 8 x 1000 FP8 21.9 -> 18.0 us, 16 x 8 x 1000 in 2 chunks 12.5, whole 13.9; but
-// 45 x 8 x 300 10.6 whole, 13.4 cut.
-// The count follows from the cache's length and holds at every position in it: FP8 at S / 4, S / 2, 3 S / 4 and S, cut finer and as
-// here, 33 x 4 x 4096 24.0 / 38.8 / 40.1 / 41.7 and 14.6 / 22.0 / 30.7 / 38.5; 17 x 4 x 2000 15.0 / 15.7 / 16.2 / 16.9 and 11.1 / 13.4 /
-// 13.8 / 14.4; 30 x 4 x 2000 11.7 / 17.0 / 20.5 / 21.7 and 11.7 / 16.8 / 16.6 / 17.0 (an empty chunk still takes a turn on a unit).
-// Of 68 shapes 6 are slower somewhere by more than 4 %: the first quarter of a long cache where a count just over 256 becomes one
-// below it (12 x 4 x 4096 13.1 / 17.8 / 20.9 / 21.2 and 14.3 / 15.1 / 15.9 / 16.3; 10 x 4 x 4096, 12 x 4 x 2000 and bf16 5 x 8 x 4096
-// alike), and two of 64-wide heads (15 x 8 x 4096 at the half, 16.2 and 18.6; 23 x 8 x 4096 at the end, 26.1 and 27.9).
+// gets a second pair, or a chunk more than the others, sets the launch's time.
+// Fewer than 256 pairs: cut where that saves the streaming of 64 KB or more against the merge (2-3 us; part of the device
+// streams faster per unit).  The count follows from the cache's length and holds at every position in it: FP8 at S / 4, S / 2,
+// 3 S / 4 and S, cut finer and as here, 33 x 4 x 4096 24.0 / 38.8 / 40.1 / 41.7 and 14.6 / 22.0 / 30.7 / 38.5 us; 17 x 4 x 2000 15.0 /
+// 15.7 / 16.2 / 16.9 and 11.1 / 13.4 / 13.8 / 14.4; 30 x 4 x 2000 11.7 / 17.0 / 20.5 / 21.7 and 11.7 / 16.8 / 16.6 / 17.0 (an empty chunk
+// still takes a turn on a unit).  Of 68 shapes 6 are slower somewhere by more than 4 %: the first quarter of a long cache where
+// a count just over 256 becomes one below it (12 x 4 x 4096 13.1 / 17.8 / 20.9 / 21.2 and 14.3 / 15.1 / 15.9 / 16.3; 10 x 4 x 4096,
+// 12 x 4 x 2000 and bf16 5 x 8 x 4096 alike), and two of 64-wide heads (15 x 8 x 4096 at the half, 16.2 and 18.6; 23 x 8 x 4096 at the
+// end, 26.1 and 27.9).
+// More than 256: a cut pays for its merge from about 100 KB that the longest chunk leaves out (kCutSaves; break-even seen between
+// 85 and 130 KB over both widths, both formats and 2 to 32 chunks), which depends on how far the cache is filled: the kernel
+// leaves the pairs whole below that, and the launch is cut at all only if the full cache saves twice as much.  All whole and as
+// here at S / 8, S / 4, S / 2, 3 S / 4 and S: 65 x 4 x 4096 FP8 13.5 / 22.0 / 39.1 / 56.1 / 72.5 and 13.7 / 18.2 / 26.8 / 36.3 / 45.5 us; 75 x 4 x
+// 1500 8.6 / 11.7 / 18.1 / 24.8 / 31.0 and 9.2 / 12.1 / 18.3 / 22.8 / 25.8 (the workgroups that then leave at once cost 0.2-0.7); 37 x 8 x
+// 1500 bf16 10.5 / 16.7 / 29.0 / 41.3 / 52.6 and 11.3 / 17.3 / 26.4 / 34.3 / 41.3; cut at every position, 8.6 -> 11.3 in the first of them.
 // Fewer than 4 rows keep the finer cut, which differs for them only in caches of a few hundred keys (3 x 4 x 300 8.3 us, whole 6.6):
 // another order of the same sums sends a row in 70 to another expert further on, and there one row is the result.
 // Rows with a position each leave more than 256 pairs whole (the whole-row kernel takes those).  key_bytes: of one key and its
@@ -1161,8 +1175,9 @@ static AttnPlan plan_shares(int B, int K, int S, int key_bytes, int sliding_wind
     const long pairs = (long)B * K, left = pairs % 256;
     if (off || B < 4 || sliding_window > 0 || left == 0 || pairs > kMaxSplitPairs || (pairs > 256 && !one_position)) return pl;
     long want = std::min(256 / left, ((long)S + pl.waves * kTile - 1) / (pl.waves * kTile));
-    if ((double)S * key_bytes * (want - 1) < (pairs > 256 ? 131072.0 : 65536.0) * want) want = 1;
+    if (pairs < 256 && (double)S * key_bytes * (want - 1) < 65536.0 * want) want = 1;
     cut_chunks(pl, S, want);
+    if (pairs > 256 && (double)(S - pl.chunk) * key_bytes < 2.0 * kCutSaves) cut_chunks(pl, S, 1);
     pl.whole = pairs > 256 && pl.n_chunks > 1 ? (int)(pairs - left) : 0;
     return pl;
 }

@@ -729,8 +729,8 @@ def test_attention_with_the_front_step_equals_the_two_launches(B, N, K, S, H, fp
     kn = U.t_f32((1 + 0.1 * rng.standard_normal(H)).astype(np.float32)) if qknorm else None
     cos_t, sin_t = O.rope_tables(S, H)
     cos_t, sin_t = U.t_f32(cos_t), U.t_f32(sin_t)
-    if positions == "full":
-        pos = torch.tensor(S - 1, dtype=torch.int32, device=dev)
+    if positions == "full" or isinstance(positions, int):
+        pos = torch.tensor(S - 1 if positions == "full" else positions, dtype=torch.int32, device=dev)
     else:
         if positions == "short":
             vals = rng.integers(0, 130, B)

@@ -98,8 +98,8 @@ def test_static_scratch_entry_point_at_drawn_shapes(seed):
 # one position for the batch: shares of fewer than 256 pairs (both cut, or both whole), whole rounds, a remainder too small to be
 # cut, a window - and pairs beyond 256 whose remainder a full workspace lets the other entry point cut
 @pytest.mark.parametrize("B,N,K,S,sw,cut", [(17, 16, 4, 1500, 0, False), (40, 16, 4, 700, 0, False), (64, 16, 4, 500, 0, False),
-                                            (73, 16, 4, 200, 0, False), (65, 16, 4, 700, 128, False), (65, 16, 4, 700, 0, True),
-                                            (33, 32, 8, 1100, 0, True)])
+                                            (73, 16, 4, 200, 0, False), (65, 16, 4, 700, 128, False), (65, 16, 4, 700, 0, False),
+                                            (65, 16, 4, 1500, 0, True), (33, 32, 8, 1500, 0, True)])
 def test_static_scratch_entry_point_with_one_position(B, N, K, S, sw, cut):
     print(f"static scratch one position B={B} N={N} K={K} S={S} sw={sw}", file=sys.stderr, flush=True)
     case = U.attention_case(B + S, B, N, K, S, 128, fp8=True)
