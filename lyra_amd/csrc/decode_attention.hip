@@ -1154,18 +1154,17 @@ static AttnPlan plan_attention(int B, int K, int S, int sliding_window) {
 // streams faster per unit).  The count follows from the cache's length and holds at every position in it: FP8 at S / 4, S / 2,
 // 3 S / 4 and S, cut finer and as here, 33 x 4 x 4096 24.0 / 38.8 / 40.1 / 41.7 and 14.6 / 22.0 / 30.7 / 38.5 us; 17 x 4 x 2000 15.0 /
 // 15.7 / 16.2 / 16.9 and 11.1 / 13.4 / 13.8 / 14.4; 30 x 4 x 2000 11.7 / 17.0 / 20.5 / 21.7 and 11.7 / 16.8 / 16.6 / 17.0 (an empty chunk
-// still takes a turn on a unit).  Of 68 shapes 6 are slower somewhere by more than 4 %: the first quarter of a long cache where
-// a count just over 256 becomes one below it (12 x 4 x 4096 13.1 / 17.8 / 20.9 / 21.2 and 14.3 / 15.1 / 15.9 / 16.3; 10 x 4 x 4096,
-// 12 x 4 x 2000 and bf16 5 x 8 x 4096 alike), and two of 64-wide heads (15 x 8 x 4096 at the half, 16.2 and 18.6; 23 x 8 x 4096 at the
-// end, 26.1 and 27.9).
+// still takes a turn on a unit).  Of 48 shapes with 16 rows and more one is slower somewhere by more than 4 %: 23 x 8 x 4096 of
+// 64-wide heads, 26.1 and 27.9 at the end.
+// Fewer than 16 rows keep the finer cut: another order of the same sums sends a row in 70 of a lyra-small step to another expert,
+// 0.02-0.05 of that row's logits, and among few rows that is the result.  It costs them 1-2 us in caches of a few hundred keys (3 x 4 x
+// 300 8.3 us, whole 6.6) and at the end of long ones (12 x 4 x 4096 13.1 / 17.8 / 20.9 / 21.2, in even shares 14.3 / 15.1 / 15.9 / 16.3).
 // More than 256: a cut pays for its merge from about 100 KB that the longest chunk leaves out (kCutSaves; break-even seen between
 // 85 and 130 KB over both widths, both formats and 2 to 32 chunks), which depends on how far the cache is filled: the kernel
 // leaves the pairs whole below that, and the launch is cut at all only if the full cache saves twice as much.  All whole and as
 // here at S / 8, S / 4, S / 2, 3 S / 4 and S: 65 x 4 x 4096 FP8 13.5 / 22.0 / 39.1 / 56.1 / 72.5 and 13.7 / 18.2 / 26.8 / 36.3 / 45.5 us; 75 x 4 x
 // 1500 8.6 / 11.7 / 18.1 / 24.8 / 31.0 and 9.2 / 12.1 / 18.3 / 22.8 / 25.8 (the workgroups that then leave at once cost 0.2-0.7); 37 x 8 x
 // 1500 bf16 10.5 / 16.7 / 29.0 / 41.3 / 52.6 and 11.3 / 17.3 / 26.4 / 34.3 / 41.3; cut at every position, 8.6 -> 11.3 in the first of them.
-// Fewer than 4 rows keep the finer cut, which differs for them only in caches of a few hundred keys (3 x 4 x 300 8.3 us, whole 6.6):
-// another order of the same sums sends a row in 70 to another expert further on, and there one row is the result.
 // Rows with a position each leave more than 256 pairs whole (the whole-row kernel takes those).  key_bytes: of one key and its
 // value.  Its parts may need more room than those of the plan above; a caller's workspace is held to that plan, and gets it
 // when it is too small for this one.
@@ -1173,7 +1172,7 @@ static AttnPlan plan_shares(int B, int K, int S, int key_bytes, int sliding_wind
     AttnPlan pl = plan_attention(B, K, S, sliding_window);
     static const bool off = env_long("LYRA_ATTN_TARGET_WGS") > 0;  // (the override states the number of chunks)
     const long pairs = (long)B * K, left = pairs % 256;
-    if (off || B < 4 || sliding_window > 0 || left == 0 || pairs > kMaxSplitPairs || (pairs > 256 && !one_position)) return pl;
+    if (off || B < 16 || sliding_window > 0 || left == 0 || pairs > kMaxSplitPairs || (pairs > 256 && !one_position)) return pl;
     long want = std::min(256 / left, ((long)S + pl.waves * kTile - 1) / (pl.waves * kTile));
     if (pairs < 256 && (double)S * key_bytes * (want - 1) < 65536.0 * want) want = 1;
     cut_chunks(pl, S, want);

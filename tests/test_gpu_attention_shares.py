@@ -161,9 +161,9 @@ def test_window_adds_in_the_order_of_tiles_at_multiples_of_32(pos):
     assert torch.equal(got, want)
 
 
-# up to 3 rows a short cache is cut into chunks whatever its format (from 4 rows on, one of FP8 this short stays whole): codes
+# up to 15 rows a short cache is cut into chunks whatever its format (from 16 rows on, one of FP8 this short stays whole): codes
 # with unit scales and the same numbers in bf16 then give the same bits.  (Small whole numbers in q and k: exact in any order.)
-@pytest.mark.parametrize("B,K,S", [(1, 4, 300), (2, 4, 300), (3, 4, 300), (3, 8, 300), (1, 1, 330)])
+@pytest.mark.parametrize("B,K,S", [(1, 4, 300), (2, 4, 300), (3, 4, 300), (3, 8, 300), (1, 1, 330), (4, 4, 300), (15, 4, 300)])
 def test_few_rows_keep_their_chunks(B, K, S):
     from lyra_amd.kernels.decode_attention import decode_attention
     from lyra_amd.nn.quant import QArray
